@@ -48,6 +48,8 @@ struct chmc_ctx {
     size_t rec_cap = 0;
     unsigned long long* d_rdf = nullptr;
     int rdf_cap = 0;
+    uint4* d_rdfu = nullptr;     // fixed-point coordinates of the RDF's chain
+    int rdfu_cap = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;
     // learned surrogate (allocated on first use)
     bool surr_alloc = false, surr_params = false;
@@ -135,6 +137,7 @@ static void destroy_ctx(chmc_ctx* c)
     if (c->d_uniforms) hipFree(c->d_uniforms);
     if (c->d_rec) hipFree(c->d_rec);
     if (c->d_rdf) hipFree(c->d_rdf);
+    if (c->d_rdfu) hipFree(c->d_rdfu);
     if (c->Gtrain) hipFree(c->Gtrain);
     if (c->utrain) hipFree(c->utrain);
     if (c->spartial) hipFree(c->spartial);
@@ -1606,8 +1609,14 @@ extern "C" int chmc_rdf(chmc_ctx* c, int chain, int nbins, double size_bin, unsi
         c->rdf_cap = nbins;
     }
     const ChainDev& cd = c->hchains[chain];
-    HIPCHK(c, hipMemsetAsync(c->d_rdf, 0, sizeof(unsigned long long) * nbins, c->stream));
-    HIPCHK(c, launch_rdf(c->v, chain, cd.natoms, nbins, size_bin, c->d_rdf, c->stream));
+    if (c->rdfu_cap < cd.natoms) {
+        if (c->d_rdfu) hipFree(c->d_rdfu);
+        c->d_rdfu = nullptr;
+        c->rdfu_cap = 0;
+        HIPCHK(c, hipMalloc(&c->d_rdfu, sizeof(uint4) * cd.natoms));
+        c->rdfu_cap = cd.natoms;
+    }
+    HIPCHK(c, launch_rdf(c->v, chain, cd.natoms, nbins, size_bin, c->d_rdfu, c->d_rdf, c->stream));
     std::vector<unsigned long long> h(nbins);
     HIPCHK(c, hipMemcpyAsync(h.data(), c->d_rdf, sizeof(unsigned long long) * nbins, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));

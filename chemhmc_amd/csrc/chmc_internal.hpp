@@ -395,7 +395,8 @@ hipError_t launch_list_sweep(const DevView& v, int mode, int q, double kick_dt, 
 hipError_t launch_list_drift(const DevView& v, int q, double dt, hipStream_t s);
 // rel64: compute the FP64 relative positions first (false when the last sweep wrote them)
 hipError_t launch_list_energy(const DevView& v, int q, bool rel64, hipStream_t s);
-hipError_t launch_rdf(const DevView& v, int chain, int natoms, int nbins, double size_bin,
+// u: natoms fixed-point coordinates of scratch; counts: nbins, cleared here
+hipError_t launch_rdf(const DevView& v, int chain, int natoms, int nbins, double size_bin, uint4* u,
                       unsigned long long* counts, hipStream_t s);
 hipError_t launch_open_potential(const double* xyz_soa, int n, int nexp, double a, double b,
                                  double* partials, int* nparts, hipStream_t s);

@@ -1,61 +1,152 @@
 // All-pairs kernels.
 //  k_rdf: radial distribution histogram, the replacement of Tag_RDF (code/modules/identical_particles.cpp:739-776).
 //    The reference runs one team per bin over all N^2 ordered pairs (O(bins * N^2)); here each pair is
-//    visited once: 256 x 256 tiles of the upper triangle, FP64 per-dimension minimum image exactly as
-//    the reference (min of (d-L)^2, d^2, (d+L)^2), bin = (int)(r / size_bin), and an LDS histogram
-//    private to each wavefront, merged into per-block sums and then into global 64-bit counters.
-//    Unordered pairs are counted twice, which equals the reference's ordered count exactly.
+//    visited once and counted twice, which equals the reference's ordered count exactly.  The bin of a
+//    pair is the reference's (int)(r / size_bin) with its FP64 minimum image (min of (d-L)^2, d^2,
+//    (d+L)^2) for every pair, but almost all of them are decided in FP32 (see below).
 //  k_open_potential: code-carsten/potential_energy.hh:6-15, sum_{i<j} a/r^n - b/r^6 with open
 //    boundaries, FP64, per-block partial sums (summed in block order on the host).
 #include "chmc_internal.hpp"
+
+#include <algorithm>
 
 #pragma clang fp contract(off)
 
 namespace chmc {
 
-__global__ __launch_bounds__(256) void k_rdf(DevView v, int chain, int nbins, double size_bin,
-                                             unsigned long long* __restrict__ counts)
+// The exact bin of a pair, as the reference computes it (no contraction)
+__device__ __forceinline__ int rdf_bin_exact(const ChainDev& C, double xi, double yi, double zi, double xj, double yj,
+                                             double zj, double size_bin)
 {
-    extern __shared__ unsigned int hist[];     // [4 waves][nbins]
-    __shared__ double jx[256], jy[256], jz[256];
-    const int I = blockIdx.y, J = blockIdx.x;
-    if (J < I) return;
+    double r = 0.0, dd, ri, si;
+    dd = xj - xi;
+    ri = (dd - C.L[0]) * (dd - C.L[0]); si = dd * dd; if (si < ri) ri = si;
+    si = (dd + C.L[0]) * (dd + C.L[0]); if (si < ri) ri = si; r += ri;
+    dd = yj - yi;
+    ri = (dd - C.L[1]) * (dd - C.L[1]); si = dd * dd; if (si < ri) ri = si;
+    si = (dd + C.L[1]) * (dd + C.L[1]); if (si < ri) ri = si; r += ri;
+    dd = zj - zi;
+    ri = (dd - C.L[2]) * (dd - C.L[2]); si = dd * dd; if (si < ri) ri = si;
+    si = (dd + C.L[2]) * (dd + C.L[2]); if (si < ri) ri = si; r += ri;
+    return (int)(sqrt(r) / size_bin);
+}
+
+// Coordinates as 32-bit fractions of the box, u = round(2^32 x / L): the minimum image of a difference is
+// then the wrap of an integer subtraction.  w = 1 where a coordinate is outside [0, L] (or not a number):
+// pairs of such an atom take the exact path.  The counts are cleared here too.
+__global__ __launch_bounds__(256) void k_rdf_prep(DevView v, int chain, int nbins, uint4* __restrict__ u,
+                                                  unsigned long long* __restrict__ counts)
+{
+    const ChainDev& C = v.chains[chain];
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < nbins) counts[i] = 0ull;
+    if (i >= C.natoms) return;
+    unsigned q[3], bad = 0u;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const double x = v.x[(size_t)d * v.Ntot + C.atom_off + i];
+        const bool ok = x >= 0.0 && x <= C.L[d];
+        bad |= ok ? 0u : 1u;
+        q[d] = ok ? (unsigned)(unsigned long long)(x / C.L[d] * 4294967296.0 + 0.5) : 0u;
+    }
+    u[i] = make_uint4(q[0], q[1], q[2], bad);
+}
+
+constexpr int kRdfJ = 32;          // j atoms per step of a workgroup
+
+// One thread per i atom (256 a workgroup, row blockIdx.y), j atoms in steps of kRdfJ along the row, read
+// through scalar registers (the index is uniform), so that a pair costs no LDS read; one LDS histogram per
+// workgroup, added to the global counters once at its end.
+//   FP32 decision: with u exact to 2^-33 L, t = |d| / size_bin from three integer differences, converted,
+// scaled and summed in FP32 is within 6.5 * 2^-24 t + 2^-32 |L| / size_bin of the exact quotient (3 roundings
+// per component, 3 of the sum of squares, halved by the root, and 1 ulp of v_sqrt_f32).  A pair whose t is
+// farther than eps from an integer, eps = (nbins + 1) 2^-21 + 2^-31 |L| / size_bin, therefore has the exact
+// bin (int)t; the others (0.05 % at 500 bins) and any NaN are binned in FP64.  Bins from nbins + 1 up are
+// never counted and need no decision.
+//   Bound: VALU issue, ~22 slots a pair.  N = 32768, 500 bins up to L / 2 (5.4e8 pairs): 308 us, at the
+// VALU time of those slots (300 us), against 1531 us with the FP64 root and division for every pair.
+__global__ __launch_bounds__(256) void k_rdf(DevView v, int chain, int nbins, double size_bin,
+                                             const uint4* __restrict__ u, unsigned long long* __restrict__ counts)
+{
+    extern __shared__ unsigned int hist[];     // [nbins]
     const ChainDev& C = v.chains[chain];
     const int n = C.natoms, off = C.atom_off, N = v.Ntot;
-    const int tid = threadIdx.x, wave = tid >> 6;
-    for (int b = tid; b < 4 * nbins; b += 256) hist[b] = 0u;
-    const int i = I * 256 + tid;
-    const int j0 = J * 256 + tid;
-    double xi = 0, yi = 0, zi = 0;
-    if (i < n) { xi = v.x[off + i]; yi = v.x[N + off + i]; zi = v.x[2 * N + off + i]; }
-    if (j0 < n) { jx[tid] = v.x[off + j0]; jy[tid] = v.x[N + off + j0]; jz[tid] = v.x[2 * N + off + j0]; }
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int i0 = blockIdx.y * 256, steps = (n + kRdfJ - 1) / kRdfJ;
+    const int first = i0 / kRdfJ + blockIdx.x;
+    if (first >= steps) return;
+    for (int b = tid; b < nbins; b += 256) hist[b] = 0u;
     __syncthreads();
-    const double L0 = C.L[0], L1 = C.L[1], L2 = C.L[2];
-    if (i < n) {
-        const int jend = min(256, n - J * 256);
-        const int jstart = (I == J) ? tid + 1 : 0;
-        unsigned int* h = &hist[wave * nbins];
-        for (int jj = jstart; jj < jend; jj++) {
-            double r = 0.0, dd, ri, si;
-            dd = jx[jj] - xi;
-            ri = (dd - L0) * (dd - L0); si = dd * dd; if (si < ri) ri = si;
-            si = (dd + L0) * (dd + L0); if (si < ri) ri = si; r += ri;
-            dd = jy[jj] - yi;
-            ri = (dd - L1) * (dd - L1); si = dd * dd; if (si < ri) ri = si;
-            si = (dd + L1) * (dd + L1); if (si < ri) ri = si; r += ri;
-            dd = jz[jj] - zi;
-            ri = (dd - L2) * (dd - L2); si = dd * dd; if (si < ri) ri = si;
-            si = (dd + L2) * (dd + L2); if (si < ri) ri = si; r += ri;
-            r = sqrt(r);
-            const int b = (int)(r / size_bin);
-            if (b < nbins) atomicAdd(&h[b], 1u);
+    const int i = i0 + tid;
+    const bool ival = i < n;
+    const uint4 ui = u[ival ? i : n - 1];
+    const double xi = v.x[off + (ival ? i : n - 1)], yi = v.x[(size_t)N + off + (ival ? i : n - 1)],
+                 zi = v.x[2 * (size_t)N + off + (ival ? i : n - 1)];
+    const float sx = (float)(C.L[0] / 4294967296.0 / size_bin), sy = (float)(C.L[1] / 4294967296.0 / size_bin),
+                sz = (float)(C.L[2] / 4294967296.0 / size_bin);
+    const double diag = sqrt(C.L[0] * C.L[0] + C.L[1] * C.L[1] + C.L[2] * C.L[2]);
+    const float half = (float)(0.5 - ((nbins + 1) / 2097152.0 + diag / size_bin / 2147483648.0) - 1e-7);
+    const float edge = (float)(nbins + 1);
+    auto exact = [&](int j) {
+        const int b = rdf_bin_exact(C, xi, yi, zi, v.x[off + j], v.x[(size_t)N + off + j], v.x[2 * (size_t)N + off + j], size_bin);
+        if (b < nbins) atomicAdd(&hist[b], 1u);
+    };
+    // KB pairs (i, j0 ... j0 + KB - 1), those with j > i where check is set
+    auto pairs = [&](int j0, auto kb, bool check) {
+        constexpr int KB = decltype(kb)::value;
+        float t[KB];
+#pragma unroll
+        for (int k = 0; k < KB; k++) {
+            const uint4 uj = u[j0 + k];
+            const float dx = sx * (float)(int)(uj.x - ui.x), dy = sy * (float)(int)(uj.y - ui.y), dz = sz * (float)(int)(uj.z - ui.z);
+            t[k] = __builtin_amdgcn_sqrtf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)));
+        }
+        unsigned late = 0u;
+#pragma unroll
+        for (int k = 0; k < KB; k++) {
+            const bool on = !check || (ival && j0 + k > i);
+            // not clearly inside a bin, and not clearly beyond the last one (either is true for a NaN)
+            const bool un = on && !(fabsf(__builtin_amdgcn_fractf(t[k]) - 0.5f) <= half) && !(t[k] >= edge);
+            late |= un ? 1u << k : 0u;
+            const int b = (int)t[k];
+            if (on && !un && b < nbins) atomicAdd(&hist[b], 1u);
+        }
+        if (__ballot(late != 0u) != 0ull)
+            while (late != 0u) {
+                const int k = __ffs(late) - 1;
+                late &= late - 1u;
+                exact(j0 + k);
+            }
+    };
+    int done = 0;
+    auto flush = [&]() {
+        __syncthreads();
+        for (int k = tid; k < nbins; k += 256) {
+            int b = k + (int)(blockIdx.x + blockIdx.y) * 64 % nbins;      // workgroups start at different counters
+            if (b >= nbins) b -= nbins;
+            const unsigned s = hist[b];
+            hist[b] = 0u;
+            if (s) atomicAdd(&counts[b], 2ull * s);
+        }
+        __syncthreads();
+    };
+    for (int J = first; J < steps; J += gridDim.x) {
+        const int j0 = J * kRdfJ, jn = min(kRdfJ, n - j0);
+        const bool odd = __ballot(ui.w != 0u || u[j0 + min(lane & (kRdfJ - 1), jn - 1)].w != 0u) != 0ull;
+        if (odd) {
+            for (int jj = 0; jj < jn; jj++)
+                if (ival && j0 + jj > i) exact(j0 + jj);
+        } else if (j0 < i0 + 256 || i0 + 256 > n || jn < kRdfJ) {
+            for (int jj = 0; jj < jn; jj++) pairs(j0 + jj, std::integral_constant<int, 1>{}, true);
+        } else {
+            for (int jj = 0; jj < kRdfJ; jj += 8) pairs(j0 + jj, std::integral_constant<int, 8>{}, false);
+        }
+        if (++done == (1 << 18)) {             // 2^31 pairs: before a 32-bit count can overflow
+            done = 0;
+            flush();
         }
     }
-    __syncthreads();
-    for (int b = tid; b < nbins; b += 256) {
-        const unsigned long long s = (unsigned long long)hist[b] + hist[nbins + b] + hist[2 * nbins + b] + hist[3 * nbins + b];
-        if (s) atomicAdd(&counts[b], 2ull * s);
-    }
+    flush();
 }
 
 // coordinate d of atom i is xyz[i * si + d * sd]: SoA (si = 1, sd = n) or AoS double[3] (si = 3, sd = 1)
@@ -93,13 +184,17 @@ __global__ __launch_bounds__(256) void k_open_potential(const double* __restrict
     if (tid == 0) partials[pid] = ((wpart[0] + wpart[1]) + wpart[2]) + wpart[3];
 }
 
-hipError_t launch_rdf(const DevView& v, int chain, int natoms, int nbins, double size_bin,
+// about 2048 workgroups (8 a CU): few enough that adding their histograms to the counters stays small,
+// rows in order, so that the long ones start first
+hipError_t launch_rdf(const DevView& v, int chain, int natoms, int nbins, double size_bin, uint4* u,
                       unsigned long long* counts, hipStream_t s)
 {
-    const int T = (natoms + 255) / 256;
-    if (T == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_rdf, dim3(T, T), dim3(256), sizeof(unsigned int) * 4 * nbins, s, v, chain, nbins,
-                       size_bin, counts);
+    hipLaunchKernelGGL(k_rdf_prep, dim3((std::max(natoms, nbins) + 255) / 256), dim3(256), 0, s, v, chain, nbins, u, counts);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || natoms == 0) return e;
+    const int rows = (natoms + 255) / 256, steps = (natoms + kRdfJ - 1) / kRdfJ;
+    const int gx = std::min(steps, std::max(1, 4096 / rows));
+    hipLaunchKernelGGL(k_rdf, dim3(gx, rows), dim3(256), sizeof(unsigned int) * nbins, s, v, chain, nbins, size_bin, u, counts);
     return hipGetLastError();
 }
 

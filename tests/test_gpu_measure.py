@@ -1,0 +1,41 @@
+"""The pair measurements (RDF histogram, open-boundary sum) at the edges of their kernels, against plain
+numpy in FP64."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _rdf_counts(x, L, nb, size):
+    """Ordered pair counts per bin: the minimum image of every dimension as min((d-L)^2, d^2, (d+L)^2),
+    bin = (int)(r / size)."""
+    L = np.broadcast_to(np.asarray(L, float), (3,))
+    c = np.zeros(nb, np.uint64)
+    for i in range(len(x) - 1):
+        d = x[i + 1:] - x[i]
+        q = np.minimum(np.minimum((d - L) ** 2, d * d), (d + L) ** 2)
+        b = np.minimum(np.sqrt((q[:, 0] + q[:, 1]) + q[:, 2]) / size, 2.0 ** 30).astype(np.int64)
+        c += 2 * np.bincount(b[b < nb], minlength=nb).astype(np.uint64)
+    return c
+
+
+def _lattice(N, L):
+    s = int(np.ceil(N ** (1 / 3) - 1e-9))
+    k = np.arange(N)
+    return (np.stack((k % s, (k // s) % s, k // (s * s)), -1) + 0.5) * (np.asarray(L, float) / s)
+
+
+# one atom, tiles of 256 i atoms and 32 j atoms with remainders, an anisotropic box, one bin, the most bins,
+# bins so narrow or so wide that every pair is decided in FP64, and a lattice whose distances lie on bin edges
+@pytest.mark.parametrize("N,L,nb,size,lattice", [
+    (1, 6.0, 10, 0.3, False), (2, 6.0, 10, 0.6, False), (31, 6.0, 100, 0.05, False), (255, 7.0, 64, 0.06, False),
+    (257, 7.0, 333, 0.02, False), (289, (5.0, 7.5, 11.0), 200, 0.04, False), (1025, 11.0, 1, 2.0, False),
+    (1100, 11.0, 4000, 0.0025, False), (600, 9.0, 50, 1e-9, False), (600, 9.0, 50, 40.0, False),
+    (512, 16.0, 64, 0.5, True), (512, 16.0, 16, 2.0, True), (700, (9.0, 9.0, 18.0), 90, 0.1, True)])
+def test_rdf_counts_edges(chmc, N, L, nb, size, lattice):
+    box = np.broadcast_to(np.asarray(L, float), (3,))
+    x = _lattice(N, box) if lattice else np.random.default_rng(N + nb).uniform(0, 1, (N, 3)) * box
+    with chmc.Engine(chmc.Chain(N=N, L=tuple(box), cutoff=2.5)) as e:
+        e.set_positions(x)
+        counts, _ = e.rdf(nb, size)
+    assert np.array_equal(counts, _rdf_counts(x, box, nb, size))
