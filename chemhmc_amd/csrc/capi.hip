@@ -1636,6 +1636,55 @@ extern "C" int chmc_rdf(chmc_ctx* c, int chain, int nbins, double size_bin, unsi
     return CHMC_OK;
 }
 
+// Memory of the open-boundary sums, file-scope device arrays, one copy per GPU, held until the process
+// ends: `scratch` holds the tile partials of chmc_potential_energy_open_noalloc, `open_buf` the atoms, tile
+// partials and result of chmc_potential_energy_open calls of at most kOpenSmall atoms, which take turns
+// (g_open_mu), so that a call allocates nothing.  Host code never passes an array's name to a kernel (on the
+// host it is only a stand-in); it uses the device address that hipGetSymbolAddress returns for the current
+// device.
+static constexpr int kOpenScratchAtoms = CHMC_OPEN_NOALLOC_MAX;
+static constexpr int kOpenScratchTiles = 256;
+static_assert(kOpenScratchTiles * 256 >= kOpenScratchAtoms && kOpenScratchTiles * 64 >= kOpenSmall, "tile partials");
+static constexpr size_t kOpenPartials = (size_t)kOpenScratchTiles * kOpenScratchTiles;
+static __device__ __align__(256) double scratch[kOpenPartials];
+static __device__ __align__(256) double open_buf[3 * (size_t)kOpenSmall + kOpenPartials + 1];
+
+static constexpr int kMaxDevices = 64;
+static std::mutex g_scratch_mu, g_open_mu;
+struct OpenMem { double *scratch, *buf; };
+static OpenMem g_open_mem[kMaxDevices] = {};
+
+// device addresses of the arrays on the current device, looked up once per device
+static hipError_t open_memory(OpenMem* out)
+{
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    OpenMem& m = g_open_mem[dev];
+    if (!m.buf) {
+        void *p = nullptr, *q = nullptr;
+        if ((e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch))) != hipSuccess) return e;
+        if ((e = hipGetSymbolAddress(&q, HIP_SYMBOL(open_buf))) != hipSuccess) return e;
+        m.scratch = static_cast<double*>(p);
+        m.buf = static_cast<double*>(q);
+    }
+    *out = m;
+    return hipSuccess;
+}
+
+// upload, sum and read back on the calling thread's stream; part: tile partials, then the result
+static hipError_t open_sum(const double* xyz, int np, int n, double a, double b, double* dx, double* part, double* result)
+{
+    const size_t nt = (size_t)open_potential_tiles(np);
+    hipError_t e = hipMemcpyAsync(dx, xyz, sizeof(double) * 3 * (size_t)np, hipMemcpyHostToDevice, hipStreamPerThread);
+    if (e == hipSuccess) e = launch_open_potential(dx, np, n, a, b, part, part + nt * nt, hipStreamPerThread);
+    if (e == hipSuccess) e = hipMemcpyAsync(result, part + nt * nt, sizeof(double), hipMemcpyDeviceToHost, hipStreamPerThread);
+    const hipError_t es = hipStreamSynchronize(hipStreamPerThread);
+    return e == hipSuccess ? es : e;
+}
+
 extern "C" int chmc_potential_energy_open(const double* xyz, int n_particles, int n, double a, double b, double* result)
 {
     if (!xyz || !result || n_particles < 0) return CHMC_E_ARG;
@@ -1644,63 +1693,25 @@ extern "C" int chmc_potential_energy_open(const double* xyz, int n_particles, in
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return fail(nullptr, CHMC_E_NODEV, "no HIP device");
     const int np = n_particles;
-    const int T = (np + 255) / 256;
-    std::vector<double> soa(3 * (size_t)np);
-    for (int i = 0; i < np; i++)
-        for (int d = 0; d < 3; d++) soa[(size_t)d * np + i] = xyz[3 * i + d];
-    double *dx = nullptr, *dp = nullptr;
-    hipStream_t s = nullptr;
-    auto cleanup = [&]() {
-        if (dx) hipFree(dx);
-        if (dp) hipFree(dp);
-        if (s) hipStreamDestroy(s);
-    };
-    hipError_t e = hipStreamCreate(&s);
-    if (e == hipSuccess) e = hipMalloc(&dx, sizeof(double) * soa.size());
-    if (e == hipSuccess) e = hipMalloc(&dp, sizeof(double) * (size_t)T * T);
-    if (e == hipSuccess) e = hipMemcpyAsync(dx, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice, s);
-    int nparts = 0;
-    if (e == hipSuccess) e = launch_open_potential(dx, np, n, a, b, dp, &nparts, s);
-    std::vector<double> parts((size_t)T * T);
-    if (e == hipSuccess) e = hipMemcpyAsync(parts.data(), dp, sizeof(double) * parts.size(), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    cleanup();
-    if (e != hipSuccess) return fail(nullptr, CHMC_E_HIP, std::string("potential_energy_open: ") + hipGetErrorString(e));
+    hipError_t e;
     double r = 0.0;
-    for (double q : parts) r += q;
+    if (np <= kOpenSmall) {
+        OpenMem m;
+        e = open_memory(&m);
+        if (e == hipSuccess) {
+            std::lock_guard<std::mutex> lk(g_open_mu);
+            e = open_sum(xyz, np, n, a, b, m.buf, m.buf + 3 * (size_t)kOpenSmall, &r);
+        }
+    } else {
+        const size_t nt = (size_t)open_potential_tiles(np);
+        double* d = nullptr;
+        e = hipMalloc(&d, sizeof(double) * (3 * (size_t)np + nt * nt + 1));
+        if (e == hipSuccess) e = open_sum(xyz, np, n, a, b, d, d + 3 * (size_t)np, &r);
+        if (d) hipFree(d);
+    }
+    if (e != hipSuccess) return fail(nullptr, CHMC_E_HIP, std::string("potential_energy_open: ") + hipGetErrorString(e));
     *result = r;
     return CHMC_OK;
-}
-
-
-// ---- the same sum without allocation ---------------------------------------------------------------
-// Block partials of chmc_potential_energy_open_noalloc live in this file-scope array, one copy per GPU,
-// held until the process ends.  Host code never passes the array's name to a kernel (on the host it is
-// only a stand-in); it uses the device address that hipGetSymbolAddress returns for the current device.
-static constexpr int kOpenScratchAtoms = CHMC_OPEN_NOALLOC_MAX;
-static constexpr int kOpenScratchTiles = (kOpenScratchAtoms + 255) / 256;
-static __device__ __align__(256) double scratch[kOpenScratchTiles * kOpenScratchTiles];
-
-static constexpr int kMaxDevices = 64;
-static std::mutex g_scratch_mu;
-static double* g_scratch_ptr[kMaxDevices] = {};
-
-// device address of `scratch` on the current device, looked up once per device
-static hipError_t open_scratch(double** out)
-{
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if (!g_scratch_ptr[dev]) {
-        void* ptr = nullptr;
-        e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-        if (e != hipSuccess) return e;
-        g_scratch_ptr[dev] = static_cast<double*>(ptr);
-    }
-    *out = g_scratch_ptr[dev];
-    return hipSuccess;
 }
 
 extern "C" int chmc_potential_energy_open_noalloc(const double* xyz_dev, int n_particles, int n, double a, double b,
@@ -1710,11 +1721,11 @@ extern "C" int chmc_potential_energy_open_noalloc(const double* xyz_dev, int n_p
     if (n_particles > kOpenScratchAtoms)
         return fail(nullptr, CHMC_E_ARG, "potential_energy_open_noalloc: n_particles " + std::to_string(n_particles) +
                                              " exceeds the scratch capacity of " + std::to_string(kOpenScratchAtoms) + " atoms");
-    double* part = nullptr;
-    hipError_t e = open_scratch(&part);
+    OpenMem m;
+    hipError_t e = open_memory(&m);
     if (e == hipSuccess)
-        e = launch_open_potential_aos(n_particles >= 2 ? xyz_dev : nullptr, n_particles >= 2 ? n_particles : 0, n, a, b,
-                                      part, result_dev, static_cast<hipStream_t>(stream));
+        e = launch_open_potential(n_particles >= 2 ? xyz_dev : nullptr, n_particles >= 2 ? n_particles : 0, n, a, b,
+                                  m.scratch, result_dev, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(nullptr, CHMC_E_HIP, std::string("potential_energy_open_noalloc: ") + hipGetErrorString(e));
     return CHMC_OK;
 }

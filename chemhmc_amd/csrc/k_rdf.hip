@@ -5,7 +5,7 @@
 //    pair is the reference's (int)(r / size_bin) with its FP64 minimum image (min of (d-L)^2, d^2,
 //    (d+L)^2) for every pair, but almost all of them are decided in FP32 (see below).
 //  k_open_potential: code-carsten/potential_energy.hh:6-15, sum_{i<j} a/r^n - b/r^6 with open
-//    boundaries, FP64, per-block partial sums (summed in block order on the host).
+//    boundaries, FP64, per-tile partial sums, added in a fixed order by k_open_sum.
 #include "chmc_internal.hpp"
 
 #include <algorithm>
@@ -149,32 +149,48 @@ __global__ __launch_bounds__(256) void k_rdf(DevView v, int chain, int nbins, do
     flush();
 }
 
-// coordinate d of atom i is xyz[i * si + d * sd]: SoA (si = 1, sd = n) or AoS double[3] (si = 3, sd = 1)
-__global__ __launch_bounds__(256) void k_open_potential(const double* __restrict__ xyz, int n, int si, int sd,
-                                                        int nexp, double a, double b, double* __restrict__ partials)
+// |n|-th power of r from q = r^2 by repeated squaring (n uniform); an odd power takes one factor sqrt(q)
+__device__ __forceinline__ double pow_from_square(double q, int n)
 {
-    __shared__ double jx[256], jy[256], jz[256];
+    const unsigned m = n < 0 ? 0u - (unsigned)n : (unsigned)n;
+    double p = (m & 1u) ? sqrt(q) : 1.0;
+    for (unsigned e = m >> 1; e != 0u; e >>= 1) {
+        if (e & 1u) p *= q;
+        q *= q;
+    }
+    return n < 0 ? 1.0 / p : p;
+}
+
+// Tiles of E x E pairs (E = 64: four waves of 64 i atoms, each a quarter of the 64 j atoms; E = 256: one i
+// atom per thread, all 256 j atoms); coordinate d of atom i is xyz[3 i + d].  The j atoms are uniform in a
+// wave and come through scalar loads.  r^n and r^6 are powers of r^2 by multiplication: a call of pow cost
+// ~150 instructions twice a pair and the root another 20.  Bound: latency below a few thousand atoms (the
+// 64-tiles put 136 workgroups on N = 1000 where 256-tiles put 10), FP64 VALU beyond.  N = 1000, n = 12:
+// 10.7 us against 225 us (pow, 256-tiles).
+template <int E>
+__global__ __launch_bounds__(256) void k_open_potential(const double* __restrict__ xyz, int n, int nexp, double a, double b,
+                                                        double* __restrict__ partials)
+{
     __shared__ double wpart[4];
     const int I = blockIdx.y, J = blockIdx.x;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pid = I * gridDim.x + J;
     if (J < I) {
         if (tid == 0) partials[pid] = 0.0;
         return;
     }
-    const int i = I * 256 + tid, j0 = J * 256 + tid;
-    double xi = 0, yi = 0, zi = 0;
-    if (i < n) { xi = xyz[i * si]; yi = xyz[i * si + sd]; zi = xyz[i * si + 2 * sd]; }
-    if (j0 < n) { jx[tid] = xyz[j0 * si]; jy[tid] = xyz[j0 * si + sd]; jz[tid] = xyz[j0 * si + 2 * sd]; }
-    __syncthreads();
+    constexpr int JN = E == 64 ? 16 : 256;
+    const int i = I * E + (tid & (E - 1)), j0 = J * E + (E == 64 ? wave * JN : 0);
     double s = 0.0;
     if (i < n) {
-        const int jend = min(256, n - J * 256);
-        const int jstart = (I == J) ? tid + 1 : 0;
-        for (int jj = jstart; jj < jend; jj++) {
-            const double d0 = xi - jx[jj], d1 = yi - jy[jj], d2 = zi - jz[jj];
-            const double r = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-            s += a / pow(r, (double)nexp) - b / pow(r, 6.0);     // lennardjones.hh:5-9
+        const double xi = xyz[3 * (size_t)i], yi = xyz[3 * (size_t)i + 1], zi = xyz[3 * (size_t)i + 2];
+        const int jend = min(j0 + JN, n);
+#pragma unroll 2
+        for (int j = j0; j < jend; j++) {
+            const double d0 = xi - xyz[3 * (size_t)j], d1 = yi - xyz[3 * (size_t)j + 1], d2 = zi - xyz[3 * (size_t)j + 2];
+            const double q = d0 * d0 + d1 * d1 + d2 * d2;
+            const double e = a / pow_from_square(q, nexp) - b / (q * q * q);     // lennardjones.hh:5-9
+            s += j > i ? e : 0.0;
         }
     }
 #pragma unroll
@@ -182,6 +198,22 @@ __global__ __launch_bounds__(256) void k_open_potential(const double* __restrict
     if ((tid & 63) == 0) wpart[tid >> 6] = s;
     __syncthreads();
     if (tid == 0) partials[pid] = ((wpart[0] + wpart[1]) + wpart[2]) + wpart[3];
+}
+
+// the sum of the tile partials in a fixed order: 1024 strided sums, then a tree
+__global__ __launch_bounds__(1024) void k_open_sum(const double* __restrict__ partials, int count, double* __restrict__ result)
+{
+    __shared__ double wpart[16];
+    double s = 0.0;
+    for (int k = threadIdx.x; k < count; k += 1024) s += partials[k];
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) s += __shfl_xor(s, m, 64);
+    if ((threadIdx.x & 63) == 0) wpart[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    s = 0.0;
+    for (int k = 0; k < 16; k++) s += wpart[k];
+    *result = s;
 }
 
 // about 2048 workgroups (8 a CU): few enough that adding their histograms to the counters stays small,
@@ -198,38 +230,25 @@ hipError_t launch_rdf(const DevView& v, int chain, int natoms, int nbins, double
     return hipGetLastError();
 }
 
-hipError_t launch_open_potential(const double* xyz_soa, int n, int nexp, double a, double b, double* partials,
-                                 int* nparts, hipStream_t s)
+// 64-tiles while their count fits the partials of 65536 atoms in 256-tiles
+int open_potential_tiles(int n)
 {
-    const int T = (n + 255) / 256;
-    *nparts = T * T;
-    if (T == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_open_potential, dim3(T, T), dim3(256), 0, s, xyz_soa, n, 1, n, nexp, a, b, partials);
-    return hipGetLastError();
+    return n <= kOpenSmall ? (n + 63) / 64 : (n + 255) / 256;
 }
 
-// the partials of k_open_potential summed by one thread in block order (the order of the host sum of
-// chmc_potential_energy_open, so both entry points return the same bits); the lower-triangle blocks
-// hold +0.0 and are skipped, which leaves every intermediate sum unchanged
-__global__ void k_open_sum(const double* __restrict__ partials, int T, double* __restrict__ result)
+hipError_t launch_open_potential(const double* xyz, int n, int nexp, double a, double b, double* partials, double* result,
+                                 hipStream_t s)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double r = 0.0;
-    for (int I = 0; I < T; I++)
-        for (int J = I; J < T; J++) r += partials[I * T + J];
-    *result = r;
-}
-
-hipError_t launch_open_potential_aos(const double* xyz_aos, int n, int nexp, double a, double b, double* partials,
-                                     double* result, hipStream_t s)
-{
-    const int T = (n + 255) / 256;
+    const int T = open_potential_tiles(n);
     if (T > 0) {
-        hipLaunchKernelGGL(k_open_potential, dim3(T, T), dim3(256), 0, s, xyz_aos, n, 3, 1, nexp, a, b, partials);
+        if (n <= kOpenSmall)
+            hipLaunchKernelGGL(k_open_potential<64>, dim3(T, T), dim3(256), 0, s, xyz, n, nexp, a, b, partials);
+        else
+            hipLaunchKernelGGL(k_open_potential<256>, dim3(T, T), dim3(256), 0, s, xyz, n, nexp, a, b, partials);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(k_open_sum, dim3(1), dim3(64), 0, s, partials, T, result);
+    hipLaunchKernelGGL(k_open_sum, dim3(1), dim3(1024), 0, s, partials, T * T, result);
     return hipGetLastError();
 }
 

@@ -39,3 +39,33 @@ def test_rdf_counts_edges(chmc, N, L, nb, size, lattice):
         e.set_positions(x)
         counts, _ = e.rdf(nb, size)
     assert np.array_equal(counts, _rdf_counts(x, box, nb, size))
+
+
+def _open_sum(x, n, a, b):
+    """(sum over pairs of a / r^n - b / r^6, sum of the terms' magnitudes)"""
+    v = m = 0.0
+    for i in range(len(x) - 1):
+        r = np.sqrt(((x[i + 1:] - x[i]) ** 2).sum(1))
+        p, q = a / r ** float(n), b / r ** 6.0
+        v += (p - q).sum()
+        m += (np.abs(p) + np.abs(q)).sum()
+    return v, m
+
+
+# 64-tiles with remainders up to their last size, the first size of the 256-tiles, and exponents even, odd,
+# zero and negative.  Each term is within ~|n| roundings of the exact one and the sums add ~50 more, so the
+# bound is 1e-13 of the terms' magnitudes
+@pytest.mark.parametrize("N,n", [(2, 12), (3, 9), (63, 12), (64, 7), (65, 1), (130, 0), (200, -2), (257, 12), (1000, 8),
+                                 (16384, 12), (16385, 12)])
+def test_open_potential_edges(chmc, N, n):
+    x = np.ascontiguousarray(_lattice(N, [1.1 * np.ceil(N ** (1 / 3) - 1e-9)] * 3)
+                             + np.random.default_rng(N).uniform(-0.2, 0.2, (N, 3)))
+    got = chmc.potential_energy_open(x, n=n, a=4.0, b=3.0)
+    v, m = _open_sum(x, n, 4.0, 3.0)
+    assert abs(got - v) <= 1e-13 * m, (got, v, m)
+
+
+def test_open_potential_coincident_pair(chmc):
+    x = np.zeros((5, 3))
+    x[2:] = [[1, 0, 0], [0, 1.2, 0], [0, 0, 1.3]]
+    assert np.isnan(chmc.potential_energy_open(x, a=4.0, b=4.0))      # inf - inf, as a / 0 - b / 0
