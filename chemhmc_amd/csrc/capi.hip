@@ -1743,9 +1743,7 @@ static int surr_ensure(chmc_ctx* c)
     HIPCHK(c, dalloc(c, &c->sv.adam_m, kSurrNTrain));
     HIPCHK(c, dalloc(c, &c->sv.adam_v, kSurrNTrain));
     HIPCHK(c, dalloc(c, &c->sv.nb_n, N));
-    HIPCHK(c, dalloc(c, &c->sv.nb_j, N * kSurrMaxNb));
     HIPCHK(c, dalloc(c, &c->sv.nb_d, N * kSurrMaxNb));
-    HIPCHK(c, dalloc(c, &c->sv.nb_f, N * kSurrMaxNb));
     HIPCHK(c, dalloc(c, &c->sv.flag, 1));
     HIPCHK(c, dalloc(c, &c->sG, N * kSurrFeat));
     HIPCHK(c, dalloc(c, &c->sg, N * kSurrFeat));
@@ -1782,8 +1780,7 @@ static int surr_descriptors(chmc_ctx* c, float* G)
     int rc = flush_drift(c);
     if (rc) return rc;
     if ((rc = ensure_bins(c))) return rc;
-    HIPCHK(c, launch_surr_pairs(c->v, c->sv, c->stream));
-    HIPCHK(c, launch_surr_desc(c->v, c->sv, G, c->stream));
+    HIPCHK(c, launch_surr_pairs(c->v, c->sv, G, c->stream));
     return CHMC_OK;
 }
 

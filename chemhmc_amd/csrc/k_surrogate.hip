@@ -9,12 +9,12 @@
 //
 // Kernels (all per sorted atom slot, so neighbour references stay valid across them):
 //   k_surr_pairs  one workgroup per cell: 27-cell j-list in LDS (as in the LJ sweep); the pairs within rc
-//                 of each i-atom are appended in j-list order (wave ballot, deterministic) with
-//                 (dx, dy, dz, r, fc, fc') to a fixed-capacity per-atom list
-//   k_surr_desc   32 lanes per atom (one per feature): G_k over the atom's list
+//                 of each i-atom are appended in j-list order (wave ballot, deterministic) with (dx, dy, dz,
+//                 neighbour slot) to a fixed-capacity per-atom list, and G_k summed over them
 //   k_surr_mlp    one wave per 16 atoms: forward and input gradient with v_mfma_f32_16x16x32_bf16
 //                 (4 + 8 MFMAs forward, 8 + 4 backward); weights staged in LDS in both orientations
-//   k_surr_force  32 lanes per atom: per-lane partial of the pair sum, one butterfly per atom; kicks p
+//   k_surr_force  32 lanes per atom: pairs staged in LDS, per-lane partial of the pair sum, one butterfly per
+//                 atom; kicks p
 //   k_surr_grad   training: MFMA forward on 32 atoms per workgroup, per-atom energy residuals, FP32
 //                 parameter gradients accumulated in LDS -> per-workgroup partials
 //   k_surr_adam   sums the partials in workgroup order and applies Adam (Kingma & Ba) to the FP32
@@ -39,16 +39,23 @@ __device__ __forceinline__ float dsilu_f(float a)
 // --------------------------------------------------------------------------------------------------
 // pair list
 // --------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_surr_pairs(DevView v, SurrView s)
+// Pair list and descriptors.  One workgroup per cell, one wave per i atom: its 64 lanes test 64 staged j atoms
+// a step and the hits go, by ballot prefix, to an LDS list of staged positions; then, 64 hits at a time and
+// densely, their geometry (dx, dy, dz, neighbour slot) goes to the atom's global list and (r, fc) to LDS, and
+// the descriptors follow with lane = (feature, every second pair).  Bound: VALU issue (402 candidate tests and
+// 32 x 55 Gaussians an atom) and the 16 B a pair written.  N = 32768, rho* = 0.84: 35.6 us; before, the test
+// loop paid the root, sine and cosine of each hit at 14 % of its lanes and wrote 28 B a pair (38 us), and a
+// second kernel read them back one pair a step (40 us).
+__global__ __launch_bounds__(256) void k_surr_pairs(DevView v, SurrView s, float* __restrict__ G_out)
 {
-    constexpr int IS = 4, JG = 16, NT = 256, W = 4;
-    __shared__ float4 sj[kMaxJ];
-    __shared__ int sidx[kMaxJ];
+    constexpr int NT = 256, W = 4;
+    __shared__ float4 sj[kMaxJ];                      // (x, y, z, sorted slot) seen from the i cell's origin
+    __shared__ unsigned short hl[W][kSurrMaxNb];      // staged positions of the wave's hits
+    __shared__ float2 rf[W][kSurrMaxNb];              // their r and fc
     __shared__ int seg_beg[27], seg_pref[28];
     __shared__ float seg_sh[27][3];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c = blockIdx.x;
-    if (c >= v.Ctot) return;
+    const int c = xcd_block(blockIdx.x, v.Ctot);
     const ChainDev& C = v.chains[v.cell_chain[c]];
     const int nx = C.nbin[0], ny = C.nbin[1], nz = C.nbin[2];
     const int lc = c - C.cell_off;
@@ -88,97 +95,139 @@ __global__ __launch_bounds__(256) void k_surr_pairs(DevView v, SurrView s)
             if (k + step < 27 && seg_pref[k + step] <= t) k += step;
         const int src = seg_beg[k] + (t - seg_pref[k]);
         const float4 q = v.xs[src];
-        sj[t] = make_float4(q.x + seg_sh[k][0], q.y + seg_sh[k][1], q.z + seg_sh[k][2], 0.f);
-        sidx[t] = src;
+        sj[t] = make_float4(q.x + seg_sh[k][0], q.y + seg_sh[k][1], q.z + seg_sh[k][2], __int_as_float(src));
     }
     __syncthreads();
     const float rc2 = C.rc2_f, rc = sqrtf(C.rc2_f);
-    const int ii = lane % IS, g = lane / IS;
-    unsigned long long pattern = 0;
-    for (int q = 0; q < JG; q++) pattern |= 1ull << (q * IS + ii);
-    const int nchunk = (ni + IS - 1) / IS;
-    for (int chunk = wave; chunk < nchunk; chunk += W) {
-        const int i = chunk * IS + ii;
-        const bool ival = i < ni;
-        const int slot = ibeg + (ival ? i : ni - 1);
+    const float mu = mu_k(lane & 31), c2 = 1.0f / (2.0f * kSurrWidth * kSurrWidth);
+    for (int i = wave; i < ni; i += W) {
+        const int slot = ibeg + i;
         const float4 xi = v.xs[slot];
         int count = 0;
-        for (int j0 = 0; j0 < nj; j0 += JG) {
-            const int j = j0 + g;
-            bool hit = false;
-            float dx = 0, dy = 0, dz = 0, r2 = 0;
-            if (ival && j < nj) {
-                const float4 q = sj[j];
-                dx = xi.x - q.x; dy = xi.y - q.y; dz = xi.z - q.z;
-                r2 = dx * dx + dy * dy + dz * dz;
-                hit = r2 < rc2 && r2 > 0.f;
-            }
-            const unsigned long long m = __ballot(hit) & pattern;
-            if (hit) {
-                const int pos = count + __popcll(m & ((1ull << lane) - 1ull));
-                if (pos < kSurrMaxNb) {
-                    const float r = sqrtf(r2);
-                    const float a = 3.14159265358979f * r / rc;
-                    const size_t e = (size_t)slot * kSurrMaxNb + pos;
-                    s.nb_d[e] = make_float4(dx, dy, dz, r);
-                    s.nb_f[e] = make_float2(0.5f * (__cosf(a) + 1.0f), -0.5f * 3.14159265358979f / rc * __sinf(a));
-                    s.nb_j[e] = sidx[j];
-                }
-            }
+        for (int j0 = 0; j0 < nj; j0 += 64) {
+            const int j = j0 + lane;
+            const float4 q = sj[min(j, nj - 1)];
+            const float dx = xi.x - q.x, dy = xi.y - q.y, dz = xi.z - q.z;
+            const float r2 = dx * dx + dy * dy + dz * dz;
+            const bool hit = j < nj && r2 < rc2 && r2 > 0.f;
+            const unsigned long long m = __ballot(hit);
+            const int pos = count + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+            if (hit && pos < kSurrMaxNb) hl[wave][pos] = (unsigned short)j;
             count += __popcll(m);
         }
-        if (ival && g == 0) {
-            s.nb_n[slot] = min(count, kSurrMaxNb);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int n = min(count, kSurrMaxNb);
+        for (int k = lane; k < n; k += 64) {
+            const float4 q = sj[hl[wave][k]];
+            const float dx = xi.x - q.x, dy = xi.y - q.y, dz = xi.z - q.z;
+            const float r = sqrtf(dx * dx + dy * dy + dz * dz);
+            s.nb_d[(size_t)slot * kSurrMaxNb + k] = make_float4(dx, dy, dz, q.w);
+            rf[wave][k] = make_float2(r, 0.5f * (__cosf(3.14159265358979f * r / rc) + 1.0f));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        float acc = 0.f;
+#pragma unroll 4
+        for (int k = lane >> 5; k < n; k += 2) {
+            const float2 q = rf[wave][k];
+            const float t = q.x - mu;
+            acc = __builtin_fmaf(__expf(-t * t * c2), q.y, acc);
+        }
+        acc += __shfl_xor(acc, 32, 64);
+        if (lane < 32) G_out[(size_t)slot * kSurrFeat + lane] = acc;
+        __builtin_amdgcn_wave_barrier();              // the lists are read before the next atom's hits replace them
+        if (lane == 0) {
+            s.nb_n[slot] = n;
             if (count > kSurrMaxNb) atomicOr(s.flag, 1);
         }
     }
 }
 
-// --------------------------------------------------------------------------------------------------
-// descriptors: 32 lanes per atom
-// --------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_surr_desc(DevView v, SurrView s, float* __restrict__ G_out)
+// The kernels over the pair list run 32 lanes an atom, one per feature, eight atoms a workgroup.  The lanes
+// first take one pair each (r, fc and fc' from the stored geometry) and leave what the feature loop needs in
+// LDS, from where every lane reads each pair: a global load of one pair for all 32 lanes moves the same 512
+// bytes as 32 different ones, and those loads bound the loops: at N = 32768 the force-matching residual took
+// 135 us and its v 99, now 48 and 23.
+struct SurrPair {
+    float4 d;                     // dx, dy, dz, neighbour slot
+    float r, fc, dfc, ir;         // distance, cutoff function and its derivative, 1 / r
+};
+__device__ __forceinline__ SurrPair load_pair(const SurrView& s, size_t e, float rc)
 {
-    const int a = blockIdx.x * 8 + (threadIdx.x >> 5);
-    const int f = threadIdx.x & 31;
-    if (a >= v.Ntot) return;
-    const float mu = mu_k(f), c2 = 1.0f / (2.0f * kSurrWidth * kSurrWidth);
-    const int n = s.nb_n[a];
-    float acc = 0.f;
+    SurrPair p;
+    p.d = s.nb_d[e];
+    p.r = sqrtf(p.d.x * p.d.x + p.d.y * p.d.y + p.d.z * p.d.z);
+    const float a = 3.14159265358979f * p.r / rc;
+    p.fc = 0.5f * (__cosf(a) + 1.0f);
+    p.dfc = -0.5f * 3.14159265358979f / rc * __sinf(a);
+    p.ir = 1.0f / p.r;
+    return p;
+}
+__device__ __forceinline__ void half_wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// one staged pair of the surrogate force: (r, fc', fc / w^2, neighbour slot) and (dx, dy, dz) / r
+struct SurrForcePairs {
+    float4 a[8][kSurrMaxNb], u[8][kSurrMaxNb];
+};
+
+// sum over the staged pairs of [g_f(i) + g_f(j)] phi_f'(r) (dx, dy, dz) / r, feature f of each lane
+__device__ __forceinline__ float3 surr_force_sum(const SurrForcePairs& st, int row, int n, const float* __restrict__ g,
+                                                 float gi, int f, float mu)
+{
+    const float c2 = 1.0f / (2.0f * kSurrWidth * kSurrWidth);
+    float fx = 0.f, fy = 0.f, fz = 0.f;
+#pragma unroll 4
     for (int q = 0; q < n; q++) {
-        const size_t e = (size_t)a * kSurrMaxNb + q;
-        const float r = s.nb_d[e].w, fc = s.nb_f[e].x;
-        const float t = r - mu;
-        acc += __expf(-t * t * c2) * fc;
+        const float4 a = st.a[row][q], u = st.u[row][q];
+        const float gj = g[(size_t)__float_as_int(a.w) * kSurrFeat + f];
+        const float t = a.x - mu;
+        const float term = (gi + gj) * (__expf(-t * t * c2) * (a.y - t * a.z));
+        fx = __builtin_fmaf(term, u.x, fx);
+        fy = __builtin_fmaf(term, u.y, fy);
+        fz = __builtin_fmaf(term, u.z, fz);
     }
-    G_out[(size_t)a * kSurrFeat + f] = acc;
+    return make_float3(fx, fy, fz);
 }
 
 // --------------------------------------------------------------------------------------------------
 // MLP forward + input gradient on the MFMA units
 // --------------------------------------------------------------------------------------------------
+// LDS rows are padded by 8 entries (16 bytes): fragment reads take 16 bytes from each of 16 rows, which at the
+// unpadded strides of 64 and 128 bytes fall on 4 or 2 distinct bank groups
+constexpr int kLdF = kSurrFeat + 8, kLdH = kSurrHid + 8;
+
+template <int W>
 struct alignas(16) MlpSmem {
-    __bf16 W1[kSurrHid][kSurrFeat];      // [out][in]
-    __bf16 W1T[kSurrFeat][kSurrHid];
-    __bf16 W2[kSurrHid][kSurrHid];
-    __bf16 W2T[kSurrHid][kSurrHid];
+    __bf16 W1[kSurrHid][kLdF];           // [out][in]
+    __bf16 W1T[kSurrFeat][kLdH];
+    __bf16 W2[kSurrHid][kLdH];
+    __bf16 W2T[kSurrHid][kLdH];
+    __bf16 act[W][16][kLdH];             // per-wave transpose buffer (D layout -> A layout)
     float b1[kSurrHid], b2[kSurrHid], w3[kSurrHid], shift[kSurrFeat], scale[kSurrFeat];
     float b3;
-    __bf16 act[4][16][kSurrHid];         // per-wave transpose buffer (D layout -> A layout)
 };
 
-__device__ void load_weights(MlpSmem& sm, const SurrView& s)
+template <typename Smem>
+__device__ void load_weights(Smem& sm, const SurrView& s)
 {
-    // the four bf16 matrices (both orientations are kept in global memory) in 16-byte pieces
-    auto copy16 = [&](void* dst, const void* src, int bytes) {
+    // the four bf16 matrices (both orientations are kept in global memory) in 16-byte pieces, row by row
+    auto copy16 = [&](auto& dst, const void* src, int cols) {
         const uint4* q = static_cast<const uint4*>(src);
-        uint4* d = static_cast<uint4*>(dst);
-        for (int t = threadIdx.x; t < bytes / 16; t += blockDim.x) d[t] = q[t];
+        const int per = cols / 8, n = (int)(sizeof(dst) / sizeof(dst[0])) * per;
+        for (int t = threadIdx.x; t < n; t += blockDim.x) *reinterpret_cast<uint4*>(&dst[t / per][8 * (t % per)]) = q[t];
     };
-    copy16(&sm.W1[0][0], s.w1b, kSurrHid * kSurrFeat * 2);
-    copy16(&sm.W1T[0][0], s.w1tb, kSurrHid * kSurrFeat * 2);
-    copy16(&sm.W2[0][0], s.w2b, kSurrHid * kSurrHid * 2);
-    copy16(&sm.W2T[0][0], s.w2tb, kSurrHid * kSurrHid * 2);
+    copy16(sm.W1, s.w1b, kSurrFeat);
+    copy16(sm.W1T, s.w1tb, kSurrHid);
+    copy16(sm.W2, s.w2b, kSurrHid);
+    copy16(sm.W2T, s.w2tb, kSurrHid);
     const float* P = s.params;
     for (int t = threadIdx.x; t < kSurrHid; t += blockDim.x) {
         sm.b1[t] = P[kOffB1 + t];
@@ -211,7 +260,8 @@ struct WaveOut {
     float e[4];             // per-atom energies of the lane's 4 rows (valid in lanes with l%16 == 0 after reduce)
 };
 
-__device__ void mlp_forward_wave(MlpSmem& sm, const float* __restrict__ G, int a0, int natoms, WaveOut& o)
+template <typename Smem>
+__device__ void mlp_forward_wave(Smem& sm, const float* __restrict__ G, int a0, int natoms, WaveOut& o)
 {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
     // z = bf16((G - shift) * scale), A layout: row m = l%16 (atom a0+m), k = 8*(l/16)..+7
@@ -228,7 +278,7 @@ __device__ void mlp_forward_wave(MlpSmem& sm, const float* __restrict__ G, int a
     // layer 1: 4 column tiles of 16 hidden units, K = 32
 #pragma unroll
     for (int t = 0; t < 4; t++) {
-        const bf16x8 wb = frag_rows(&sm.W1[16 * t][0], kSurrFeat, 0);
+        const bf16x8 wb = frag_rows(&sm.W1[16 * t][0], kLdF, 0);
         f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(za, wb, acc, 0, 0, 0);
         const int n = 16 * t + (l & 15);
@@ -243,14 +293,14 @@ __device__ void mlp_forward_wave(MlpSmem& sm, const float* __restrict__ G, int a
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     // layer 2: K = 64 (two k tiles), 4 column tiles
-    const bf16x8 h1a0 = frag_rows(&sm.act[w][0][0], kSurrHid, 0);
-    const bf16x8 h1a1 = frag_rows(&sm.act[w][0][0], kSurrHid, 32);
+    const bf16x8 h1a0 = frag_rows(&sm.act[w][0][0], kLdH, 0);
+    const bf16x8 h1a1 = frag_rows(&sm.act[w][0][0], kLdH, 32);
     float part[4] = { 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h1a0, frag_rows(&sm.W2[16 * t][0], kSurrHid, 0), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h1a1, frag_rows(&sm.W2[16 * t][0], kSurrHid, 32), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h1a0, frag_rows(&sm.W2[16 * t][0], kLdH, 0), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h1a1, frag_rows(&sm.W2[16 * t][0], kLdH, 32), acc, 0, 0, 0);
         const int n = 16 * t + (l & 15);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -270,7 +320,8 @@ __device__ void mlp_forward_wave(MlpSmem& sm, const float* __restrict__ G, int a
 }
 
 // backward from d2 = de * w3 * silu'(a2) to d1 = (d2 W2) * silu'(a1), d2 and d1 in D layout
-__device__ void mlp_backward_wave(MlpSmem& sm, const WaveOut& o, const float de[4], f32x4 d2[4], f32x4 d1[4])
+template <typename Smem>
+__device__ void mlp_backward_wave(Smem& sm, const WaveOut& o, const float de[4], f32x4 d2[4], f32x4 d1[4])
 {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
     __builtin_amdgcn_wave_barrier();
@@ -286,13 +337,13 @@ __device__ void mlp_backward_wave(MlpSmem& sm, const WaveOut& o, const float de[
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const bf16x8 d2a0 = frag_rows(&sm.act[w][0][0], kSurrHid, 0);
-    const bf16x8 d2a1 = frag_rows(&sm.act[w][0][0], kSurrHid, 32);
+    const bf16x8 d2a0 = frag_rows(&sm.act[w][0][0], kLdH, 0);
+    const bf16x8 d2a1 = frag_rows(&sm.act[w][0][0], kLdH, 32);
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d2a0, frag_rows(&sm.W2T[16 * t][0], kSurrHid, 0), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d2a1, frag_rows(&sm.W2T[16 * t][0], kSurrHid, 32), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d2a0, frag_rows(&sm.W2T[16 * t][0], kLdH, 0), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d2a1, frag_rows(&sm.W2T[16 * t][0], kLdH, 32), acc, 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < 4; i++) d1[t][i] = acc[i] * dsilu_f(o.a1[t][i]);
     }
@@ -301,7 +352,7 @@ __device__ void mlp_backward_wave(MlpSmem& sm, const WaveOut& o, const float de[
 __global__ __launch_bounds__(256) void k_surr_mlp(DevView v, SurrView s, const float* __restrict__ G,
                                                    float* __restrict__ g_out, float* __restrict__ e_out)
 {
-    __shared__ MlpSmem sm;
+    __shared__ MlpSmem<4> sm;
     load_weights(sm, s);
     __syncthreads();
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -330,13 +381,13 @@ __global__ __launch_bounds__(256) void k_surr_mlp(DevView v, SurrView s, const f
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const bf16x8 d1a0 = frag_rows(&sm.act[w][0][0], kSurrHid, 0);
-    const bf16x8 d1a1 = frag_rows(&sm.act[w][0][0], kSurrHid, 32);
+    const bf16x8 d1a0 = frag_rows(&sm.act[w][0][0], kLdH, 0);
+    const bf16x8 d1a1 = frag_rows(&sm.act[w][0][0], kLdH, 32);
 #pragma unroll
     for (int t = 0; t < 2; t++) {
         f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d1a0, frag_rows(&sm.W1T[16 * t][0], kSurrHid, 0), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d1a1, frag_rows(&sm.W1T[16 * t][0], kSurrHid, 32), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d1a0, frag_rows(&sm.W1T[16 * t][0], kLdH, 0), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d1a1, frag_rows(&sm.W1T[16 * t][0], kLdH, 32), acc, 0, 0, 0);
         const int n = 16 * t + (l & 15);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -352,26 +403,21 @@ __global__ __launch_bounds__(256) void k_surr_mlp(DevView v, SurrView s, const f
 __global__ __launch_bounds__(256) void k_surr_force(DevView v, SurrView s, const float* __restrict__ g,
                                                     double kick_dt, int store)
 {
-    const int a = blockIdx.x * 8 + (threadIdx.x >> 5);
+    __shared__ SurrForcePairs st;
+    const int row = threadIdx.x >> 5, a = blockIdx.x * 8 + row;
     const int f = threadIdx.x & 31;
     if (a >= v.Ntot) return;
-    const float mu = mu_k(f), c2 = 1.0f / (2.0f * kSurrWidth * kSurrWidth), iw2 = 1.0f / (kSurrWidth * kSurrWidth);
-    const float gi = g[(size_t)a * kSurrFeat + f];
+    const ChainDev& C = v.chains[v.atom_chain[__float_as_int(v.xs[a].w)]];
+    const float iw2 = 1.0f / (kSurrWidth * kSurrWidth), rc = sqrtf(C.rc2_f);
     const int n = s.nb_n[a];
-    float fx = 0.f, fy = 0.f, fz = 0.f;
-    for (int q = 0; q < n; q++) {
-        const size_t e = (size_t)a * kSurrMaxNb + q;
-        const float4 d = s.nb_d[e];
-        const float2 fc = s.nb_f[e];
-        const int j = s.nb_j[e];
-        const float t = d.w - mu;
-        const float ex = __expf(-t * t * c2);
-        const float dphi = ex * (fc.y - t * iw2 * fc.x);
-        const float term = (gi + g[(size_t)j * kSurrFeat + f]) * dphi / d.w;
-        fx += term * d.x;
-        fy += term * d.y;
-        fz += term * d.z;
+    for (int q = f; q < n; q += 32) {
+        const SurrPair p = load_pair(s, (size_t)a * kSurrMaxNb + q, rc);
+        st.a[row][q] = make_float4(p.r, p.dfc, iw2 * p.fc, p.d.w);
+        st.u[row][q] = make_float4(p.d.x * p.ir, p.d.y * p.ir, p.d.z * p.ir, 0.f);
     }
+    half_wave_lds_sync();
+    float3 F = surr_force_sum(st, row, n, g, g[(size_t)a * kSurrFeat + f], f, mu_k(f));
+    float fx = F.x, fy = F.y, fz = F.z;
 #pragma unroll
     for (int m = 1; m < 32; m <<= 1) {
         fx += __shfl_xor(fx, m, 64);
@@ -380,7 +426,6 @@ __global__ __launch_bounds__(256) void k_surr_force(DevView v, SurrView s, const
     }
     if (f == 0) {
         const int atom = __float_as_int(v.xs[a].w);
-        const ChainDev& C = v.chains[v.atom_chain[atom]];
         const int N = v.Ntot;
         const float f3[3] = { fx, fy, fz };
         const double kdt = kick_dt * C.beta;
@@ -398,7 +443,7 @@ __global__ __launch_bounds__(256) void k_surr_force(DevView v, SurrView s, const
 constexpr int kGradRows = 32;          // atoms per training workgroup (2 waves x 16)
 
 struct GradSmem {
-    MlpSmem m;
+    MlpSmem<2> m;
     float d2[kGradRows][kSurrHid];
     float d1[kGradRows][kSurrHid];
     __bf16 h1[kGradRows][kSurrHid];
@@ -479,16 +524,37 @@ __global__ __launch_bounds__(128) void k_surr_grad(SurrView s, const float* __re
     }
 }
 
-// fixed-order sum of the workgroup partials (no update): gradient checks against the oracle
-// (partials of ngrad floats: the trained parameters, then ngrad - kSurrNTrain loss sums)
-__global__ __launch_bounds__(256) void k_surr_sum(const float* __restrict__ partial, int nparts, int ngrad,
-                                                  float* __restrict__ out)
+// Fixed-order sum of the workgroup partials (partials of ngrad floats: the trained parameters, then
+// ngrad - kSurrNTrain loss sums): 64 consecutive entries per workgroup of 16 waves, wave w the partials
+// w, w + 16, ..., then the 16 wave sums in order.  Returns the sum of entry p = 64 blockIdx + lane in wave 0.
+// (One thread an entry summing all partials was a chain of 256 load latencies on 25 workgroups: the Adam
+// step took 63 us at 256 partials, now 5.4; bound: latency and the 6.5 MB of partials.)
+__device__ __forceinline__ float partial_sum(const float* __restrict__ partial, int nparts, int ngrad)
 {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= ngrad) return;
-    float gsum = 0.f;
-    for (int b = 0; b < nparts; b++) gsum += partial[(size_t)b * ngrad + p];
-    out[p] = gsum;
+    __shared__ float ws[16][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane;
+    float g = 0.f;
+    if (p < ngrad) {
+#pragma unroll 8
+        for (int b = w; b < nparts; b += 16) g += partial[(size_t)b * ngrad + p];
+    }
+    ws[w][lane] = g;
+    __syncthreads();
+    if (w != 0) return 0.f;
+    g = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; k++) g += ws[k][lane];
+    return g;
+}
+
+// the summed gradient without an update: gradient checks against the oracle
+__global__ __launch_bounds__(1024) void k_surr_sum(const float* __restrict__ partial, int nparts, int ngrad,
+                                                   float* __restrict__ out)
+{
+    const int p = blockIdx.x * 64 + threadIdx.x;
+    const float gsum = partial_sum(partial, nparts, ngrad);
+    if (threadIdx.x < 64 && p < ngrad) out[p] = gsum;
 }
 
 // the bfloat16 copies (both orientations) of W1 / W2 entry p of the parameter blob
@@ -505,15 +571,14 @@ __device__ __forceinline__ void store_bf16_weight(const SurrView& s, int p, floa
     }
 }
 
-// one thread per trainable parameter: fixed-order sum over workgroup partials, then Adam
-__global__ __launch_bounds__(256) void k_surr_adam(SurrView s, const float* __restrict__ partial, int nparts, int ngrad,
-                                                   float lr, float beta1, float beta2, float eps, int step,
-                                                   float* __restrict__ loss_out)
+// the fixed-order sum over workgroup partials, then Adam, one lane of wave 0 per trainable parameter
+__global__ __launch_bounds__(1024) void k_surr_adam(SurrView s, const float* __restrict__ partial, int nparts, int ngrad,
+                                                    float lr, float beta1, float beta2, float eps, int step,
+                                                    float* __restrict__ loss_out)
 {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= ngrad) return;
-    float gsum = 0.f;
-    for (int b = 0; b < nparts; b++) gsum += partial[(size_t)b * ngrad + p];
+    const int p = blockIdx.x * 64 + threadIdx.x;
+    const float gsum = partial_sum(partial, nparts, ngrad);
+    if (threadIdx.x >= 64 || p >= ngrad) return;
     if (p >= kSurrNTrain) {                      // the loss slots
         if (loss_out) loss_out[p - kSurrNTrain] = gsum;
         return;
@@ -544,7 +609,8 @@ __global__ __launch_bounds__(256) void k_surr_targets(DevView v, SurrView s, flo
     double acc = 0.0;
     const int n = s.nb_n[a];
     for (int q = 0; q < n; q++) {
-        const double r = s.nb_d[(size_t)a * kSurrMaxNb + q].w;
+        const float4 d = s.nb_d[(size_t)a * kSurrMaxNb + q];
+        const double r = sqrtf(d.x * d.x + d.y * d.y + d.z * d.z);
         const double sr2 = C.sigma2 / (r * r);
         const double sr6 = sr2 * sr2 * sr2;
         acc += sr6 * (sr6 - 1.0);
@@ -553,7 +619,8 @@ __global__ __launch_bounds__(256) void k_surr_targets(DevView v, SurrView s, flo
 }
 
 // D layout -> bf16 A-layout transpose buffer of this wave, then the two K = 32 fragments of a 64-wide row
-__device__ __forceinline__ void act_store(MlpSmem& sm, const f32x4 x[4])
+template <typename Smem>
+__device__ __forceinline__ void act_store(Smem& sm, const f32x4 x[4])
 {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
     __builtin_amdgcn_wave_barrier();
@@ -567,16 +634,17 @@ __device__ __forceinline__ void act_store(MlpSmem& sm, const f32x4 x[4])
 }
 
 // x[16 rows][64] (act buffer) times a 64 x 64 bf16 matrix given by rows B[n][k] (B = W2: x W2^T; B = W2T: x W2)
-__device__ __forceinline__ void act_times(MlpSmem& sm, const __bf16* B, f32x4 out[4])
+template <typename Smem>
+__device__ __forceinline__ void act_times(Smem& sm, const __bf16* B, f32x4 out[4])
 {
     const int w = threadIdx.x >> 6;
-    const bf16x8 a0 = frag_rows(&sm.act[w][0][0], kSurrHid, 0);
-    const bf16x8 a1 = frag_rows(&sm.act[w][0][0], kSurrHid, 32);
+    const bf16x8 a0 = frag_rows(&sm.act[w][0][0], kLdH, 0);
+    const bf16x8 a1 = frag_rows(&sm.act[w][0][0], kLdH, 32);
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, frag_rows(B + 16 * t * kSurrHid, kSurrHid, 0), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, frag_rows(B + 16 * t * kSurrHid, kSurrHid, 32), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, frag_rows(B + 16 * t * kLdH, kLdH, 0), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, frag_rows(B + 16 * t * kLdH, kLdH, 32), acc, 0, 0, 0);
         out[t] = acc;
     }
 }
@@ -596,7 +664,7 @@ template <bool W16>
 __global__ __launch_bounds__(256) void k_lsurr_desc_mlp(DevView v, SurrView s, int q, float* __restrict__ g_out,
                                                         float* __restrict__ e_out, float* __restrict__ G_out)
 {
-    __shared__ MlpSmem sm;
+    __shared__ MlpSmem<2> sm;
     __shared__ float sG[32][kSurrFeat];
     __shared__ float srd[32][kDescPairCap];
     __shared__ int4 seg_tab[W16 ? 32 : 1][kSegStride / 4];   // W16: segment starts of each slot's cell
@@ -683,13 +751,13 @@ __global__ __launch_bounds__(256) void k_lsurr_desc_mlp(DevView v, SurrView s, i
     f32x4 d2[4], d1[4];
     mlp_backward_wave(sm, o, one, d2, d1);
     act_store(sm, d1);
-    const bf16x8 d1a0 = frag_rows(&sm.act[w][0][0], kSurrHid, 0);
-    const bf16x8 d1a1 = frag_rows(&sm.act[w][0][0], kSurrHid, 32);
+    const bf16x8 d1a0 = frag_rows(&sm.act[w][0][0], kLdH, 0);
+    const bf16x8 d1a1 = frag_rows(&sm.act[w][0][0], kLdH, 32);
 #pragma unroll
     for (int t = 0; t < 2; t++) {
         f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d1a0, frag_rows(&sm.W1T[16 * t][0], kSurrHid, 0), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d1a1, frag_rows(&sm.W1T[16 * t][0], kSurrHid, 32), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d1a0, frag_rows(&sm.W1T[16 * t][0], kLdH, 0), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d1a1, frag_rows(&sm.W1T[16 * t][0], kLdH, 32), acc, 0, 0, 0);
         const int n = 16 * t + (l & 15);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -715,39 +783,32 @@ __device__ __forceinline__ float d2silu_f(float a)
 __global__ __launch_bounds__(256) void k_surr_fm_resid(DevView v, SurrView s, const float* __restrict__ g,
                                                        float4* __restrict__ R, float* __restrict__ u_out)
 {
-    const int a = blockIdx.x * 8 + (threadIdx.x >> 5);
+    __shared__ SurrForcePairs st;
+    const int row = threadIdx.x >> 5, a = blockIdx.x * 8 + row;
     const int f = threadIdx.x & 31;
     if (a >= v.Ntot) return;
     const int atom = __float_as_int(v.xs[a].w);
     const ChainDev& C = v.chains[v.atom_chain[atom]];
-    const float mu = mu_k(f), c2 = 1.0f / (2.0f * kSurrWidth * kSurrWidth), iw2 = 1.0f / (kSurrWidth * kSurrWidth);
-    const float gi = g[(size_t)a * kSurrFeat + f];
+    const float iw2 = 1.0f / (kSurrWidth * kSurrWidth), rc = sqrtf(C.rc2_f);
     const float sig2 = (float)C.sigma2, c48 = (float)(48.0 * C.eps);
     const int n = s.nb_n[a];
-    float ex_ = 0.f, ey = 0.f, ez = 0.f, lx = 0.f, ly = 0.f, lz = 0.f;
+    float lx = 0.f, ly = 0.f, lz = 0.f;
     double uacc = 0.0;
-    for (int q = 0; q < n; q++) {
-        const size_t e = (size_t)a * kSurrMaxNb + q;
-        const float4 d = s.nb_d[e];
-        const float2 fc = s.nb_f[e];
-        const int j = s.nb_j[e];
-        const float t = d.w - mu;
-        const float ex = __expf(-t * t * c2);
-        const float dphi = ex * (fc.y - t * iw2 * fc.x);
-        const float term = (gi + g[(size_t)j * kSurrFeat + f]) * dphi / d.w;
-        ex_ += term * d.x;
-        ey += term * d.y;
-        ez += term * d.z;
-        if ((q & 31) == f) {
-            const float sr2 = sig2 / (d.w * d.w), sr6 = sr2 * sr2 * sr2;
-            const float cf = c48 * sr6 * (0.5f - sr6) / (d.w * d.w);
-            lx += cf * d.x;
-            ly += cf * d.y;
-            lz += cf * d.z;
-            const double r = d.w, dr2 = C.sigma2 / (r * r), dr6 = dr2 * dr2 * dr2;
-            uacc += dr6 * (dr6 - 1.0);
-        }
+    for (int q = f; q < n; q += 32) {
+        const SurrPair p = load_pair(s, (size_t)a * kSurrMaxNb + q, rc);
+        st.a[row][q] = make_float4(p.r, p.dfc, iw2 * p.fc, p.d.w);
+        st.u[row][q] = make_float4(p.d.x * p.ir, p.d.y * p.ir, p.d.z * p.ir, 0.f);
+        const float sr2 = sig2 / (p.r * p.r), sr6 = sr2 * sr2 * sr2;
+        const float cf = c48 * sr6 * (0.5f - sr6) / (p.r * p.r);
+        lx += cf * p.d.x;
+        ly += cf * p.d.y;
+        lz += cf * p.d.z;
+        const double r = p.r, dr2 = C.sigma2 / (r * r), dr6 = dr2 * dr2 * dr2;
+        uacc += dr6 * (dr6 - 1.0);
     }
+    half_wave_lds_sync();
+    const float3 F = surr_force_sum(st, row, n, g, g[(size_t)a * kSurrFeat + f], f, mu_k(f));
+    float ex_ = F.x, ey = F.y, ez = F.z;
 #pragma unroll
     for (int m = 1; m < 32; m <<= 1) {
         ex_ += __shfl_xor(ex_, m, 64);
@@ -769,36 +830,51 @@ __global__ __launch_bounds__(256) void k_surr_fm_resid(DevView v, SurrView s, co
 __global__ __launch_bounds__(256) void k_surr_fm_v(DevView v, SurrView s, const float4* __restrict__ R, float cw,
                                                    float* __restrict__ vout)
 {
-    const int a = blockIdx.x * 8 + (threadIdx.x >> 5);
+    __shared__ float4 st[8][kSurrMaxNb];              // (r, fc' s, fc s / w^2), s = (d / r) . (R_i - R_j)
+    const int row = threadIdx.x >> 5, a = blockIdx.x * 8 + row;
     const int f = threadIdx.x & 31;
     if (a >= v.Ntot) return;
+    const ChainDev& C = v.chains[v.atom_chain[__float_as_int(v.xs[a].w)]];
     const float mu = mu_k(f), c2 = 1.0f / (2.0f * kSurrWidth * kSurrWidth), iw2 = 1.0f / (kSurrWidth * kSurrWidth);
+    const float rc = sqrtf(C.rc2_f);
     const float4 Ri = R[a];
     const int n = s.nb_n[a];
+    for (int q = f; q < n; q += 32) {
+        const SurrPair p = load_pair(s, (size_t)a * kSurrMaxNb + q, rc);
+        const float4 Rj = R[__float_as_int(p.d.w)];
+        const float sc = (p.d.x * (Ri.x - Rj.x) + p.d.y * (Ri.y - Rj.y) + p.d.z * (Ri.z - Rj.z)) * p.ir;
+        st[row][q] = make_float4(p.r, p.dfc * sc, iw2 * p.fc * sc, 0.f);
+    }
+    half_wave_lds_sync();
     float acc = 0.f;
+#pragma unroll 4
     for (int q = 0; q < n; q++) {
-        const size_t e = (size_t)a * kSurrMaxNb + q;
-        const float4 d = s.nb_d[e];
-        const float2 fc = s.nb_f[e];
-        const float4 Rj = R[s.nb_j[e]];
-        const float t = d.w - mu;
-        const float dphi = __expf(-t * t * c2) * (fc.y - t * iw2 * fc.x);
-        acc += dphi * (d.x * (Ri.x - Rj.x) + d.y * (Ri.y - Rj.y) + d.z * (Ri.z - Rj.z)) / d.w;
+        const float4 p = st[row][q];
+        const float t = p.x - mu;
+        acc = __builtin_fmaf(__expf(-t * t * c2), p.y - t * p.z, acc);
     }
     vout[(size_t)a * kSurrFeat + f] = cw * acc;
 }
 
-constexpr int kFmRows = 32;            // rows per chunk of the force-matching gradient (2 waves x 16)
+constexpr int kFmRows = 64;            // rows per chunk of the force-matching gradient (4 waves x 16)
+constexpr int kLdR = kFmRows + 8;      // transposed operands, padded rows
+
+// x = p[0] + p[1] + p[2] in bfloat16 pieces of 8 significant bits each (24 in all): the products with a
+// bfloat16 operand, summed in FP32, are those of the FP32 value
+__device__ __forceinline__ void split3(float x, __bf16 p[3])
+{
+    p[0] = (__bf16)x;
+    const float r = x - (float)p[0];
+    p[1] = (__bf16)r;
+    p[2] = (__bf16)(r - (float)p[1]);
+}
 
 struct FmSmem {
-    MlpSmem m;
-    float D1[kFmRows][kSurrHid], D2[kFmRows][kSurrHid];      // de delta + tangent terms
-    float dl1[kFmRows][kSurrHid], dl2[kFmRows][kSurrHid];    // delta1, delta2 (backward of e with de = 1)
-    float q3[kFmRows][kSurrHid];                             // h2 de + silu'(a2) t2  (w3 gradient)
-    __bf16 h1[kFmRows][kSurrHid], ta1[kFmRows][kSurrHid];
-    __bf16 z[kFmRows][kSurrFeat], uu[kFmRows][kSurrFeat];
-    float de[kFmRows];
-    float lsum[2][2];                                        // per wave: sum (e - u)^2, sum |R|^2
+    MlpSmem<4> m;
+    __bf16 d[2][3][kSurrHid][kLdR];    // [unit][row]: D (de delta + tangent terms) and delta, in three pieces
+    __bf16 x[2][kSurrHid][kLdR];       // [input][row]: h1 and ta1 for W2; z and u for W1
+    float bsum[3][4][kSurrHid];        // per wave: the b1, b2 and w3 gradients
+    float ssum[3][4];                  // per wave: sum de, sum (e - u)^2, sum |R|^2
 };
 
 // Gradient of the energy + force-matching loss over rows [0, nrows) (sorted slots of the current
@@ -809,9 +885,13 @@ struct FmSmem {
 //   zb1 = silu''(a1) t1 gamma1 + silu'(a1) ab1, D2 = de delta2 + zb2, D1 = de delta1 + zb1
 //   dW2 = D2^T h1 + delta2^T ta1, dW1 = D1^T z + delta1^T u, db = sum D, dw3 = h2^T de + sum silu'(a2) t2
 // bfloat16 operands of the MFMA products (delta2, u, ta1, zb2) are rounded once and the rounded ta1 and
-// u enter the weight gradients.  Each workgroup takes rows_per_wg consecutive rows in chunks of 32 and
+// u enter the weight gradients.  Each workgroup takes rows_per_wg consecutive rows in chunks of 64 and
 // writes one partial of kSurrNTrain + 2 floats (the last two: sum (e - u)^2 and sum |R|^2).
-__global__ __launch_bounds__(128) void k_surr_grad_fm(SurrView s, const float* __restrict__ G,
+// The weight gradients contract over the rows on the matrix cores: D and delta, FP32, go transposed to LDS in
+// three bfloat16 pieces (split3, exact to 24 bits), the other operand is bfloat16 as it is; wave w owns the
+// 16 output units 16 w of both matrices.  (On the VALU from LDS, 4 x 4 blocks a thread, they were most of the
+// kernel's 100 us at N = 32768; now 30.)  Bound: latency, one workgroup of four waves a CU.
+__global__ __launch_bounds__(256) void k_surr_grad_fm(SurrView s, const float* __restrict__ G,
                                                       const float* __restrict__ u, const float* __restrict__ vin,
                                                       const float4* __restrict__ R, int nrows, int rows_per_wg,
                                                       float two_over_n, float* __restrict__ partial)
@@ -819,17 +899,36 @@ __global__ __launch_bounds__(128) void k_surr_grad_fm(SurrView s, const float* _
     __shared__ FmSmem sm;
     load_weights(sm.m, s);
     const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
-    if (tid < 4) sm.lsum[tid >> 1][tid & 1] = 0.f;
     __syncthreads();
-    // register-blocked weight gradients: blocks b = tid + 128 j of 4 x 4 (W2: b < 256, W1: 256 <= b < 384)
-    float acc[3][4][4];
+    f32x4 acc2[4], acc1[2];
 #pragma unroll
-    for (int j = 0; j < 3; j++)
+    for (int t = 0; t < 4; t++) acc2[t] = f32x4{ 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
-        for (int x = 0; x < 4; x++)
+    for (int t = 0; t < 2; t++) acc1[t] = f32x4{ 0.f, 0.f, 0.f, 0.f };
+    float accb1[4] = { 0.f, 0.f, 0.f, 0.f }, accb2[4] = { 0.f, 0.f, 0.f, 0.f }, accw3[4] = { 0.f, 0.f, 0.f, 0.f };
+    float accb3 = 0.f, le = 0.f, lf = 0.f;
+    // four rows 4 (l / 16) .. + 3 of the wave's 16, unit n: 8 bytes of a transposed row
+    const int mrow = 16 * w + 4 * (l >> 4);
+    auto put4 = [&](__bf16* row, const __bf16 q[4]) { *reinterpret_cast<uint2*>(row + mrow) = *reinterpret_cast<const uint2*>(q); };
+    // acc += A B over the chunk's rows for the wave's 16 units and NT tiles of inputs
+    auto contract = [&](f32x4* acc, auto nt) {
+        constexpr int NT = decltype(nt)::value;
 #pragma unroll
-            for (int y = 0; y < 4; y++) acc[j][x][y] = 0.f;
-    float accb = 0.f, accw3 = 0.f, accb3 = 0.f;
+        for (int k0 = 0; k0 < kFmRows; k0 += 32) {
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                bf16x8 A[3];
+#pragma unroll
+                for (int q = 0; q < 3; q++) A[q] = frag_rows(&sm.d[h][q][16 * w][0], kLdR, k0);
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const bf16x8 B = frag_rows(&sm.x[h][16 * t][0], kLdR, k0);
+#pragma unroll
+                    for (int q = 2; q >= 0; q--) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[q], B, acc[t], 0, 0, 0);
+                }
+            }
+        }
+    };
     const int wg0 = blockIdx.x * rows_per_wg;
     const int wg1 = min(nrows, wg0 + rows_per_wg);
     for (int base = wg0; base < wg1; base += kFmRows) {
@@ -837,12 +936,12 @@ __global__ __launch_bounds__(128) void k_surr_grad_fm(SurrView s, const float* _
         WaveOut o;
         mlp_forward_wave(sm.m, G, r0, wg1, o);
         float de[4];
-        float le = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int rr = r0 + 4 * (l >> 4) + i;
             const float res = rr < wg1 ? o.e[i] - u[rr] : 0.f;
             de[i] = two_over_n * res;
+            accb3 += de[i];
             le += res * res;
         }
         f32x4 s1[4], s2[4], dl2[4], gam[4];
@@ -858,27 +957,23 @@ __global__ __launch_bounds__(128) void k_surr_grad_fm(SurrView s, const float* _
         }
         act_store(sm.m, dl2);
         act_times(sm.m, &sm.m.W2T[0][0], gam);              // gamma1 = bf16(delta2) W2
-        // u = bf16(v * scale) in A layout: row l % 16, features 8 (l / 16) .. + 7
-        bf16x8 ua;
+        // u = bf16(v * scale) and z in A layout: row l % 16, features 8 (l / 16) .. + 7
+        bf16x8 ua, za;
         {
             const int m = l & 15, k0 = 8 * (l >> 4);
             const int rr = r0 + m;
 #pragma unroll
-            for (int i = 0; i < 8; i++)
-                ua[i] = (__bf16)(rr < wg1 ? vin[(size_t)rr * kSurrFeat + k0 + i] * sm.m.scale[k0 + i] : 0.f);
-            const int mm = 16 * w + m;
-#pragma unroll
             for (int i = 0; i < 8; i++) {
-                sm.uu[mm][k0 + i] = ua[i];
+                ua[i] = (__bf16)(rr < wg1 ? vin[(size_t)rr * kSurrFeat + k0 + i] * sm.m.scale[k0 + i] : 0.f);
                 const float gv = rr < wg1 ? G[(size_t)rr * kSurrFeat + k0 + i] : 0.f;
-                sm.z[mm][k0 + i] = (__bf16)((gv - sm.m.shift[k0 + i]) * sm.m.scale[k0 + i]);
+                za[i] = (__bf16)((gv - sm.m.shift[k0 + i]) * sm.m.scale[k0 + i]);
             }
         }
         f32x4 t1[4], ta1[4], t2[4], zb2[4], ab1[4];
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             f32x4 a = { 0.f, 0.f, 0.f, 0.f };
-            t1[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ua, frag_rows(&sm.m.W1[16 * t][0], kSurrFeat, 0), a, 0, 0, 0);
+            t1[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ua, frag_rows(&sm.m.W1[16 * t][0], kLdF, 0), a, 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 4; i++) ta1[t][i] = s1[t][i] * t1[t][i];
         }
@@ -890,137 +985,125 @@ __global__ __launch_bounds__(128) void k_surr_grad_fm(SurrView s, const float* _
 #pragma unroll
             for (int i = 0; i < 4; i++) zb2[t][i] = sm.m.w3[n] * d2silu_f(o.a2[t][i]) * t2[t][i];
         }
-        // rows of ta1 (rounded as the product saw them) into the gradient stage before act is reused
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) sm.ta1[16 * w + 4 * (l >> 4) + i][16 * t + (l & 15)] = (__bf16)ta1[t][i];
         act_store(sm.m, zb2);
         act_times(sm.m, &sm.m.W2T[0][0], ab1);              // ab1 = bf16(zb2) W2
+        // operands of dW2 = D2^T h1 + delta2^T ta1
+        bool valid[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) valid[i] = r0 + 4 * (l >> 4) + i < wg1;
+        f32x4 D1[4], dl1[4];
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             const int n = 16 * t + (l & 15);
+            __bf16 dp[3][4], ep[3][4], hq[4], tq[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int m = 16 * w + 4 * (l >> 4) + i;
-                const bool valid = r0 + 4 * (l >> 4) + i < wg1;
-                const float dl1 = gam[t][i] * s1[t][i];
+                const float dl = gam[t][i] * s1[t][i];
                 const float zb1 = d2silu_f(o.a1[t][i]) * t1[t][i] * gam[t][i] + s1[t][i] * ab1[t][i];
                 const float h2 = (float)(__bf16)silu_f(o.a2[t][i]);
-                sm.D1[m][n] = valid ? de[i] * dl1 + zb1 : 0.f;
-                sm.D2[m][n] = valid ? de[i] * dl2[t][i] + zb2[t][i] : 0.f;
-                sm.dl1[m][n] = valid ? dl1 : 0.f;
-                sm.dl2[m][n] = valid ? dl2[t][i] : 0.f;
-                sm.q3[m][n] = valid ? h2 * de[i] + s2[t][i] * t2[t][i] : 0.f;
-                sm.h1[m][n] = (__bf16)silu_f(o.a1[t][i]);
+                dl1[t][i] = valid[i] ? dl : 0.f;
+                D1[t][i] = valid[i] ? de[i] * dl + zb1 : 0.f;
+                const float D2 = valid[i] ? de[i] * dl2[t][i] + zb2[t][i] : 0.f;
+                accb1[t] += D1[t][i];
+                accb2[t] += D2;
+                accw3[t] += valid[i] ? h2 * de[i] + s2[t][i] * t2[t][i] : 0.f;
+                __bf16 p[3];
+                split3(D2, p);
+                dp[0][i] = p[0]; dp[1][i] = p[1]; dp[2][i] = p[2];
+                split3(valid[i] ? dl2[t][i] : 0.f, p);
+                ep[0][i] = p[0]; ep[1][i] = p[1]; ep[2][i] = p[2];
+                hq[i] = (__bf16)silu_f(o.a1[t][i]);
+                tq[i] = (__bf16)ta1[t][i];
             }
-        }
-        if ((l & 15) == 0) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) sm.de[16 * w + 4 * (l >> 4) + i] = de[i];
+            for (int q = 0; q < 3; q++) {
+                put4(&sm.d[0][q][n][0], dp[q]);
+                put4(&sm.d[1][q][n][0], ep[q]);
+            }
+            put4(&sm.x[0][n][0], hq);
+            put4(&sm.x[1][n][0], tq);
         }
-        // loss sums: (e - u)^2 over the lane's rows (lanes l % 16 == 0 hold them), |R|^2 over rows l < 16
-        float lf = 0.f;
         if (l < 16 && r0 + l < wg1) {
             const float4 q = R[r0 + l];
-            lf = q.x * q.x + q.y * q.y + q.z * q.z;
-        }
-        le = (l & 15) == 0 ? le : 0.f;
-#pragma unroll
-        for (int m = 1; m < 64; m <<= 1) {
-            le += __shfl_xor(le, m, 64);
-            lf += __shfl_xor(lf, m, 64);
-        }
-        if (l == 0) {
-            sm.lsum[w][0] += le;
-            sm.lsum[w][1] += lf;
+            lf += q.x * q.x + q.y * q.y + q.z * q.z;
         }
         __syncthreads();
-        // weight gradients of this chunk
+        contract(acc2, std::integral_constant<int, 4>{});
+        __syncthreads();
+        // operands of dW1 = D1^T z + delta1^T u
 #pragma unroll
-        for (int j = 0; j < 3; j++) {
-            const int b = tid + 128 * j;
-            if (b < 256) {
-                const int o0 = 4 * (b >> 4), i0 = 4 * (b & 15);
-                for (int m = 0; m < kFmRows; m++) {
-                    const float4 dv = *reinterpret_cast<const float4*>(&sm.D2[m][o0]);
-                    const float4 ev = *reinterpret_cast<const float4*>(&sm.dl2[m][o0]);
-                    const float d4[4] = { dv.x, dv.y, dv.z, dv.w }, e4[4] = { ev.x, ev.y, ev.z, ev.w };
+        for (int t = 0; t < 4; t++) {
+            const int n = 16 * t + (l & 15);
+            __bf16 dp[3][4], ep[3][4];
 #pragma unroll
-                    for (int y = 0; y < 4; y++) {
-                        const float h = (float)sm.h1[m][i0 + y], ta = (float)sm.ta1[m][i0 + y];
+            for (int i = 0; i < 4; i++) {
+                __bf16 p[3];
+                split3(D1[t][i], p);
+                dp[0][i] = p[0]; dp[1][i] = p[1]; dp[2][i] = p[2];
+                split3(dl1[t][i], p);
+                ep[0][i] = p[0]; ep[1][i] = p[1]; ep[2][i] = p[2];
+            }
 #pragma unroll
-                        for (int x = 0; x < 4; x++) acc[j][x][y] += d4[x] * h + e4[x] * ta;
-                    }
-                }
-            } else {
-                const int bb = b - 256, o0 = 4 * (bb >> 3), k0 = 4 * (bb & 7);
-                for (int m = 0; m < kFmRows; m++) {
-                    const float4 dv = *reinterpret_cast<const float4*>(&sm.D1[m][o0]);
-                    const float4 ev = *reinterpret_cast<const float4*>(&sm.dl1[m][o0]);
-                    const float d4[4] = { dv.x, dv.y, dv.z, dv.w }, e4[4] = { ev.x, ev.y, ev.z, ev.w };
-#pragma unroll
-                    for (int y = 0; y < 4; y++) {
-                        const float zz = (float)sm.z[m][k0 + y], uv = (float)sm.uu[m][k0 + y];
-#pragma unroll
-                        for (int x = 0; x < 4; x++) acc[j][x][y] += d4[x] * zz + e4[x] * uv;
-                    }
-                }
+            for (int q = 0; q < 3; q++) {
+                put4(&sm.d[0][q][n][0], dp[q]);
+                put4(&sm.d[1][q][n][0], ep[q]);
             }
         }
-        if (tid < 64) {
-            for (int m = 0; m < kFmRows; m++) {
-                accb += sm.D1[m][tid];
-                accw3 += sm.q3[m][tid];
-            }
-        } else {
-            for (int m = 0; m < kFmRows; m++) accb += sm.D2[m][tid - 64];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            sm.x[0][8 * (l >> 4) + i][16 * w + (l & 15)] = za[i];
+            sm.x[1][8 * (l >> 4) + i][16 * w + (l & 15)] = ua[i];
         }
-        if (tid == 0)
-            for (int m = 0; m < kFmRows; m++) accb3 += sm.de[m];
+        __syncthreads();
+        contract(acc1, std::integral_constant<int, 2>{});
         __syncthreads();
     }
+    // column sums over the lanes that hold a unit's rows, then over the waves in order
+    auto rows_sum = [](float x) {
+        x += __shfl_xor(x, 16, 64);
+        return x + __shfl_xor(x, 32, 64);
+    };
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const float b1 = rows_sum(accb1[t]), b2 = rows_sum(accb2[t]), w3 = rows_sum(accw3[t]);
+        if (l < 16) {
+            sm.bsum[0][w][16 * t + l] = b1;
+            sm.bsum[1][w][16 * t + l] = b2;
+            sm.bsum[2][w][16 * t + l] = w3;
+        }
+    }
+    accb3 = rows_sum(accb3);                             // every lane of a row's 16 holds the row's values
+    le = rows_sum(le);
+#pragma unroll
+    for (int m = 1; m < 16; m <<= 1) lf += __shfl_xor(lf, m, 64);
+    if (l == 0) {
+        sm.ssum[0][w] = accb3;
+        sm.ssum[1][w] = le;
+        sm.ssum[2][w] = lf;
+    }
+    __syncthreads();
     float* out = partial + (size_t)blockIdx.x * (kSurrNTrain + 2);
 #pragma unroll
-    for (int j = 0; j < 3; j++) {
-        const int b = tid + 128 * j;
-        if (b < 256) {
-            const int o0 = 4 * (b >> 4), i0 = 4 * (b & 15);
+    for (int i = 0; i < 4; i++) {
+        const int unit = 16 * w + 4 * (l >> 4) + i;
 #pragma unroll
-            for (int x = 0; x < 4; x++)
+        for (int t = 0; t < 4; t++) out[kOffW2 + unit * kSurrHid + 16 * t + (l & 15)] = acc2[t][i];
 #pragma unroll
-                for (int y = 0; y < 4; y++) out[kOffW2 + (o0 + x) * kSurrHid + i0 + y] = acc[j][x][y];
-        } else {
-            const int bb = b - 256, o0 = 4 * (bb >> 3), k0 = 4 * (bb & 7);
-#pragma unroll
-            for (int x = 0; x < 4; x++)
-#pragma unroll
-                for (int y = 0; y < 4; y++) out[kOffW1 + (o0 + x) * kSurrFeat + k0 + y] = acc[j][x][y];
-        }
+        for (int t = 0; t < 2; t++) out[kOffW1 + unit * kSurrFeat + 16 * t + (l & 15)] = acc1[t][i];
     }
+    auto waves = [](const float (*q)[kSurrHid], int k) { return ((q[0][k] + q[1][k]) + q[2][k]) + q[3][k]; };
     if (tid < 64) {
-        out[kOffB1 + tid] = accb;
-        out[kOffW3 + tid] = accw3;
-    } else {
-        out[kOffB2 + tid - 64] = accb;
+        out[kOffB1 + tid] = waves(sm.bsum[0], tid);
+        out[kOffB2 + tid] = waves(sm.bsum[1], tid);
+        out[kOffW3 + tid] = waves(sm.bsum[2], tid);
     }
-    if (tid == 0) {
-        out[kOffB3] = accb3;
-        out[kSurrNTrain] = sm.lsum[0][0] + sm.lsum[1][0];
-        out[kSurrNTrain + 1] = sm.lsum[0][1] + sm.lsum[1][1];
-    }
+    if (tid < 3) out[tid == 0 ? kOffB3 : kSurrNTrain + tid - 1] = ((sm.ssum[tid][0] + sm.ssum[tid][1]) + sm.ssum[tid][2]) + sm.ssum[tid][3];
 }
 
 // ---- launch wrappers --------------------------------------------------------------------------------
-hipError_t launch_surr_pairs(const DevView& v, const SurrView& s, hipStream_t st)
+hipError_t launch_surr_pairs(const DevView& v, const SurrView& s, float* G, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_surr_pairs, dim3(v.Ctot), dim3(256), 0, st, v, s);
-    return hipGetLastError();
-}
-
-hipError_t launch_surr_desc(const DevView& v, const SurrView& s, float* G, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_surr_desc, dim3((v.Ntot + 7) / 8), dim3(256), 0, st, v, s, G);
+    hipLaunchKernelGGL(k_surr_pairs, dim3(v.Ctot), dim3(256), 0, st, v, s, G);
     return hipGetLastError();
 }
 
@@ -1049,7 +1132,7 @@ hipError_t launch_surr_train_step(const SurrView& s, const float* G, const float
     hipLaunchKernelGGL(k_surr_grad, dim3(nb), dim3(128), 0, st, s, G, u, row0, nrows, partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_surr_adam, dim3((kSurrNGrad + 255) / 256), dim3(256), 0, st, s, partial, nb, kSurrNGrad, lr,
+    hipLaunchKernelGGL(k_surr_adam, dim3((kSurrNGrad + 63) / 64), dim3(1024), 0, st, s, partial, nb, kSurrNGrad, lr,
                        0.9f, 0.999f, 1e-8f, step, loss_out);
     return hipGetLastError();
 }
@@ -1061,7 +1144,7 @@ hipError_t launch_surr_grad_only(const SurrView& s, const float* G, const float*
     hipLaunchKernelGGL(k_surr_grad, dim3(nb), dim3(128), 0, st, s, G, u, row0, nrows, partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_surr_sum, dim3((kSurrNGrad + 255) / 256), dim3(256), 0, st, partial, nb, kSurrNGrad, grad_out);
+    hipLaunchKernelGGL(k_surr_sum, dim3((kSurrNGrad + 63) / 64), dim3(1024), 0, st, partial, nb, kSurrNGrad, grad_out);
     return hipGetLastError();
 }
 
@@ -1083,15 +1166,15 @@ hipError_t launch_surr_fm(const DevView& v, const SurrView& s, const float* G, c
     hipLaunchKernelGGL(k_surr_fm_resid, dim3((nrows + 7) / 8), dim3(256), 0, st, v, s, g, R, u);
     hipLaunchKernelGGL(k_surr_fm_v, dim3((nrows + 7) / 8), dim3(256), 0, st, v, s, R,
                        (float)(2.0 * w_force / (3.0 * nrows)), vbuf);
-    hipLaunchKernelGGL(k_surr_grad_fm, dim3(nb), dim3(128), 0, st, s, G, u, vbuf, R, nrows, rows_per_wg,
+    hipLaunchKernelGGL(k_surr_grad_fm, dim3(nb), dim3(256), 0, st, s, G, u, vbuf, R, nrows, rows_per_wg,
                        (float)(2.0 / nrows), partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     constexpr int ng = kSurrNTrain + 2;
     if (grad_out)
-        hipLaunchKernelGGL(k_surr_sum, dim3((ng + 255) / 256), dim3(256), 0, st, partial, nb, ng, grad_out);
+        hipLaunchKernelGGL(k_surr_sum, dim3((ng + 63) / 64), dim3(1024), 0, st, partial, nb, ng, grad_out);
     else
-        hipLaunchKernelGGL(k_surr_adam, dim3((ng + 255) / 256), dim3(256), 0, st, s, partial, nb, ng, lr, 0.9f, 0.999f,
+        hipLaunchKernelGGL(k_surr_adam, dim3((ng + 63) / 64), dim3(1024), 0, st, s, partial, nb, ng, lr, 0.9f, 0.999f,
                            1e-8f, step, loss_out);
     return hipGetLastError();
 }

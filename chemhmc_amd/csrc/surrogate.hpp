@@ -26,9 +26,7 @@ struct SurrView {
     __bf16* w2tb;           // [64*64] bfloat16 copy of W2 transposed
     float *adam_m, *adam_v; // [kSurrNTrain]
     int* nb_n;              // [Ntot] pairs per atom (by sorted slot)
-    int* nb_j;              // [Ntot * kSurrMaxNb] sorted slot of the neighbour
-    float4* nb_d;           // (dx, dy, dz, r)
-    float2* nb_f;           // (fc, dfc/dr)
+    float4* nb_d;           // [Ntot * kSurrMaxNb] (dx, dy, dz, sorted slot of the neighbour as float bits)
     int* flag;              // bit 0: a list overflowed kSurrMaxNb; bit 1: a j-list overflowed the LDS stage
 };
 
@@ -100,8 +98,8 @@ __device__ __forceinline__ int stage_pairs(const ChainDev& C, const float4* __re
     return np;
 }
 
-hipError_t launch_surr_pairs(const DevView& v, const SurrView& s, hipStream_t st);
-hipError_t launch_surr_desc(const DevView& v, const SurrView& s, float* G, hipStream_t st);
+// pair list and descriptors G[slot][32]
+hipError_t launch_surr_pairs(const DevView& v, const SurrView& s, float* G, hipStream_t st);
 hipError_t launch_surr_mlp(const DevView& v, const SurrView& s, const float* G, float* g, float* e, hipStream_t st);
 hipError_t launch_surr_force(const DevView& v, const SurrView& s, const float* g, double kick_dt, bool store, hipStream_t st);
 hipError_t launch_surr_targets(const DevView& v, const SurrView& s, float* u, hipStream_t st);
