@@ -31,7 +31,7 @@ struct chmc_ctx {
     ChainDev* d_chains = nullptr;
     std::vector<void*> allocs;
     int bin_state = 2;           // 0: bins of the current positions, 1: counted (placement pending), 2: stale
-    bool have_bins = false;      // a placement exists that the local binning path can start from
+    bool have_bins = false;      // a placement of earlier positions of this configuration exists
     int force_kind = 0;          // 0 none, 1 fp32 stored, 2 fp64 stored
     int islots = 82;            // LJ sweep tiling: i-slots * 10 + waves per workgroup
     double pending_drift = 0.0;  // drift deferred into the next binning (integrator sequencing)
@@ -225,10 +225,8 @@ extern "C" int chmc_create(chmc_ctx** out, int nchains, const chmc_chain_desc* c
     if ((e = dalloc(c, &v.f32, 3 * (size_t)N)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.cell_of, N)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.slot, N)) != hipSuccess) return bail("hipMalloc", e);
-    if ((e = dalloc(c, &v.newcell, N)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.count, Cn)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.offs_buf, 2 * ((size_t)Cn + 1))) != hipSuccess) return bail("hipMalloc", e);
-    if ((e = dalloc(c, &v.bflag, 2)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.skey, N)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.satom, N)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.perm_buf, 2 * (size_t)N)) != hipSuccess) return bail("hipMalloc", e);
@@ -254,7 +252,6 @@ extern "C" int chmc_create(chmc_ctx** out, int nchains, const chmc_chain_desc* c
     if ((e = hipMemcpy(chunks, c->hchunks.data(), sizeof(Chunk) * c->nchunks, hipMemcpyHostToDevice)) != hipSuccess) return bail("hipMemcpy", e);
     // permute_vector = identity (parallel_binning_init, identical_particles_binning.cpp:37-44)
     if ((e = hipMemcpy(v.perm_buf, iota.data(), sizeof(int) * N, hipMemcpyHostToDevice)) != hipSuccess) return bail("hipMemcpy", e);
-    if ((e = hipMemset(v.bflag, 0, sizeof(int) * 2)) != hipSuccess) return bail("hipMemset", e);
     v.par = 0;
     if ((e = hipMemset(v.cell_of, 0, sizeof(int) * N)) != hipSuccess) return bail("hipMemset", e);
     if ((e = hipMemcpy(v.invperm, iota.data(), sizeof(int) * N, hipMemcpyHostToDevice)) != hipSuccess) return bail("hipMemcpy", e);
@@ -355,7 +352,7 @@ extern "C" int chmc_set_positions(chmc_ctx* c, int chain, const double* xyz)
     int rc = flush_drift(c);
     if (rc) return rc;
     c->bin_state = 2;
-    c->have_bins = false;     // arbitrary new positions: the next binning takes the general path
+    c->have_bins = false;
     c->force_kind = 0;
     return put_soa(c, c->v.x, chain, xyz);
 }
@@ -445,18 +442,19 @@ static int flush_drift(chmc_ctx* c)
 // kernel; a counted state only needs the placement
 static int ensure_bins(chmc_ctx* c)
 {
-    if (c->pending_drift != 0.0 || c->bin_state == 2) {
-        HIPCHK(c, launch_count(c->v, c->pending_drift, c->stream));
-        c->pending_drift = 0.0;
-        c->bin_state = 1;
-    }
-    if (c->bin_state == 1) {
+    const bool moved = c->pending_drift != 0.0 || c->bin_state == 2;
+    if (!moved && c->bin_state == 0) return CHMC_OK;
+    if (moved && bin_small(c->v)) {
+        HIPCHK(c, launch_bin_small(c->v, c->pending_drift, id_order(c), c->stream));
+    } else {
+        if (moved) HIPCHK(c, launch_count(c->v, c->pending_drift, c->stream));
         HIPCHK(c, launch_scan(c->v, c->stream));
-        HIPCHK(c, launch_place(c->v, c->have_bins && !id_order(c), id_order(c), c->stream));
-        c->v.par ^= 1;                 // the placement wrote the other perm/offs buffer
-        c->bin_state = 0;
-        c->have_bins = true;
+        HIPCHK(c, launch_place(c->v, id_order(c), c->stream));
     }
+    c->pending_drift = 0.0;
+    c->v.par ^= 1;                     // the placement wrote the other perm/offs buffer
+    c->bin_state = 0;
+    c->have_bins = true;
     return CHMC_OK;
 }
 
@@ -485,7 +483,8 @@ static int do_force_kick(chmc_ctx* c, double dt, bool storef, bool fuse_drift, d
 {
     int rc = ensure_bins(c);
     if (rc) return rc;
-    const bool fuse = fuse_drift && !fp64_md(c);
+    // small contexts drift and bin in one launch instead (a count fused here would leave two more)
+    const bool fuse = fuse_drift && !fp64_md(c) && !bin_small(c->v);
     const int mode = LJ_FORCE | LJ_KICK | (storef ? LJ_STOREF : 0) | (fuse ? LJ_DRIFT : 0);
     HIPCHK(c, launch_lj(c->v, mode, fp64_md(c), c->islots, dt, fuse ? drift_dt : 0.0, c->stream));
     c->force_kind = (storef && !fuse) ? (fp64_md(c) ? 2 : 1) : 0;
@@ -1320,8 +1319,9 @@ static int enqueue_trajectory(chmc_ctx* c, const chmc_hmc_params& hp, int steps,
         return CHMC_OK;
     }
     // heat bath + K_i + the count phase of the binning of the (accepted or restored) positions
-    HIPCHK(c, launch_heatbath(c->v, hp.seed, -1, true, false, c->stream));
-    c->bin_state = 1;
+    const bool count = !bin_small(c->v);
+    HIPCHK(c, launch_heatbath(c->v, hp.seed, -1, count, false, c->stream));
+    c->bin_state = count ? 1 : 2;
     // a zero-length binomial draw leaves x and p unchanged (the reference's size_t loop would not end, Q18)
     if (steps > 0 && (rc = integrate_seq(c, hp.scheme, hp.dt, steps, hp.lambda, false))) return rc;
     // V_f: after LEAP/OMF2/OMF4 the last binning is of the final positions; after a closing drift
@@ -2126,11 +2126,15 @@ static int time_force_is(chmc_ctx* c, int islots, int reps, double* ms_bin, doub
 {
     int rc = do_bin(c);
     if (rc) return rc;
-    const bool local = !id_order(c);
     auto rebin = [&]() -> hipError_t {
-        hipError_t e = launch_count(c->v, 0.0, c->stream);
-        if (e == hipSuccess) e = launch_scan(c->v, c->stream);
-        if (e == hipSuccess) e = launch_place(c->v, local, id_order(c), c->stream);
+        hipError_t e = hipSuccess;
+        if (bin_small(c->v)) {
+            e = launch_bin_small(c->v, 0.0, id_order(c), c->stream);
+        } else {
+            e = launch_count(c->v, 0.0, c->stream);
+            if (e == hipSuccess) e = launch_scan(c->v, c->stream);
+            if (e == hipSuccess) e = launch_place(c->v, id_order(c), c->stream);
+        }
         c->v.par ^= 1;
         return e;
     };

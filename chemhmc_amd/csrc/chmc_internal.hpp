@@ -6,14 +6,12 @@
 //   f64           : double SoA [3][Ntot]      (+grad U, FP64 path)
 //   atom_chain    : int [Ntot]
 //   cell_of, slot : int [Ntot]                (cell of each atom at the last binning, arrival slot)
-//   newcell       : int [Ntot]                (new cell id, indexed by the atom's previous sorted slot)
 //   count         : int [Ctot]                (zero between binnings; the scan clears it)
 //   offs_buf      : int [2][Ctot + 1]         (global exclusive scans of the counts: current / next)
 //   skey, satom   : int [Ntot]                (unsorted within-cell scatter, sort key and atom)
 //   perm_buf      : int [2][Ntot]             (sorted slot -> atom: current / next)
 //   invperm       : int [Ntot]                (atom -> current sorted slot)
 //   xs            : float4 [Ntot]             (sorted cell-relative FP32 coordinates, atom id in w)
-//   bflag         : int [2]                   (locality-violation flag, by target buffer)
 //   par (argument): which perm/offs buffer is current; the host flips it after every placement
 //   cell_chain    : int [Ctot]
 // Chains are contiguous in both the atom and the cell index spaces, so the global scan of the
@@ -138,7 +136,7 @@ struct DevView {
     const Chunk* chunks;
     double *x, *p, *x_saved, *f64;
     float* f32;
-    int *cell_of, *slot, *newcell, *count, *offs_buf, *skey, *satom, *perm_buf, *invperm, *bflag;
+    int *cell_of, *slot, *count, *offs_buf, *skey, *satom, *perm_buf, *invperm;
     int par;              // current binning buffer (0/1)
     float4* xs;
     double* red;          // [nchains][RED_NSLOT]
@@ -342,11 +340,14 @@ __device__ __forceinline__ int* offs_next(const DevView& v) { return v.offs_buf 
 __device__ __forceinline__ const int* perm_cur(const DevView& v) { return v.perm_buf + bin_parity(v) * v.Ntot; }
 __device__ __forceinline__ int* perm_next(const DevView& v) { return v.perm_buf + (bin_parity(v) ^ 1) * v.Ntot; }
 
-// binning: count (cell, slot, new cell at the previous slot) -> scan -> placement, either general
-// (scatter + rank by key) or local (collect from the previous neighbour cells)
+// binning: count (cell, arrival slot) -> scan -> placement (scatter + rank by key); contexts of at most
+// kBinSmall atoms and cells do it in one launch
 hipError_t launch_count(const DevView& v, double drift_dt, hipStream_t s);
 hipError_t launch_scan(const DevView& v, hipStream_t s);
-hipError_t launch_place(const DevView& v, bool local, bool atom_id_order, hipStream_t s);
+hipError_t launch_place(const DevView& v, bool atom_id_order, hipStream_t s);
+constexpr int kBinSmall = 4096;
+inline bool bin_small(const DevView& v) { return v.Ntot <= kBinSmall && v.Ctot <= kBinSmall; }
+hipError_t launch_bin_small(const DevView& v, double drift_dt, bool atom_id_order, hipStream_t s);
 
 // per-chain sums of the per-cell (V, W, pairs, K) and per-chunk (K) partials into red[]
 enum { SUM_CELLS = 1, SUM_CHUNKS_KI = 2, SUM_CHUNKS_K = 4, SUM_TILES = 8 };

@@ -257,7 +257,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_lj(DevView v, double kick_dt, d
                             v.x[d * N + atom] = xv;
                             x3[d] = xv;
                         }
-                        count_atom(v, C, atom, ibeg + i, c, x3);
+                        count_atom(v, C, atom, x3);
                     }
                 }
             }

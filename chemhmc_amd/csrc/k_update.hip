@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void k_heatbath(DevView v, uint64_t seed, long
         s += (px * px + py * py + pz * pz) / (2 * C.mass);
         if (count) {
             const double x3[3] = { v.x[a], v.x[N + a], v.x[2 * N + a] };
-            count_atom(v, C, a, v.invperm[a], v.cell_of[a], x3);
+            count_atom(v, C, a, x3);
         }
     }
     const double t = block_sum_256(s);
