@@ -232,6 +232,7 @@ extern "C" int chmc_create(chmc_ctx** out, int nchains, const chmc_chain_desc* c
     if ((e = dalloc(c, &v.perm_buf, 2 * (size_t)N)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.invperm, N)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.xs, N)) != hipSuccess) return bail("hipMalloc", e);
+    if ((e = dalloc(c, &v.xs64, 3 * (size_t)N)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.red, (size_t)nchains * RED_NSLOT)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.chunk_part, (size_t)c->nchunks)) != hipSuccess) return bail("hipMalloc", e);
     if ((e = dalloc(c, &v.cell_part, 4 * (size_t)Cn)) != hipSuccess) return bail("hipMalloc", e);
@@ -501,7 +502,7 @@ static int do_energy(chmc_ctx* c, bool rebin, bool sums = true)
     if (rc) return rc;
     rc = rebin ? do_bin(c) : ensure_bins(c);
     if (rc) return rc;
-    HIPCHK(c, launch_lj(c->v, LJ_ENERGY, true, c->islots, 0.0, 0.0, c->stream));
+    HIPCHK(c, launch_energy(c->v, false, c->stream));
     if (sums) HIPCHK(c, launch_reduce(c->v, SUM_CELLS, c->stream));
     return CHMC_OK;
 }
@@ -583,7 +584,7 @@ extern "C" int chmc_evaluate_potential(chmc_ctx* c, double* V)
         rc = ensure_bins(c);
         if (rc) return rc;
     }
-    HIPCHK(c, launch_lj(c->v, LJ_ENERGY, true, c->islots, 0.0, 0.0, c->stream));
+    HIPCHK(c, launch_energy(c->v, c->bin_state != 0, c->stream));
     HIPCHK(c, launch_reduce(c->v, SUM_CELLS, c->stream));
     return read_red(c, RED_V, V);
 }

@@ -12,6 +12,7 @@
 //   perm_buf      : int [2][Ntot]             (sorted slot -> atom: current / next)
 //   invperm       : int [Ntot]                (atom -> current sorted slot)
 //   xs            : float4 [Ntot]             (sorted cell-relative FP32 coordinates, atom id in w)
+//   xs64          : double SoA [3][Ntot]      (sorted FP64 positions)
 //   par (argument): which perm/offs buffer is current; the host flips it after every placement
 //   cell_chain    : int [Ctot]
 // Chains are contiguous in both the atom and the cell index spaces, so the global scan of the
@@ -139,6 +140,7 @@ struct DevView {
     int *cell_of, *slot, *count, *offs_buf, *skey, *satom, *perm_buf, *invperm;
     int par;              // current binning buffer (0/1)
     float4* xs;
+    double* xs64;
     double* red;          // [nchains][RED_NSLOT]
     double* chunk_part;   // [nchunks]: per-chunk kinetic energy
     double* cell_part;    // [Ctot * 4]: energy, virial, interacting pairs, kinetic energy
@@ -356,6 +358,8 @@ hipError_t launch_drift(const DevView& v, double dt, hipStream_t s);
 hipError_t launch_kick(const DevView& v, double dt, bool fp64, hipStream_t s);
 // tiling: i-slots per wave (4, 8, 16) x waves per workgroup (1, 2, 4), encoded islots * 10 + waves
 hipError_t launch_lj(const DevView& v, int mode, bool fp64, int tiling, double kick_dt, double drift_dt, hipStream_t s);
+// FP64 energy, virial, interacting pairs and kinetic energy per cell; stale: positions moved since the binning
+hipError_t launch_energy(const DevView& v, bool stale, hipStream_t s);
 hipError_t launch_kinetic(const DevView& v, hipStream_t s);
 // slots: write the momenta in the current list buffer's slot order (pl) instead of atom order (p)
 hipError_t launch_heatbath(const DevView& v, uint64_t seed, long long traj_or_neg, bool count, bool slots, hipStream_t s);

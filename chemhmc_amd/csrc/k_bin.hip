@@ -12,7 +12,8 @@
 //                      its id for in-cell order by atom id)
 //   k_cell_rank      : 16 lanes per cell rank the cell's entries by key -> the stable order
 //   k_bin_small      : all of it in one workgroup's LDS for small contexts
-// The placement writes the next perm/offs buffers, invperm and the FP32 cell-relative coordinates; the
+// The placement writes the next perm/offs buffers, invperm and the sorted coordinates (FP64, and FP32 relative
+// to the cell); the
 // host then flips the parity argument that selects the current buffers.
 #include "chmc_internal.hpp"
 #include "bin_device.hpp"
@@ -90,6 +91,8 @@ __device__ __forceinline__ void place_atom(const DevView& v, int* perm_n, int po
 {
     perm_n[pos] = atom;
     v.invperm[atom] = pos;
+#pragma unroll
+    for (int d = 0; d < 3; d++) v.xs64[(size_t)d * v.Ntot + pos] = x3[d];
     v.xs[pos] = make_float4((float)(x3[0] - o[0]), (float)(x3[1] - o[1]), (float)(x3[2] - o[2]), __int_as_float(atom));
 }
 

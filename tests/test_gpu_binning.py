@@ -70,3 +70,52 @@ def test_cell_md_sequence(chmc, N):
                     e.update_momenta(0.002 if k == 2 else 0.004)
             out.append((e.positions(), e.momenta()))
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+# FP64 sweep: both workgroup shapes (fewer than 512 cells, and more), cells denser than one LDS pass (768
+# neighbour entries), atoms with more than 64 neighbours within rc, one- and two-cell boxes, an empty cell
+@pytest.mark.parametrize("N,L", [(1, 6.0), (60, 2.6), (700, 5.1), (2500, 8.0), (6000, 20.0), (9000, 21.0), (400, (30.0, 6.0, 5.2)),
+                                 (3000, 9.5)])
+def test_fp64_sweep_sizes(chmc, orc, N, L):
+    box = np.broadcast_to(np.asarray(L, float), (3,)).copy()
+    rng = np.random.default_rng(N)
+    s = int(np.ceil(N ** (1 / 3) - 1e-9))
+    k = np.arange(N)
+    x = ((np.stack((k % s, (k // s) % s, k // (s * s)), -1) + 0.5) / s + rng.uniform(-0.2, 0.2, (N, 3)) / s) * box
+    x -= box * np.floor(x / box)
+    sig = 0.8 * float(np.min(box / s))
+    with chmc.Engine(chmc.Chain(N=N, L=tuple(box), cutoff=RC, sigma=sig, beta=0.8)) as e:
+        e.set_positions(x)
+        e.compute_force(fp64=True)
+        f, fo = e.force(), orc.force_binning(x, box, RC, sigma=sig)
+        # a few roundings per term of up to several hundred terms, against the largest force
+        assert np.max(np.abs(f - fo)) <= 1e-12 * max(np.max(np.abs(fo)), 1e-300)
+        V, W = e.compute_potential()[0], e.virial()[0]
+        Vo, Wo = orc.potential_binning(x, box, RC, sigma=sig), orc.virial_binning(x, box, RC, sigma=sig)
+        assert abs(V - Vo) <= 1e-12 * abs(Vo) and abs(W - Wo) <= 1e-12 * abs(Wo)
+        nc, ni = e.pair_counts()
+        assert (nc, ni) == orc.pair_counts(x, box, RC)
+        # the kick of an FP64 force evaluation
+        p = rng.normal(size=(N, 3))
+        e.set_momenta(p)
+        e.kick(0.01)
+        assert np.allclose(e.momenta(), p - 0.01 * 0.8 * f, rtol=0, atol=1e-13 * max(1.0, np.max(np.abs(f))))
+
+
+# evaluate_potential takes the bins as they are: positions that moved (also across the box) keep their old
+# cells, and the pairs are those of the old stencil at the current positions
+@pytest.mark.parametrize("N,step", [(2000, 0.05), (2000, 3.0), (20000, 0.3)])
+def test_evaluate_potential_with_old_bins(chmc, orc, N, step):
+    L = (N / 0.7) ** (1 / 3)
+    with chmc.Engine(chmc.Chain(N=N, L=L, cutoff=RC)) as e:
+        e.init_lattice(5, 0.1)
+        e.bin()
+        perm, cnt, off = e.bins()
+        e.set_momenta(np.random.default_rng(N).normal(size=(N, 3)))
+        e.update_positions(step)
+        x = e.positions()
+        V = e.evaluate_potential()[0]
+        Vo = orc.potential_binning(x, [L] * 3, RC, bins=(perm, cnt, off))
+        assert abs(V - Vo) <= 1e-11 * abs(Vo)
+        Vn = orc.potential_binning(x, [L] * 3, RC)
+        assert abs(e.compute_potential()[0] - Vn) <= 1e-11 * abs(Vn)
