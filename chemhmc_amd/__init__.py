@@ -274,7 +274,7 @@ class Engine:
         self._ck(lib().chmc_set_positions(self._h, chain, _c(x)), "set_positions")
 
     def positions(self, chain=0):
-        out = np.zeros((self.chains[chain].N, 3))
+        out = np.empty((self.chains[chain].N, 3))         # filled by the call
         self._ck(lib().chmc_get_positions(self._h, chain, out), "get_positions")
         return out
 
@@ -282,7 +282,7 @@ class Engine:
         self._ck(lib().chmc_set_momenta(self._h, chain, _c(p)), "set_momenta")
 
     def momenta(self, chain=0):
-        out = np.zeros((self.chains[chain].N, 3))
+        out = np.empty((self.chains[chain].N, 3))         # filled by the call
         self._ck(lib().chmc_get_momenta(self._h, chain, out), "get_momenta")
         return out
 
@@ -305,7 +305,7 @@ class Engine:
         self._ck(lib().chmc_compute_force(self._h, int(bool(fp64))), "compute_force")
 
     def force(self, chain=0):
-        out = np.zeros((self.chains[chain].N, 3))
+        out = np.empty((self.chains[chain].N, 3))         # filled by the call
         self._ck(lib().chmc_get_force(self._h, chain, out), "get_force")
         return out
 
@@ -407,8 +407,8 @@ class Engine:
 
     def surrogate_features(self, chain=0):
         n = self.chains[chain].N
-        G = np.zeros((n, SURR_NFEAT), np.float32)
-        g = np.zeros((n, SURR_NFEAT), np.float32)
+        G = np.empty((n, SURR_NFEAT), np.float32)         # filled by the call
+        g = np.empty((n, SURR_NFEAT), np.float32)
         self._ck(lib().chmc_surrogate_features(self._h, int(chain), G.ctypes.data, g.ctypes.data), "surrogate_features")
         return G, g
 

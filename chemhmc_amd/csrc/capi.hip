@@ -51,6 +51,11 @@ struct chmc_ctx {
     uint4* d_rdfu = nullptr;     // fixed-point coordinates of the RDF's chain
     int rdfu_cap = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;
+    // pinned host memory of the context (made on first use): two transfer buffers of stage_cap bytes, and the
+    // words kernels leave for the host (per-chain sums, list flags)
+    char* stage[2] = { nullptr, nullptr };
+    size_t stage_cap = 0;
+    hipEvent_t stage_ev[2] = { nullptr, nullptr };
     // learned surrogate (allocated on first use)
     bool surr_alloc = false, surr_params = false;
     SurrView sv{};
@@ -142,6 +147,10 @@ static void destroy_ctx(chmc_ctx* c)
     if (c->utrain) hipFree(c->utrain);
     if (c->spartial) hipFree(c->spartial);
     if (c->xtrain) hipFree(c->xtrain);
+    if (c->stage[0]) hipHostFree(c->stage[0]);
+    if (c->v.host_red) hipHostFree(c->v.host_red);
+    for (hipEvent_t e : c->stage_ev)
+        if (e) hipEventDestroy(e);
     if (c->ev0) hipEventDestroy(c->ev0);
     if (c->ev1) hipEventDestroy(c->ev1);
     if (c->ev2) hipEventDestroy(c->ev2);
@@ -307,33 +316,106 @@ extern "C" int chmc_num_atoms(const chmc_ctx* c, int* total, int* nchains)
 }
 
 // ---- state transfer ------------------------------------------------------------------------------
+// Arrays cross between the caller's memory and the device through the context's pinned buffers: a kernel
+// writes or reads the caller's layout (AoS, atom order) straight in pinned memory, so the host only copies.
+// Pageable copies of three SoA arrays with host transposes took most of a call: set_positions +
+// compute_force + get_force at N = 32768 216 us of which kernels are 45, now 167; the surrogate features there
+// (8 MB, permuted on the host) 0.8 ms of the evaluation 1.4.  Larger arrays alternate between the two buffers,
+// the copy of one overlapping the kernel of the other.
+constexpr size_t kStageMax = (size_t)4 << 20;
+
+static int stage_ensure(chmc_ctx* c)
+{
+    if (c->stage_cap) return CHMC_OK;
+    int nmax = 1;
+    for (const ChainDev& cd : c->hchains) nmax = std::max(nmax, cd.natoms);
+    const size_t cap = std::min(kStageMax, std::max<size_t>((24 * (size_t)nmax + 4095) / 4096 * 4096, 16384));
+    for (hipEvent_t& e : c->stage_ev)
+        if (!e) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    void* p = nullptr;
+    HIPCHK(c, hipHostMalloc(&p, 2 * cap, hipHostMallocDefault));
+    c->stage[0] = static_cast<char*>(p);
+    c->stage[1] = c->stage[0] + cap;
+    c->stage_cap = cap;
+    return CHMC_OK;
+}
+
+// rows of row_bytes from the device: launch(first row, rows, buffer) writes a part, use(buffer, first row,
+// rows) takes it.  Returns with every part taken (and the stream drained up to the last kernel).
+template <typename Launch, typename Use>
+static int staged_get(chmc_ctx* c, size_t rows, size_t row_bytes, Launch launch, Use use)
+{
+    int rc = stage_ensure(c);
+    if (rc) return rc;
+    const size_t per = c->stage_cap / row_bytes, parts = (rows + per - 1) / per;
+    for (size_t k = 0; k <= parts; k++) {
+        if (k < parts) {
+            HIPCHK(c, launch(k * per, std::min(per, rows - k * per), c->stage[k & 1]));
+            if (parts > 1) HIPCHK(c, hipEventRecord(c->stage_ev[k & 1], c->stream));
+        }
+        if (k == 0) continue;
+        if (parts > 1) HIPCHK(c, hipEventSynchronize(c->stage_ev[(k - 1) & 1]));
+        else HIPCHK(c, hipStreamSynchronize(c->stream));
+        use(c->stage[(k - 1) & 1], (k - 1) * per, std::min(per, rows - (k - 1) * per));
+    }
+    return CHMC_OK;
+}
+
+// rows to the device: fill(buffer, first row, rows) on the host, then launch(first row, rows, buffer)
+template <typename Fill, typename Launch>
+static int staged_put(chmc_ctx* c, size_t rows, size_t row_bytes, Fill fill, Launch launch)
+{
+    int rc = stage_ensure(c);
+    if (rc) return rc;
+    const size_t per = c->stage_cap / row_bytes, parts = (rows + per - 1) / per;
+    for (size_t k = 0; k < parts; k++) {
+        if (k >= 2) HIPCHK(c, hipEventSynchronize(c->stage_ev[k & 1]));
+        fill(c->stage[k & 1], k * per, std::min(per, rows - k * per));
+        HIPCHK(c, launch(k * per, std::min(per, rows - k * per), c->stage[k & 1]));
+        if (parts > 1) HIPCHK(c, hipEventRecord(c->stage_ev[k & 1], c->stream));
+    }
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return CHMC_OK;
+}
+
 static int put_soa(chmc_ctx* c, double* dbase, int chain, const double* aos)
 {
     const ChainDev& cd = c->hchains[chain];
-    const int n = cd.natoms;
-    std::vector<double> h(3 * (size_t)n);
-    for (int i = 0; i < n; i++)
-        for (int d = 0; d < 3; d++) h[(size_t)d * n + i] = aos[3 * i + d];
-    for (int d = 0; d < 3; d++)
-        HIPCHK(c, hipMemcpyAsync(dbase + (size_t)d * c->Ntot + cd.atom_off, h.data() + (size_t)d * n,
-                                 sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return CHMC_OK;
+    return staged_put(c, (size_t)cd.natoms, 24,
+                      [&](char* buf, size_t r0, size_t n) { std::memcpy(buf, aos + 3 * r0, 24 * n); },
+                      [&](size_t r0, size_t n, const char* buf) {
+                          return launch_put_aos(dbase + cd.atom_off + r0, (size_t)c->Ntot, (int)n,
+                                                reinterpret_cast<const double*>(buf), c->stream);
+                      });
 }
 
 template <typename T>
 static int get_soa(chmc_ctx* c, const T* dbase, int chain, double* aos)
 {
     const ChainDev& cd = c->hchains[chain];
-    const int n = cd.natoms;
-    std::vector<T> h(3 * (size_t)n);
-    for (int d = 0; d < 3; d++)
-        HIPCHK(c, hipMemcpyAsync(h.data() + (size_t)d * n, dbase + (size_t)d * c->Ntot + cd.atom_off,
-                                 sizeof(T) * n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int i = 0; i < n; i++)
-        for (int d = 0; d < 3; d++) aos[3 * i + d] = (double)h[(size_t)d * n + i];
-    return CHMC_OK;
+    return staged_get(c, (size_t)cd.natoms, 24,
+                      [&](size_t r0, size_t n, char* buf) {
+                          return launch_get_aos(dbase + cd.atom_off + r0, (size_t)c->Ntot, (int)n,
+                                                reinterpret_cast<double*>(buf), c->stream);
+                      },
+                      [&](const char* buf, size_t r0, size_t n) { std::memcpy(aos + 3 * r0, buf, 24 * n); });
+}
+
+// every coordinate in [0, L): the first one outside, or -1
+static long long first_outside(const double* xyz, int n, const double L[3])
+{
+    double lim[12];
+    for (int k = 0; k < 12; k++) lim[k] = L[k % 3];
+    long long i = 0;
+    const long long n3 = 3 * (long long)n;
+    for (; i + 12 <= n3; i += 12) {                  // four particles at a time, without branches
+        int bad = 0;
+        for (int k = 0; k < 12; k++) bad |= !(xyz[i + k] >= 0.0) | !(xyz[i + k] < lim[k]);
+        if (bad) break;
+    }
+    for (; i < n3; i++)
+        if (!(xyz[i] >= 0.0 && xyz[i] < L[i % 3])) return i;
+    return -1;
 }
 
 static int flush_drift(chmc_ctx* c);
@@ -344,12 +426,9 @@ extern "C" int chmc_set_positions(chmc_ctx* c, int chain, const double* xyz)
     c->list_valid = false;             // positions change outside the lists
     const ChainDev& cd = c->hchains[chain];
     // check_in_volume (identical_particles.cpp:228-236): every coordinate in [0, L)
-    for (int i = 0; i < cd.natoms; i++)
-        for (int d = 0; d < 3; d++) {
-            const double q = xyz[3 * i + d];
-            if (!(q >= 0.0 && q < cd.L[d]))
-                return fail(c, CHMC_E_ARG, "particle " + std::to_string(i) + " outside the box in dimension " + std::to_string(d));
-        }
+    const long long out = first_outside(xyz, cd.natoms, cd.L);
+    if (out >= 0)
+        return fail(c, CHMC_E_ARG, "particle " + std::to_string(out / 3) + " outside the box in dimension " + std::to_string(out % 3));
     int rc = flush_drift(c);
     if (rc) return rc;
     c->bin_state = 2;
@@ -507,12 +586,26 @@ static int do_energy(chmc_ctx* c, bool rebin, bool sums = true)
     return CHMC_OK;
 }
 
-static int read_red(chmc_ctx* c, int slot, double* out)
+// the words that kernels leave in pinned memory for the host
+static int host_words(chmc_ctx* c)
 {
-    std::vector<double> h((size_t)c->nchains * RED_NSLOT);
-    HIPCHK(c, hipMemcpyAsync(h.data(), c->v.red, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream));
+    if (c->v.host_red) return CHMC_OK;
+    void* p = nullptr;
+    HIPCHK(c, hipHostMalloc(&p, sizeof(double) * ((size_t)c->nchains * RED_NSLOT + 2), hipHostMallocDefault));
+    c->v.host_red = static_cast<double*>(p);
+    c->v.host_flag = reinterpret_cast<int*>(c->v.host_red + (size_t)c->nchains * RED_NSLOT);
+    return CHMC_OK;
+}
+
+// per-chain sums of the partials (launch_reduce), one slot of them read back: the sums go to pinned memory
+// too, so that the host waits for the kernel and no copy follows it
+static int reduce_read(chmc_ctx* c, int what, int slot, double* out)
+{
+    int rc = host_words(c);
+    if (rc) return rc;
+    HIPCHK(c, launch_reduce(c->v, what | SUM_HOST, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int k = 0; k < c->nchains; k++) out[k] = h[(size_t)k * RED_NSLOT + slot];
+    for (int k = 0; k < c->nchains; k++) out[k] = c->v.host_red[(size_t)k * RED_NSLOT + slot];
     return CHMC_OK;
 }
 
@@ -568,9 +661,9 @@ extern "C" int chmc_get_force(chmc_ctx* c, int chain, double* grad)
 extern "C" int chmc_compute_potential(chmc_ctx* c, double* V)
 {
     if (!c || !V) return CHMC_E_ARG;
-    int rc = do_energy(c, true);
+    int rc = do_energy(c, true, false);
     if (rc) return rc;
-    return read_red(c, RED_V, V);
+    return reduce_read(c, SUM_CELLS, RED_V, V);
 }
 
 extern "C" int chmc_evaluate_potential(chmc_ctx* c, double* V)
@@ -585,25 +678,24 @@ extern "C" int chmc_evaluate_potential(chmc_ctx* c, double* V)
         if (rc) return rc;
     }
     HIPCHK(c, launch_energy(c->v, c->bin_state != 0, c->stream));
-    HIPCHK(c, launch_reduce(c->v, SUM_CELLS, c->stream));
-    return read_red(c, RED_V, V);
+    return reduce_read(c, SUM_CELLS, RED_V, V);
 }
 
 extern "C" int chmc_virial(chmc_ctx* c, double* W)
 {
     if (!c || !W) return CHMC_E_ARG;
-    int rc = do_energy(c, false);
+    int rc = do_energy(c, false, false);
     if (rc) return rc;
-    return read_red(c, RED_W, W);
+    return reduce_read(c, SUM_CELLS, RED_W, W);
 }
 
 extern "C" int chmc_pair_counts(chmc_ctx* c, int chain, long long* ncand, long long* nint)
 {
     if (!c || chain < 0 || chain >= c->nchains) return CHMC_E_ARG;
-    int rc = do_energy(c, false);
+    int rc = do_energy(c, false, false);
     if (rc) return rc;
     std::vector<double> ni(c->nchains);
-    rc = read_red(c, RED_NINT, ni.data());
+    rc = reduce_read(c, SUM_CELLS, RED_NINT, ni.data());
     if (rc) return rc;
     // candidates of the 27-cell stencil: sum over cells of count(c) * sum_{27 neighbours} count(n), minus self
     const ChainDev& cd = c->hchains[chain];
@@ -636,8 +728,7 @@ extern "C" int chmc_kinetic(chmc_ctx* c, double* K)
 {
     if (!c || !K) return CHMC_E_ARG;
     HIPCHK(c, launch_kinetic(c->v, c->stream));
-    HIPCHK(c, launch_reduce(c->v, SUM_CHUNKS_K, c->stream));
-    return read_red(c, RED_K, K);
+    return reduce_read(c, SUM_CHUNKS_K, RED_K, K);
 }
 
 extern "C" int chmc_update_momenta(chmc_ctx* c, double dt)
@@ -901,6 +992,8 @@ static int list_import(chmc_ctx* c)
 static int list_export(chmc_ctx* c, bool saved)
 {
     if (!c->lstate) return CHMC_OK;
+    const int rc = host_words(c);
+    if (rc) return rc;
     HIPCHK(c, launch_list_export(c->v, saved, c->stream));
     c->lstate = false;
     return CHMC_OK;
@@ -992,11 +1085,11 @@ static int list_energy(chmc_ctx* c, bool sums)
     return CHMC_OK;
 }
 
+// the list flags, which the export of the slot-ordered state (every MD call ends with one) left in pinned memory
 static int list_check_overflow(chmc_ctx* c)
 {
-    int f[4] = { 0, 0, 0, 0 };
-    HIPCHK(c, hipMemcpyAsync(f, c->v.lflag, sizeof(f), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    const int* f = c->v.host_flag;
     if (f[2] & 3) return fail(c, CHMC_E_STATE, "neighbour list capacity exceeded (cell members or list entries); results invalid");
     if (f[2] & 4)
         return fail(c, CHMC_E_STATE, "an atom's momentum exceeded 10 sqrt(m / beta), the bound of the list check interval: "
@@ -1849,12 +1942,19 @@ extern "C" int chmc_surrogate_eval(chmc_ctx* c, double* energy, int store_force)
     }
     if (store_force) c->force_kind = 1;
     if (energy) {
-        std::vector<float> e(c->Ntot);
-        HIPCHK(c, hipMemcpy(e.data(), c->se, sizeof(float) * c->Ntot, hipMemcpyDeviceToHost));
         for (int k = 0; k < c->nchains; k++) {
             const ChainDev& cd = c->hchains[k];
-            double sum = 0.0;
-            for (int i = 0; i < cd.natoms; i++) sum += e[cd.atom_off + i];     // sorted slots of chain k
+            double sum = 0.0;                                   // in the order of the chain's sorted slots
+            const int rc2 = staged_get(c, (size_t)cd.natoms, sizeof(float),
+                                       [&](size_t r0, size_t n, char* buf) {
+                                           return launch_copy_words(c->se + cd.atom_off + r0, (int)n,
+                                                                    reinterpret_cast<float*>(buf), c->stream);
+                                       },
+                                       [&](const char* buf, size_t, size_t n) {
+                                           const float* e = reinterpret_cast<const float*>(buf);
+                                           for (size_t i = 0; i < n; i++) sum += e[i];
+                                       });
+            if (rc2) return rc2;
             energy[k] = sum;
         }
     }
@@ -1890,25 +1990,17 @@ extern "C" int chmc_surrogate_features(chmc_ctx* c, int chain, float* G, float* 
     if (!c || chain < 0 || chain >= c->nchains) return CHMC_E_ARG;
     if (!c->surr_alloc) return fail(c, CHMC_E_STATE, "surrogate not evaluated");
     const ChainDev& cd = c->hchains[chain];
-    std::vector<int> perm(cd.natoms);
-    if (c->surr_lists_eval) {       // slot order of the chain's current list buffer
-        int cur = 0;
-        HIPCHK(c, hipMemcpy(&cur, c->v.lbuf + chain, sizeof(int), hipMemcpyDeviceToHost));
-        HIPCHK(c, hipMemcpy(perm.data(), c->v.lperm + (size_t)cur * c->Ntot + cd.atom_off, sizeof(int) * cd.natoms,
-                            hipMemcpyDeviceToHost));
-    } else {                        // order of the current binning
-        HIPCHK(c, hipMemcpy(perm.data(), c->v.perm_buf + (size_t)c->v.par * c->Ntot + cd.atom_off, sizeof(int) * cd.natoms,
-                            hipMemcpyDeviceToHost));
-    }
-    std::vector<float> hG((size_t)cd.natoms * kSurrFeat), hg((size_t)cd.natoms * kSurrFeat);
-    HIPCHK(c, hipMemcpy(hG.data(), c->sG + (size_t)cd.atom_off * kSurrFeat, sizeof(float) * hG.size(), hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(hg.data(), c->sg + (size_t)cd.atom_off * kSurrFeat, sizeof(float) * hg.size(), hipMemcpyDeviceToHost));
-    for (int k = 0; k < cd.natoms; k++) {
-        const int a = perm[k] - cd.atom_off;
-        for (int f = 0; f < kSurrFeat; f++) {
-            if (G) G[(size_t)a * kSurrFeat + f] = hG[(size_t)k * kSurrFeat + f];
-            if (g) g[(size_t)a * kSurrFeat + f] = hg[(size_t)k * kSurrFeat + f];
-        }
+    const size_t row = sizeof(float) * kSurrFeat;
+    for (int which = 0; which < 2; which++) {
+        float* out = which == 0 ? G : g;
+        if (!out) continue;
+        int rc = staged_get(c, (size_t)cd.natoms, row,
+                            [&](size_t r0, size_t n, char* buf) {
+                                return launch_get_features(c->v, which == 0 ? c->sG : c->sg, chain, c->surr_lists_eval, (int)r0,
+                                                           (int)n, reinterpret_cast<float*>(buf), c->stream);
+                            },
+                            [&](const char* buf, size_t r0, size_t n) { std::memcpy(out + r0 * kSurrFeat, buf, n * row); });
+        if (rc) return rc;
     }
     return CHMC_OK;
 }
@@ -2243,9 +2335,9 @@ extern "C" int chmc_list_stats(chmc_ctx* c, int chain, long long* entries, long 
     if (!c || chain < 0 || chain >= c->nchains) return CHMC_E_ARG;
     int rc = flush_drift(c);
     if (rc) return rc;
-    if ((rc = list_import(c)) || (rc = list_invalidate(c)) || (rc = list_energy(c, true)) || (rc = list_export(c, false))) return rc;
+    if ((rc = list_import(c)) || (rc = list_invalidate(c)) || (rc = list_energy(c, false)) || (rc = list_export(c, false))) return rc;
     std::vector<double> nintv(c->nchains);
-    if ((rc = read_red(c, RED_NINT, nintv.data()))) return rc;
+    if ((rc = reduce_read(c, SUM_TILES, RED_NINT, nintv.data()))) return rc;
     const ChainDev& cd = c->hchains[chain];
     std::vector<int> n(cd.natoms);
     int cur = 0;

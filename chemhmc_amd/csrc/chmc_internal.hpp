@@ -142,6 +142,8 @@ struct DevView {
     float4* xs;
     double* xs64;
     double* red;          // [nchains][RED_NSLOT]
+    double* host_red;     // the same in pinned host memory (SUM_HOST)
+    int* host_flag;       // [4] the list flags in pinned host memory, written by the export
     double* chunk_part;   // [nchunks]: per-chunk kinetic energy
     double* cell_part;    // [Ctot * 4]: energy, virial, interacting pairs, kinetic energy
     ChainState* state;    // [nchains]
@@ -352,7 +354,7 @@ inline bool bin_small(const DevView& v) { return v.Ntot <= kBinSmall && v.Ctot <
 hipError_t launch_bin_small(const DevView& v, double drift_dt, bool atom_id_order, hipStream_t s);
 
 // per-chain sums of the per-cell (V, W, pairs, K) and per-chunk (K) partials into red[]
-enum { SUM_CELLS = 1, SUM_CHUNKS_KI = 2, SUM_CHUNKS_K = 4, SUM_TILES = 8 };
+enum { SUM_CELLS = 1, SUM_CHUNKS_KI = 2, SUM_CHUNKS_K = 4, SUM_TILES = 8, SUM_HOST = 16 };
 hipError_t launch_reduce(const DevView& v, int what, hipStream_t s);
 hipError_t launch_drift(const DevView& v, double dt, hipStream_t s);
 hipError_t launch_kick(const DevView& v, double dt, bool fp64, hipStream_t s);
@@ -409,5 +411,14 @@ int open_potential_tiles(int n);
 hipError_t launch_open_potential(const double* xyz, int n, int nexp, double a, double b, double* partials, double* result,
                                  hipStream_t s);
 hipError_t launch_fill_int(int* p, int value, int n, hipStream_t s);
+// transfers: n atoms of an SoA array (component stride apart) to or from AoS rows in pinned host memory, n
+// floats, and atoms [a0, a0 + n) of a chain's per-slot features src[slot][32] (lists: slots of the chain's current
+// list buffer, else of the current binning) in atom order
+hipError_t launch_put_aos(double* soa, size_t stride, int n, const double* aos, hipStream_t s);
+hipError_t launch_get_aos(const double* soa, size_t stride, int n, double* aos, hipStream_t s);
+hipError_t launch_get_aos(const float* soa, size_t stride, int n, double* aos, hipStream_t s);
+hipError_t launch_copy_words(const float* src, int n, float* out, hipStream_t s);
+hipError_t launch_get_features(const DevView& v, const float* src, int chain, bool lists, int a0, int n, float* out,
+                               hipStream_t s);
 
 }  // namespace chmc

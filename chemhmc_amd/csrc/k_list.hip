@@ -1172,9 +1172,11 @@ __global__ __launch_bounds__(256) void k_limport(DevView v)
 }
 
 // saved: also h_x (xl_saved, in the start buffer's slot order) into x_saved
+// the list flags go to pinned host memory, where the host reads them once the call's work is done
 __global__ __launch_bounds__(256) void k_lexport(DevView v, int saved)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < 4) v.host_flag[s] = v.lflag[s];
     if (s >= v.Ntot) return;
     const int ch = v.atom_chain[s];
     const int cur = *list_cur(v, ch), pord = *list_pord(v, ch);

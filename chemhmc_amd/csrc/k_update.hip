@@ -138,6 +138,9 @@ __device__ void chain_sums(const DevView& v, int ch, int what)
 __global__ __launch_bounds__(256) void k_reduce(DevView v, int what)
 {
     chain_sums(v, blockIdx.x, what);
+    // thread 0 wrote the sums: for the host too
+    if ((what & SUM_HOST) && threadIdx.x == 0)
+        for (int k = 0; k < RED_NSLOT; k++) v.host_red[blockIdx.x * RED_NSLOT + k] = v.red[blockIdx.x * RED_NSLOT + k];
 }
 
 // One workgroup per chain: V_f, W_f, K_f from the energy sweep's partials, K_i from the heat bath's,
@@ -439,6 +442,67 @@ __global__ __launch_bounds__(256) void k_spec_broadcast(DevView v, int src, int 
             dst[w] = e;
         }
     }
+}
+
+// ---- transfers to and from pinned host memory (one element a thread, coalesced on the host's side) ----
+__global__ __launch_bounds__(256) void k_put_aos(double* __restrict__ soa, size_t stride, int n, const double* __restrict__ aos)
+{
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k < 3 * n) soa[(size_t)(k % 3) * stride + k / 3] = aos[k];
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_get_aos(const T* __restrict__ soa, size_t stride, int n, double* __restrict__ aos)
+{
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k < 3 * n) aos[k] = (double)soa[(size_t)(k % 3) * stride + k / 3];
+}
+
+__global__ __launch_bounds__(256) void k_copy_words(const float* __restrict__ src, int n, float* __restrict__ out)
+{
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k < n) out[k] = src[k];
+}
+
+__global__ __launch_bounds__(256) void k_get_features(DevView v, const float* __restrict__ src, int chain, int lists, int a0,
+                                                      int n, float* __restrict__ out)
+{
+    const int k = blockIdx.x * 256 + threadIdx.x;             // 32 threads an atom
+    if (k >> 5 >= n) return;
+    const int atom = v.chains[chain].atom_off + a0 + (k >> 5);
+    const int slot = (lists ? list_buf(v, *list_cur(v, chain)).linv : v.invperm)[atom];
+    out[k] = src[(size_t)slot * 32 + (k & 31)];
+}
+
+hipError_t launch_put_aos(double* soa, size_t stride, int n, const double* aos, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_put_aos, dim3((3 * n + 255) / 256), dim3(256), 0, s, soa, stride, n, aos);
+    return hipGetLastError();
+}
+
+hipError_t launch_get_aos(const double* soa, size_t stride, int n, double* aos, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_get_aos<double>, dim3((3 * n + 255) / 256), dim3(256), 0, s, soa, stride, n, aos);
+    return hipGetLastError();
+}
+
+hipError_t launch_get_aos(const float* soa, size_t stride, int n, double* aos, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_get_aos<float>, dim3((3 * n + 255) / 256), dim3(256), 0, s, soa, stride, n, aos);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_words(const float* src, int n, float* out, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_copy_words, dim3((n + 255) / 256), dim3(256), 0, s, src, n, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_get_features(const DevView& v, const float* src, int chain, bool lists, int a0, int n, float* out,
+                               hipStream_t s)
+{
+    hipLaunchKernelGGL(k_get_features, dim3((32 * n + 255) / 256), dim3(256), 0, s, v, src, chain, lists ? 1 : 0, a0, n, out);
+    return hipGetLastError();
 }
 
 // Standalone kick with the stored force: p -= (dt*beta) f  (identical_particles.cpp:686-688)
