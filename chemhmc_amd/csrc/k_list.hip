@@ -699,6 +699,27 @@ __device__ __forceinline__ void list_drift_slot(const DevView& v, const ListBuf&
     if (v.lcheck_dt != 0.0 && pn[0] * pn[0] + pn[1] * pn[1] + pn[2] * pn[2] > C.p2max) atomicOr(&v.lflag[2], 4);
 }
 
+// What the tail of a list sweep needs of its chain, read before the sweep's first store: read where it is
+// used, every one of these was a vector load of its own behind the stores (the compiler cannot know that they
+// leave the chain alone), a chain of seven load latencies at the end of each wave (N = 4001: sweep FILL_TC).
+struct TailConst {
+    double kdt, coeff_x, trig2, p2max;     // uniform
+    double L, lsize;                       // of the lane's dimension
+    int atom_off;
+};
+__device__ __forceinline__ TailConst tail_const(const DevView& v, const ChainDev& C, double kick_dt, int d)
+{
+    TailConst t;
+    t.kdt = kick_dt * C.beta;              // dt * coeff_p, coeff_p = beta (identical_particles.cpp:642-644)
+    t.coeff_x = C.coeff_x;                 // compute_coeff_position, :646-648
+    t.trig2 = trigger2(v, C);
+    t.p2max = C.p2max;
+    t.L = C.L[d];
+    t.lsize = C.lsize[d];
+    t.atom_off = C.atom_off;
+    return t;
+}
+
 // The per-atom tail of a list sweep, on lanes sub = 0, 1, 2 of the slot (one dimension each; fd is the
 // force component of the lane's dimension): store the force in atom order, kick p in FP64, optionally
 // drift x in FP64 (identical_particles.cpp:651-673), then lane 0 writes the FP32 coordinates of the other
@@ -706,33 +727,40 @@ __device__ __forceinline__ void list_drift_slot(const DevView& v, const ListBuf&
 // rebuild position.  Thread 0 clears the requests of this evaluation's parity when its rebuild check ran
 // (checked), and otherwise carries a pending one over to the next parity.
 template <int MODE, int LP>
-__device__ __forceinline__ void list_tail(const DevView& v, const ListBuf& L, const ChainDev& C, const Chunk& tl, int s,
+__device__ __forceinline__ void list_tail(const DevView& v, const ListBuf& L, const TailConst& C, const Chunk& tl, int s,
                                           bool val, int sub, int d, int atom, float fd, double p_d, double x_d,
-                                          float4 ref, double kick_dt, double drift_dt, int q, int checked)
+                                          float4 ref, double drift_dt, int q, int checked)
 {
     const int N = v.Ntot;
     double e = 0.0, pn = 0.0;
     float rel = 0.f;
+    // FP64 position relative to the rebuild cell origin (list_rel of the lane's dimension)
+    auto list_rel_d = [&](double x) {
+        const double o = (double)((__float_as_int(ref.w) >> (10 * d)) & 1023) * C.lsize;
+        double r = x - o;
+        const double diff = r - (double)ref_coord(ref, d);
+        if (diff > 0.5 * C.L) r -= C.L;
+        else if (diff < -0.5 * C.L) r += C.L;
+        return r;
+    };
     if (val && sub < 3) {
         if constexpr ((MODE & LJ_STOREF) != 0) v.f32[d * N + atom] = fd;
         pn = p_d;
         if constexpr ((MODE & LJ_KICK) != 0) {
-            const double kdt = kick_dt * C.beta;       // dt * coeff_p, coeff_p = beta (:642-644)
-            pn = lp_round(pn - kdt * (double)fd, v.lp_scale);
+            pn = lp_round(pn - C.kdt * (double)fd, v.lp_scale);
             v.pl[d * N + s] = pn;
         }
         if constexpr ((MODE & LJ_DRIFT) != 0) {
-            const double coeff_x = C.coeff_x;          // compute_coeff_position, identical_particles.cpp:646-648
             double xv = x_d;
-            xv += drift_dt * coeff_x * pn;
+            xv += drift_dt * C.coeff_x * pn;
             xv = lp_round(xv, v.lp_scale);
-            xv = wrap_box(xv, C.L[d]);
+            xv = wrap_box(xv, C.L);
             v.xl[d * N + s] = xv;
-            const double r = list_rel(C, ref, d, xv);
+            const double r = list_rel_d(xv);
             e = r - (double)ref_coord(ref, d);
             rel = (float)r;
         }
-        if constexpr ((MODE & LJ_REL64) != 0) v.rel64[4 * (size_t)s + d] = list_rel(C, ref, d, x_d);
+        if constexpr ((MODE & LJ_REL64) != 0) v.rel64[4 * (size_t)s + d] = list_rel_d(x_d);
     }
     if constexpr ((MODE & LJ_DRIFT) != 0) {
         // lane 0 of the slot gathers the y, z coordinates and the squared displacement and momentum over
@@ -741,7 +769,7 @@ __device__ __forceinline__ void list_tail(const DevView& v, const ListBuf& L, co
         const double e2 = group_sum<4>(e * e), p2 = group_sum<4>(pn * pn);
         if (val && sub == 0) {
             L.xsl[(size_t)(q ^ 1) * N + s] = make_float4(rel, ry, rz, 0.f);
-            if (e2 > trigger2(v, C)) request(v, q ^ 1, tl.chain);
+            if (e2 > C.trig2) request(v, q ^ 1, tl.chain);
             if (v.lcheck_dt != 0.0 && p2 > C.p2max) atomicOr(&v.lflag[2], 4);
         }
     }
@@ -787,6 +815,7 @@ __global__ __launch_bounds__(kTile * LP) void k_lsweep(DevView v, double kick_dt
     const bool val = s < tl.end;
     const int d = sub < 3 ? sub : 0;                      // the per-dimension tail runs on lanes 0, 1, 2
     const float4* __restrict__ xq = L.xsl + (size_t)q * N;
+    const float eps48 = C.eps48_f;
     const int* segs = reinterpret_cast<const int*>(seg_tab[W16 ? t : 0]);
     float ax = 0.f, ay = 0.f, az = 0.f;
     float4 xi = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -880,6 +909,7 @@ __global__ __launch_bounds__(kTile * LP) void k_lsweep(DevView v, double kick_dt
         }
     }
     // the tail's operands, fetched after the pairs (fewer registers live through the pair loop)
+    const TailConst tc = tail_const(v, C, kick_dt, d);
     if (val && sub < 3) {
         p_d = v.pl[d * N + s];
         if constexpr ((MODE & (LJ_DRIFT | LJ_REL64)) != 0) {
@@ -890,8 +920,8 @@ __global__ __launch_bounds__(kTile * LP) void k_lsweep(DevView v, double kick_dt
     ax = group_sum<LP>(ax);
     ay = group_sum<LP>(ay);
     az = group_sum<LP>(az);
-    list_tail<MODE, LP>(v, L, C, tl, s, val, sub, d, atom, C.eps48_f * (d == 0 ? ax : (d == 1 ? ay : az)), p_d, x_d, ref,
-                        kick_dt, drift_dt, q, checked);
+    list_tail<MODE, LP>(v, L, tc, tl, s, val, sub, d, atom, eps48 * (d == 0 ? ax : (d == 1 ? ay : az)), p_d, x_d, ref,
+                        drift_dt, q, checked);
 }
 
 // Surrogate forces on the lists (same tiles, lanes, entries and tail as k_lsweep): for every listed pair
@@ -1008,11 +1038,12 @@ __global__ __launch_bounds__(kTile * LP) void k_lsurr_sweep(DevView v, const flo
             if (two) pair_force(pd1, g1);
         }
     }
+    const TailConst tc = tail_const(v, C, kick_dt, d);
     ax = group_sum<LP>(ax);
     ay = group_sum<LP>(ay);
     az = group_sum<LP>(az);
-    list_tail<MODE, LP>(v, L, C, tl, s, val, sub, d, atom, d == 0 ? ax : (d == 1 ? ay : az), p_d, x_d, ref, kick_dt,
-                        drift_dt, q, checked);
+    list_tail<MODE, LP>(v, L, tc, tl, s, val, sub, d, atom, d == 0 ? ax : (d == 1 ? ay : az), p_d, x_d, ref, drift_dt, q,
+                        checked);
 }
 
 __global__ __launch_bounds__(256) void k_ldrift(DevView v, double dt, int q)
