@@ -701,7 +701,8 @@ __device__ __forceinline__ void list_drift_slot(const DevView& v, const ListBuf&
 
 // What the tail of a list sweep needs of its chain, read before the sweep's first store: read where it is
 // used, every one of these was a vector load of its own behind the stores (the compiler cannot know that they
-// leave the chain alone), a chain of seven load latencies at the end of each wave (N = 4001: sweep FILL_TC).
+// leave the chain alone), a chain of seven load latencies at the end of each wave (sweep at N = 4001: 4.84 us,
+// now 4.36; at N = 1,048,576: 172 us, now 153).
 struct TailConst {
     double kdt, coeff_x, trig2, p2max;     // uniform
     double L, lsize;                       // of the lane's dimension
