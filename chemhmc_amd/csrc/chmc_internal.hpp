@@ -324,16 +324,19 @@ __device__ __forceinline__ int entry_slot(const int* segs, unsigned e) { return 
 // FP64 position of coordinate x (dimension d) relative to the rebuild cell origin of reference ref,
 // taken through the periodic image nearest the rebuild position r0 (an atom moves far less than L / 2
 // between rebuilds, so the image is the one of the same box or of a neighbour box)
-__device__ __forceinline__ double list_rel(const ChainDev& C, const float4 ref, int d, double x)
+__device__ __forceinline__ double list_rel(const float4 ref, int d, double x, double L, double lsize)
 {
     const int cell = __float_as_int(ref.w);
-    const double o = (double)((cell >> (10 * d)) & 1023) * C.lsize[d];
     const float r0 = d == 0 ? ref.x : (d == 1 ? ref.y : ref.z);
-    double r = x - o;
+    double r = __builtin_fma(-(double)((cell >> (10 * d)) & 1023), lsize, x);     // one rounding, whoever calls
     const double diff = r - (double)r0;
-    if (diff > 0.5 * C.L[d]) r -= C.L[d];
-    else if (diff < -0.5 * C.L[d]) r += C.L[d];
+    if (diff > 0.5 * L) r -= L;
+    else if (diff < -0.5 * L) r += L;
     return r;
+}
+__device__ __forceinline__ double list_rel(const ChainDev& C, const float4 ref, int d, double x)
+{
+    return list_rel(ref, d, x, C.L[d], C.lsize[d]);
 }
 __device__ __forceinline__ float ref_coord(const float4 ref, int d) { return d == 0 ? ref.x : (d == 1 ? ref.y : ref.z); }
 

@@ -735,15 +735,6 @@ __device__ __forceinline__ void list_tail(const DevView& v, const ListBuf& L, co
     const int N = v.Ntot;
     double e = 0.0, pn = 0.0;
     float rel = 0.f;
-    // FP64 position relative to the rebuild cell origin (list_rel of the lane's dimension)
-    auto list_rel_d = [&](double x) {
-        const double o = (double)((__float_as_int(ref.w) >> (10 * d)) & 1023) * C.lsize;
-        double r = x - o;
-        const double diff = r - (double)ref_coord(ref, d);
-        if (diff > 0.5 * C.L) r -= C.L;
-        else if (diff < -0.5 * C.L) r += C.L;
-        return r;
-    };
     if (val && sub < 3) {
         if constexpr ((MODE & LJ_STOREF) != 0) v.f32[d * N + atom] = fd;
         pn = p_d;
@@ -757,11 +748,11 @@ __device__ __forceinline__ void list_tail(const DevView& v, const ListBuf& L, co
             xv = lp_round(xv, v.lp_scale);
             xv = wrap_box(xv, C.L);
             v.xl[d * N + s] = xv;
-            const double r = list_rel_d(xv);
+            const double r = list_rel(ref, d, xv, C.L, C.lsize);
             e = r - (double)ref_coord(ref, d);
             rel = (float)r;
         }
-        if constexpr ((MODE & LJ_REL64) != 0) v.rel64[4 * (size_t)s + d] = list_rel_d(x_d);
+        if constexpr ((MODE & LJ_REL64) != 0) v.rel64[4 * (size_t)s + d] = list_rel(ref, d, x_d, C.L, C.lsize);
     }
     if constexpr ((MODE & LJ_DRIFT) != 0) {
         // lane 0 of the slot gathers the y, z coordinates and the squared displacement and momentum over
