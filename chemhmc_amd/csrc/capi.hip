@@ -899,7 +899,6 @@ static int list_setup(chmc_ctx* c, double skin, const std::vector<double>& skins
     HIPCHK(c, lalloc(c, &v.tcur, (size_t)v.ntiles));
     HIPCHK(c, lalloc(c, &v.lflag, 4));
     HIPCHK(c, lalloc(c, &v.lreq, 2 * ((size_t)c->nchains + 1)));
-    HIPCHK(c, lalloc(c, &v.lscan_tmp, (size_t)lcells));
     HIPCHK(c, lalloc(c, &v.lref, 2 * N));
     HIPCHK(c, lalloc(c, &v.rel64, 4 * N));
     HIPCHK(c, lalloc(c, &v.xsl, 2 * 2 * N));

@@ -61,7 +61,6 @@
 //   one), which the export follows.  lbuf[k] / lbuf[nchains + k]
 //   are chain k's current and start buffers; tcur[t] repeats the current buffer of tile t's chain, so
 //   that a sweep workgroup finds its buffer with one load that depends on nothing but its index.
-//   lscan_tmp     : int [Cl]                  (global exclusive scan of the counts, rebuild scratch)
 //   tiles         : 32-slot ranges that never straddle chains (sweep / energy workgroups)
 #pragma once
 #include <hip/hip_runtime.h>
@@ -153,7 +152,7 @@ struct DevView {
                                     // with first batches of 10 ... 16 entries)
     const int* lcell_chain;
     const Chunk* tiles;
-    int *lcount, *loffs, *lperm, *linv, *nbn, *lflag, *lreq, *lscan_tmp, *lcs, *ctab;
+    int *lcount, *loffs, *lperm, *linv, *nbn, *lflag, *lreq, *lcs, *ctab;
     int* lrank;           // [dense] rank of each counted member in its list cell (k_lscan_chains)
     char* nb;             // list rows (entry bytes: 2 with entry16, else 4)
     size_t nb_stride;     // bytes of one buffer's rows: Ntot * nbcap * entry bytes

@@ -147,94 +147,76 @@ __device__ __forceinline__ void rank_cell_members(const DevView& v, int q, int c
 
 constexpr int kRankWaves = 16;     // cells ranked per 1024-thread workgroup of k_lscan and k_lscan_chains
 
-// chains with more list cells than kScanCells: workgroup 0 scans all counts (zero in chains that did
-// not count) and each rebuilding chain's cells get atom_off + the scan relative to the chain's first
-// cell, in the list offsets of the buffer being rebuilt.  It runs on one CU, so every global access is
-// coalesced: rounds of 8192 counts go through LDS, each thread scans 8 contiguous ones, a block scan
-// over the threads and a running carry join the rounds.  The workgroups after it rank the members of
-// every list cell of a rebuilding chain for the build.
-__global__ __launch_bounds__(1024) void k_lscan(DevView v, int q, int cb)
+// Chains with more list cells than kScanCells: the first workgroups scan kScanPart cells each into the list
+// offsets of the buffers being rebuilt (a chain's offsets start at its atom_off).  Each adds up by itself the
+// counts that its first chain has before its part, so no workgroup waits for another (one workgroup scanning
+// everything in rounds took 62 us over the 42,875 cells of N = 1,048,576, most of it one CU's loads; in a run
+// that rebuilds at every tenth check the launch took 8.7 us on average and now takes 6.6).  The workgroups
+// after them rank the members of every list cell of a rebuilding chain for the build, in turn: few enough that
+// an idle launch stays small.
+constexpr int kScanPart = 8192;
+constexpr int kRankGroups = 512;
+
+__global__ __launch_bounds__(1024) void k_lscan(DevView v, int q, int cb, int parts)
 {
     if (*req_any(v, q) == 0) return;
-    if (blockIdx.x > 0) {                  // workgroups after the first rank the members of kRankWaves cells
-        __shared__ int rank_ids[kRankWaves][256];
-        const int wid = threadIdx.x >> 6;
-        const int cell = ((int)blockIdx.x - 1) * kRankWaves + wid;
-        if (cell < v.Cl) rank_cell_members(v, q, cb, cell, threadIdx.x & 63, rank_ids[wid]);
+    constexpr int T = 1024, PT = kScanPart / T;
+    __shared__ int buf[kScanPart];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    if ((int)blockIdx.x >= parts) {
+        int* ids = buf + wid * 256;
+        for (int cell = ((int)blockIdx.x - parts) * kRankWaves + wid; cell < v.Cl; cell += ((int)gridDim.x - parts) * kRankWaves)
+            rank_cell_members(v, q, cb, cell, lane, ids);
         return;
     }
-    constexpr int T = 1024, PT = 8;
-    __shared__ int buf[T * PT];
-    __shared__ int wsum[16];
-    __shared__ int carry;
+    __shared__ int wsum[16], psum[16];
     const int* __restrict__ cnt = v.lcount + (size_t)cb * v.Cl;
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int n = v.Cl;
-    if (tid == 0) carry = 0;
-    for (int r0 = 0; r0 < n; r0 += T * PT) {
+    const int r0 = blockIdx.x * kScanPart, n = min(v.Cl - r0, kScanPart);
+    int before = 0;                                        // the first chain's members before this part
+    for (int c = v.chains[v.lcell_chain[r0]].lcell_off + tid; c < r0; c += T) before += cnt[c];
 #pragma unroll
-        for (int k = 0; k < PT; k++) {
-            const int c = r0 + k * T + tid;
-            buf[k * T + tid] = c < n ? cnt[c] : 0;
-        }
-        __syncthreads();
-        int vals[PT];
-        int s = 0;
+    for (int m = 1; m < 64; m <<= 1) before += __shfl_xor(before, m, 64);
+    if (lane == 0) psum[wid] = before;
 #pragma unroll
-        for (int k = 0; k < PT; k++) {
-            vals[k] = buf[tid * PT + k];
-            s += vals[k];
-        }
-        int incl = s;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += t;
-        }
-        if (lane == 63) wsum[wid] = incl;
-        __syncthreads();
-        if (wid == 0) {
-            int w = lane < 16 ? wsum[lane] : 0;
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) {
-                const int t = __shfl_up(w, o, 64);
-                if (lane >= o) w += t;
-            }
-            if (lane < 16) wsum[lane] = w;
-        }
-        __syncthreads();
-        int run = carry + incl - s + (wid > 0 ? wsum[wid - 1] : 0);
-#pragma unroll
-        for (int k = 0; k < PT; k++) {
-            buf[tid * PT + k] = run;
-            run += vals[k];
-        }
-        __syncthreads();                      // every thread has read carry; buf holds the round's scan
-        if (tid == T - 1) carry = run;
-#pragma unroll
-        for (int k = 0; k < PT; k++) {
-            const int c = r0 + k * T + tid;
-            if (c < n) v.lscan_tmp[c] = buf[k * T + tid];
-        }
-        __syncthreads();                      // buf free, carry final
+    for (int k = 0; k < PT; k++) {
+        const int c = k * T + tid;
+        buf[c] = c < n ? cnt[r0 + c] : 0;
     }
-    // list offsets of the rebuilding chains (chains are contiguous in cell space: a thread's cells change
-    // chain rarely, so the chain's flag, buffer and base are looked up once per change)
-    int kprev = -1, base = 0;
-    bool rq = false;
-    int* loffs = nullptr;
-#pragma unroll 4
-    for (int c = tid; c < n; c += T) {
-        const int k = v.lcell_chain[c];
-        const int sc = v.lscan_tmp[c];
-        if (k != kprev) {
-            kprev = k;
-            rq = *req(v, q, k) != 0;
-            const ChainDev& C = v.chains[k];
-            base = C.atom_off - v.lscan_tmp[C.lcell_off];
-            loffs = list_buf(v, *list_start(v, k) ^ 1).loffs;
-        }
-        if (rq) loffs[c] = base + sc;
+    __syncthreads();
+    before = 0;
+    for (int w = 0; w < 16; w++) before += psum[w];
+    int vals[PT];
+    int s = 0;
+#pragma unroll
+    for (int k = 0; k < PT; k++) {
+        vals[k] = buf[tid * PT + k];
+        s += vals[k];
+    }
+    int incl = s;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += t;
+    }
+    if (lane == 63) wsum[wid] = incl;
+    __syncthreads();
+    int run = incl - s;
+    for (int w = 0; w < wid; w++) run += wsum[w];
+#pragma unroll
+    for (int k = 0; k < PT; k++) {
+        buf[tid * PT + k] = run;
+        run += vals[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PT; k++) {
+        const int c = k * T + tid;
+        if (c >= n) continue;
+        const int ch = v.lcell_chain[r0 + c];
+        if (*req(v, q, ch) == 0) continue;
+        const ChainDev& C = v.chains[ch];
+        const int in_part = C.lcell_off >= r0 ? buf[c] - buf[C.lcell_off - r0] : before + buf[c];
+        list_buf(v, *list_start(v, ch) ^ 1).loffs[r0 + c] = C.atom_off + in_part;
     }
 }
 
@@ -284,13 +266,16 @@ __global__ __launch_bounds__(1024) void k_lscan_chains(DevView v, int q, int cb)
 
 constexpr int kLMaxJ = 1024;      // staged neighbour members per pass (a cell never spans two passes)
 constexpr int kJPad = 64;         // far entries past a pass's members: one iteration of the pair test
-constexpr int kBuildWaves = 4;    // waves of a build workgroup
+// Waves of a build workgroup: 4, or 16 where the cells are so few (kSmallBuild: two workgroups a CU) that a
+// rebuild is one workgroup's latency (N = 4001, 125 cells: rebuild 33.9 us with 4 waves, 20.8 with 16)
+constexpr int kBuildWaves = 4, kBuildWavesSmall = 16, kSmallBuild = 512;
 
-// exclusive scan of n <= kScanCells values in LDS by one 256-thread workgroup
-__device__ __forceinline__ void block_scan_256(int* a, int n, int* wsum)
+// exclusive scan of n <= kScanCells values in LDS by one workgroup of NT threads
+template <int NT>
+__device__ __forceinline__ void block_scan(int* a, int n, int* wsum)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int per = (n + 255) / 256;
+    const int per = (n + NT - 1) / NT;
     const int beg = min(tid * per, n), end = min(beg + per, n);
     int s = 0;
     for (int i = beg; i < end; i++) s += a[i];
@@ -346,13 +331,13 @@ __device__ __forceinline__ void build_step(const float4* sj, int j0, int lane, c
 // group of 64 tested pairs; two own atoms x 32 members took ~18 and 6-9 % more build time).  The loop
 // reads two groups of 64 while the second starts inside the members, then at most one more, so no read
 // passes jn + 63 and the padding stays one group.
-template <bool W16>
+template <int W, bool W16>
 __device__ __forceinline__ void build_pass(const float4* sj, const float4* si, int* icount, int ni, int jn,
                                            float rl2, int nbcap, char* __restrict__ nbb)
 {
     static_assert(kJPad >= 64, "every step reads fewer than 64 entries past the members");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int i = wave; i < ni; i += kBuildWaves) {
+    for (int i = wave; i < ni; i += W) {
         const float4 xi = si[i];
         int count = icount[i];
         const int rowoff = __float_as_int(xi.w) * nbcap;
@@ -377,13 +362,13 @@ __device__ __forceinline__ void build_pass(const float4* sj, const float4* si, i
 //            is fixed by the slot order and not by the arrival order of the count.
 // A neighbourhood of more than kLMaxJ members is staged in passes of whole cells; the own cell is
 // loaded with the first pass.
-template <bool SCAN, bool W16, bool RANKED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_lbuild(DevView v, int q, int cb)
+template <int W, bool SCAN, bool W16, bool RANKED>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == kBuildWaves ? 6 : 4))) void k_lbuild(DevView v, int q, int cb)
 {
     const int c = xcd_block(blockIdx.x, v.Cl);
     const int ch = v.lcell_chain[c];
     if (*req_any(v, q) == 0 || *req(v, q, ch) == 0) return;
-    constexpr int NT = 256, W = kBuildWaves, PT = (kLMaxJ + NT - 1) / NT;
+    constexpr int NT = 64 * W, PT = (kLMaxJ + NT - 1) / NT;
     // staged j in slot order: coordinates relative to the i-cell origin, list entry in w; padded past the
     // pass's members to a whole iteration of the test loop with far-away entries
     __shared__ float4 sj[kLMaxJ + kJPad];
@@ -394,35 +379,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
     float4* si = dyn_lds;
     int* icount = reinterpret_cast<int*>(dyn_lds + v.lcap_max);
     int* sido = icount + v.lcap_max;
-    __shared__ int seg_cell[27], seg_beg[27], seg_cnt[27], seg_pref[28], seg_code[27], wsum[4];
+    __shared__ int seg_cell[27], seg_beg[27], seg_cnt[27], seg_pref[28], seg_code[27], wsum[W];
     __shared__ float seg_sh[27][3];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     constexpr bool e16 = W16;              // 16-bit segment-relative entries
+    // the chain's constants, read before the first store: behind one, each of these would be a vector load of
+    // its own where it is used
     const ChainDev& C = v.chains[ch];
+    const int lcap = C.lcap, lcell_off = C.lcell_off, lncells = C.lncells, atom_off = C.atom_off, tile_first = C.tile_first;
+    const size_t ldense_off = (size_t)C.ldense_off;
+    const float rl2 = C.rl2_f;
     const int tb = *list_start(v, ch) ^ 1;
     const ListBuf L = list_buf(v, tb);
     const int nx = C.lnbin[0], ny = C.lnbin[1], nz = C.lnbin[2];
-    const int lc = c - C.lcell_off;
+    const int lc = c - lcell_off;
     const int bz = lc / (nx * ny), by = (lc - bz * nx * ny) / nx, bx = lc - nx * (by + bz * ny);
-    const int* __restrict__ cnt = v.lcount + (size_t)cb * v.Cl + C.lcell_off;
-    const float4* __restrict__ mem = v.lmem + C.ldense_off;
-    const double* __restrict__ memx = v.lmemx + C.ldense_off;
-    const double* __restrict__ memp = v.lmemp + C.ldense_off;
+    const int* __restrict__ cnt = v.lcount + (size_t)cb * v.Cl + lcell_off;
+    const float4* __restrict__ mem = v.lmem + ldense_off;
+    const double* __restrict__ memx = v.lmemx + ldense_off;
+    const double* __restrict__ memp = v.lmemp + ldense_off;
     const size_t xstride = (size_t)v.ldense;
     const int N = v.Ntot;
-    if (tid == 0) {
-        *list_cur(v, ch) = tb;
-        if (lc == 0) atomicAdd(&v.lflag[3], 1);        // chain rebuilds run (statistics)
-    }
     // the own cell's members and their FP64 positions (one per thread, in bounds for every thread
     // below lcap): issued first, their latency overlaps the offsets
     float4 meo = make_float4(0.f, 0.f, 0.f, 0.f);
     double xo[3] = { 0.0, 0.0, 0.0 }, po[3] = { 0.0, 0.0, 0.0 };
     int orank = 0;                                   // RANKED: the member's rank by atom id (k_lscan_chains)
-    if (tid < C.lcap) {
-        const size_t mi = (size_t)lc * C.lcap + tid;
+    if (tid < lcap) {
+        const size_t mi = (size_t)lc * lcap + tid;
         meo = mem[mi];
-        if constexpr (RANKED) orank = v.lrank[C.ldense_off + mi];
+        if constexpr (RANKED) orank = v.lrank[ldense_off + mi];
 #pragma unroll
         for (int d = 0; d < 3; d++) {
             xo[d] = memx[d * xstride + mi];
@@ -445,10 +431,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
             seg_cell[lane] = jl;
             seg_code[lane] = image_code(dd[0], dd[1], dd[2]);
             if constexpr (!SCAN) {
-                seg_beg[lane] = L.loffs[C.lcell_off + jl];
-                nk = min(L.loffs[C.lcell_off + jl + 1] - L.loffs[C.lcell_off + jl], C.lcap);
+                seg_beg[lane] = L.loffs[lcell_off + jl];
+                nk = min(L.loffs[lcell_off + jl + 1] - L.loffs[lcell_off + jl], lcap);
             } else {
-                nk = min(cnt[jl], C.lcap);
+                nk = min(cnt[jl], lcap);
             }
             seg_cnt[lane] = nk;
         }
@@ -464,13 +450,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
     }
     int* scan = reinterpret_cast<int*>(sj);          // SCAN: sj is free until the first pass is staged
     if constexpr (SCAN) {
-        for (int i = tid; i < C.lncells; i += NT) scan[i] = cnt[i];
+        for (int i = tid; i < lncells; i += NT) scan[i] = cnt[i];
     }
     __syncthreads();
+    if (tid == 0) {
+        *list_cur(v, ch) = tb;
+        if (lc == 0) atomicAdd(&v.lflag[3], 1);        // chain rebuilds run (statistics)
+    }
     const int ni = seg_cnt[13];                      // segment 13: the cell itself (ni <= lcap <= 256)
     if (ni == 0) return;
 
-    const float rl2 = C.rl2_f;
     const int nbcap = v.nbcap;
     int ibeg = 0;
     for (int k0 = 0; k0 < 27;) {
@@ -495,15 +484,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
                 for (int step = 16; step > 0; step >>= 1)
                     if (k + step < k1 && seg_pref[k + step] <= jlo + t) k += step;
                 kk[u] = k;
-                const size_t mi = (size_t)seg_cell[k] * C.lcap + (jlo + t - seg_pref[k]);
+                const size_t mi = (size_t)seg_cell[k] * lcap + (jlo + t - seg_pref[k]);
                 me[u] = mem[mi];
-                if constexpr (RANKED) rk[u] = v.lrank[C.ldense_off + mi];
+                if constexpr (RANKED) rk[u] = v.lrank[ldense_off + mi];
             }
         }
         if constexpr (SCAN) {
             if (first) {
-                block_scan_256(scan, C.lncells, wsum);     // ends with a barrier: scan[] final
-                if (tid < 27) seg_beg[tid] = C.atom_off + scan[seg_cell[tid]];
+                block_scan<NT>(scan, lncells, wsum);     // ends with a barrier: scan[] final
+                if (tid < 27) seg_beg[tid] = atom_off + scan[seg_cell[tid]];
             }
         }
         if constexpr (!RANKED) {
@@ -535,7 +524,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
             L.lperm[slot] = a;
             L.linv[a] = slot;
             if (e16) L.lcs[slot] = lc;
-            tile_cur_mark(v, C, slot, tb);
+            if ((slot - atom_off) % kTile == 0) v.tcur[tile_first + (slot - atom_off) / kTile] = tb;   // tile_cur_mark
             si[r] = make_float4(meo.x, meo.y, meo.z, __int_as_float(slot));
             icount[r] = 0;
         }
@@ -560,7 +549,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
         }
         if (tid < kJPad) sj[jn + tid] = make_float4(kFarShift, kFarShift, kFarShift, 0.f);
         __syncthreads();
-        build_pass<W16>(sj, si, icount, ni, jn, rl2, nbcap, L.nb);
+        build_pass<W, W16>(sj, si, icount, ni, jn, rl2, nbcap, L.nb);
         k0 = k1;
     }
     __syncthreads();
@@ -642,19 +631,27 @@ hipError_t launch_list_rebuild(const DevView& v, int q, int cb, hipStream_t s)
         const int grid = v.nchains + (v.Cl + kRankWaves - 1) / kRankWaves;
         hipLaunchKernelGGL(k_lscan_chains, dim3(grid), dim3(1024), 0, s, v, q, cb);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        if (v.entry16) hipLaunchKernelGGL((k_lbuild<false, true, true>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
-        else hipLaunchKernelGGL((k_lbuild<false, false, true>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
+        if (v.entry16) hipLaunchKernelGGL((k_lbuild<kBuildWaves, false, true, true>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
+        else hipLaunchKernelGGL((k_lbuild<kBuildWaves, false, false, true>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
         return hipGetLastError();
     }
     if (v.lscan_in_build) {
-        if (v.entry16) hipLaunchKernelGGL((k_lbuild<true, true, false>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
-        else hipLaunchKernelGGL((k_lbuild<true, false, false>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
+        if (v.Cl <= kSmallBuild) {
+            const dim3 t(64 * kBuildWavesSmall);
+            if (v.entry16) hipLaunchKernelGGL((k_lbuild<kBuildWavesSmall, true, true, false>), dim3(v.Cl), t, dyn, s, v, q, cb);
+            else hipLaunchKernelGGL((k_lbuild<kBuildWavesSmall, true, false, false>), dim3(v.Cl), t, dyn, s, v, q, cb);
+            return hipGetLastError();
+        }
+        if (v.entry16) hipLaunchKernelGGL((k_lbuild<kBuildWaves, true, true, false>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
+        else hipLaunchKernelGGL((k_lbuild<kBuildWaves, true, false, false>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(k_lscan, dim3(1 + (v.Cl + kRankWaves - 1) / kRankWaves), dim3(1024), 0, s, v, q, cb);
+    const int parts = (v.Cl + kScanPart - 1) / kScanPart;
+    const int rankers = min((v.Cl + kRankWaves - 1) / kRankWaves, kRankGroups);
+    hipLaunchKernelGGL(k_lscan, dim3(parts + rankers), dim3(1024), 0, s, v, q, cb, parts);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if (v.entry16) hipLaunchKernelGGL((k_lbuild<false, true, true>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
-    else hipLaunchKernelGGL((k_lbuild<false, false, true>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
+    if (v.entry16) hipLaunchKernelGGL((k_lbuild<kBuildWaves, false, true, true>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
+    else hipLaunchKernelGGL((k_lbuild<kBuildWaves, false, false, true>), dim3(v.Cl), dim3(256), dyn, s, v, q, cb);
     return hipGetLastError();
 }
 
@@ -1105,11 +1102,7 @@ __global__ __launch_bounds__(256) void k_lenergy(DevView v, int q)
         if (val) load_seg_row<8>(L, C, s, sub, seg_tab[t]);
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        if (tl.begin == C.atom_off) *req(v, q, tl.chain) = 0;
-        if (blockIdx.x == 0) *req_any(v, q) = 0;
-    }
-    const int N = v.Ntot;
+    const int N = v.Ntot, atom_off = C.atom_off;
     const int* segs = reinterpret_cast<const int*>(seg_tab[W16 ? t : 0]);
     double au = 0.0, aw = 0.0, an = 0.0, ak = 0.0;
     if (val) {
@@ -1175,6 +1168,9 @@ __global__ __launch_bounds__(256) void k_lenergy(DevView v, int q)
     if (threadIdx.x == 0) {
         double* tp = &v.tile_part[4 * tile];
         tp[0] = au; tp[1] = aw; tp[2] = an; tp[3] = ak;
+        // the requests of this parity are consumed (last, so that the chain's constants above stay scalar loads)
+        if (tl.begin == atom_off) *req(v, q, tl.chain) = 0;
+        if (blockIdx.x == 0) *req_any(v, q) = 0;
     }
 }
 
