@@ -881,20 +881,43 @@ __global__ __launch_bounds__(kTile * LP) void k_lsweep(DevView v, double kick_dt
         }
     }
     __syncthreads();                                      // shift_tab, seg_tab
+    // the entries past the first batch, kRest per lane and step; past the count the no-op entry
+    constexpr int kRest = LP == 4 ? 4 : 2;
+    int k = sub + kBatch * LP;
+    unsigned er[kRest];
+    auto load_rest = [&] {
+#pragma unroll
+        for (int u = 0; u < kRest; u++) {
+            const int ku = min(k + u * LP, n - 1);
+            const unsigned e = W16 ? (unsigned)list_row<uint16_t>(v, L, s)[ku] : (unsigned)list_row<int>(v, L, s)[ku];
+            er[u] = k + u * LP < n ? e : W16 ? (unsigned)kPadEntry : ((unsigned)s << kImageBits) | kFarCode;
+        }
+    };
     if (val) {
         if constexpr (W16) {
             float4 pw[kBatch];
 #pragma unroll
             for (int u = 0; u < kBatch; u++) pw[u] = xq[slot_of(ent[u])];
+            if (k < n) load_rest();
 #pragma unroll
             for (int u = 0; u < kBatch; u++) pair(pw[u], ent[u]);
         } else {
+            if (k < n) load_rest();
 #pragma unroll
             for (int u = 0; u < kBatch; u++) pair(pj[u], ent[u]);
         }
-        for (int k = sub + kBatch * LP; k < n; k += LP) {
-            const unsigned ee = W16 ? (unsigned)list_row<uint16_t>(v, L, s)[k] : (unsigned)list_row<int>(v, L, s)[k];
-            pair(xq[slot_of(ee)], ee);
+        while (k < n) {
+            float4 pr[kRest];
+            unsigned ec[kRest];
+#pragma unroll
+            for (int u = 0; u < kRest; u++) {
+                ec[u] = er[u];
+                pr[u] = xq[slot_of(ec[u])];
+            }
+            k += kRest * LP;
+            if (k < n) load_rest();
+#pragma unroll
+            for (int u = 0; u < kRest; u++) pair(pr[u], ec[u]);
         }
     }
     // the tail's operands, fetched after the pairs (fewer registers live through the pair loop)
