@@ -699,7 +699,7 @@ __device__ __forceinline__ void list_drift_slot(const DevView& v, const ListBuf&
 // What the tail of a list sweep needs of its chain, read before the sweep's first store: read where it is
 // used, every one of these was a vector load of its own behind the stores (the compiler cannot know that they
 // leave the chain alone), a chain of seven load latencies at the end of each wave (sweep at N = 4001: 4.84 us,
-// now 4.36; at N = 1,048,576: 172 us, now 153).
+// then 4.36; at N = 1,048,576: 172 us, then 153).
 struct TailConst {
     double kdt, coeff_x, trig2, p2max;     // uniform
     double L, lsize;                       // of the lane's dimension
@@ -777,7 +777,7 @@ __device__ __forceinline__ void list_tail(const DevView& v, const ListBuf& L, co
 
 // LP lanes per slot, kTile slots per workgroup.  Each lane first loads up to kBatch of its list entries
 // and gathers their coordinates, so that one memory latency covers most lists; the per-atom tail (kick,
-// drift, next-parity coordinates, displacement test) runs on three lanes, one per dimension.  The
+// drift, next-parity coordinates, displacement test) runs on three lanes of four, one per dimension.  The
 // workgroup's list buffer comes from tcur[blockIdx], so nothing delays the first list load but the
 // tile's own two scalar loads.  32-bit entries (W16 false) carry the slot and the image code, so the
 // gathers are issued before the barrier that publishes the shift table.  16-bit entries (W16) are read
@@ -794,6 +794,7 @@ __global__ __launch_bounds__(kTile * LP) void k_lsweep(DevView v, double kick_dt
     constexpr int kShifts = W16 ? kSegStride : 64;
     __shared__ float4 shift_tab[kShifts];                // image shift by segment (W16) or 6-bit image code
     __shared__ int4 seg_tab[W16 ? kTile : 1][kSegStride / 4];   // W16: segment starts of each slot's cell
+    __shared__ float4 fsum[LP == 4 ? 1 : kTile];
     const int tile = xcd_block(blockIdx.x, v.ntiles);
     const Chunk tl = v.tiles[tile];
     const ListBuf L = list_buf(v, v.tcur[tile]);
@@ -802,15 +803,11 @@ __global__ __launch_bounds__(kTile * LP) void k_lsweep(DevView v, double kick_dt
     const int t = threadIdx.x / LP, sub = threadIdx.x % LP;
     const int s = tl.begin + t;
     const bool val = s < tl.end;
-    const int d = sub < 3 ? sub : 0;                      // the per-dimension tail runs on lanes 0, 1, 2
     const float4* __restrict__ xq = L.xsl + (size_t)q * N;
     const float eps48 = C.eps48_f;
     const int* segs = reinterpret_cast<const int*>(seg_tab[W16 ? t : 0]);
     float ax = 0.f, ay = 0.f, az = 0.f;
     float4 xi = make_float4(0.f, 0.f, 0.f, 0.f);
-    int atom = 0;
-    double p_d = 0.0, x_d = 0.0;
-    float4 ref = make_float4(0.f, 0.f, 0.f, 0.f);
     // neighbour slot and shift-table index of an entry
     auto slot_of = [&](unsigned e) -> unsigned {
         if constexpr (W16) return (unsigned)entry_slot(segs, e);
@@ -834,6 +831,27 @@ __global__ __launch_bounds__(kTile * LP) void k_lsweep(DevView v, double kick_dt
         ax = __builtin_fmaf(gq, dx, ax);
         ay = __builtin_fmaf(gq, dy, ay);
         az = __builtin_fmaf(gq, dz, az);
+    };
+    // the tail of slot st on four lanes: the operands, fetched after the pairs (fewer registers live through
+    // the pair loop: before them, the sweep of N = 1,048,576 lost a wave per SIMD and 2.5 %), then the update
+    auto tail = [&](int st, int ts, float fx, float fy, float fz) {
+        const int s = tl.begin + st;
+        const bool val = s < tl.end;
+        const int d = ts < 3 ? ts : 0;
+        int atom = 0;
+        double p_d = 0.0, x_d = 0.0;
+        float4 ref = make_float4(0.f, 0.f, 0.f, 0.f);
+        const TailConst tc = tail_const(v, C, kick_dt, d);
+        if (val && ts < 3) {
+            if constexpr ((MODE & LJ_STOREF) != 0) atom = L.lperm[s];     // the stored force is in atom order
+            p_d = v.pl[d * N + s];
+            if constexpr ((MODE & (LJ_DRIFT | LJ_REL64)) != 0) {
+                x_d = v.xl[d * N + s];
+                ref = L.lref[s];
+            }
+        }
+        list_tail<MODE, 4>(v, L, tc, tl, s, val, ts, d, atom, eps48 * (d == 0 ? fx : (d == 1 ? fy : fz)), p_d, x_d, ref,
+                           drift_dt, q, checked);
     };
     if (threadIdx.x < kShifts) {
         const int k = threadIdx.x;
@@ -872,7 +890,6 @@ __global__ __launch_bounds__(kTile * LP) void k_lsweep(DevView v, double kick_dt
 #pragma unroll
             for (int u = 0; u < kBatch; u++) ent[u] = (unsigned)nbs[sub + u * LP];
         }
-        if constexpr ((MODE & LJ_STOREF) != 0) atom = L.lperm[s];     // the stored force is in atom order
         xi = xq[s];
         n = L.nbn[s];
         if constexpr (!W16) {
@@ -881,7 +898,9 @@ __global__ __launch_bounds__(kTile * LP) void k_lsweep(DevView v, double kick_dt
         }
     }
     __syncthreads();                                      // shift_tab, seg_tab
-    // the entries past the first batch, kRest per lane and step; past the count the no-op entry
+    // the entries past the first batch, kRest per lane and step, a step's entries loaded ahead; past the count
+    // the no-op entry.  One entry at a time, each step was two memory latencies in sequence: 4 lanes a slot at
+    // densities up to 0.9 (rows of 49 to 82 entries, first batch 64; 617,055 atoms) 80.3 us, now 72.4
     constexpr int kRest = LP == 4 ? 4 : 2;
     int k = sub + kBatch * LP;
     unsigned er[kRest];
@@ -920,20 +939,23 @@ __global__ __launch_bounds__(kTile * LP) void k_lsweep(DevView v, double kick_dt
             for (int u = 0; u < kRest; u++) pair(pr[u], ec[u]);
         }
     }
-    // the tail's operands, fetched after the pairs (fewer registers live through the pair loop)
-    const TailConst tc = tail_const(v, C, kick_dt, d);
-    if (val && sub < 3) {
-        p_d = v.pl[d * N + s];
-        if constexpr ((MODE & (LJ_DRIFT | LJ_REL64)) != 0) {
-            x_d = v.xl[d * N + s];
-            ref = L.lref[s];
-        }
-    }
     ax = group_sum<LP>(ax);
     ay = group_sum<LP>(ay);
     az = group_sum<LP>(az);
-    list_tail<MODE, LP>(v, L, tc, tl, s, val, sub, d, atom, eps48 * (d == 0 ? ax : (d == 1 ? ay : az)), p_d, x_d, ref,
-                        drift_dt, q, checked);
+    // With more than four lanes a slot the sums go through LDS to the first four lanes per slot of the
+    // workgroup, so that half of its waves (8 lanes) run the tail's ~150 instructions with three lanes of
+    // four busy, not all of them with three of eight: the pairs and the gathers each fill about three
+    // quarters of the sweep, so their instructions count (N = 1,048,576: 152 -> 144 us; 8 x 32,768: 33.0 -> 30.5)
+    if constexpr (LP == 4) {
+        tail(t, sub, ax, ay, az);
+    } else {
+        if (sub == 0) fsum[t] = make_float4(ax, ay, az, 0.f);
+        __syncthreads();
+        if (threadIdx.x >= 4 * kTile) return;
+        const int tt = threadIdx.x >> 2;
+        const float4 f = fsum[tt];
+        tail(tt, threadIdx.x & 3, f.x, f.y, f.z);
+    }
 }
 
 // Surrogate forces on the lists (same tiles, lanes, entries and tail as k_lsweep): for every listed pair

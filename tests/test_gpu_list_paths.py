@@ -62,3 +62,37 @@ def test_build_lists_every_pair(chmc, N, L, bits):
         scale = np.sqrt(np.mean(f ** 2)) + np.max(np.abs(f)) * 1e-2
         near = 4e-2 * (48 * RC ** -7)            # a pair within 1e-6 of rc may fall on either side
         assert np.max(np.abs(fl - f)) <= 2e-4 * scale + near
+
+
+# rows below, at and past the first batch of every sweep shape (64 to 128 entries; about 125 rho entries a row),
+# with the steps after it partly and wholly filled, and a last tile of 5 slots
+@pytest.mark.parametrize("rho", [0.5, 0.72, 0.95, 1.1])
+@pytest.mark.parametrize("bits", [32, 16])
+def test_sweep_shapes_past_the_first_batch(chmc, rho, bits):
+    N, dt = 997, 0.004
+    L = (N / rho) ** (1 / 3)
+    i = np.arange(N)
+    rng = np.random.default_rng(7)
+    x = (np.stack((i % 10, (i // 10) % 10, i // 100), -1) + 0.5 + rng.uniform(-0.15, 0.15, (N, 3))) / 10 * L
+    p = rng.normal(size=(N, 3))
+    with chmc.Engine(chmc.Chain(N=N, L=L, cutoff=RC)) as e:
+        e.set_list_entry_bits(bits)
+        e.set_skin(SKIN)
+        first = None
+        for lanes in (8, 4, 16, 810, 811, 812, 816):
+            e.set_list_lanes(lanes)
+            e.set_positions(x)
+            e.set_momenta(p)
+            e.integrate(chmc.LEAPFROG, 0.0, 1)
+            fl = e.force()
+            e.compute_force(fp64=True)
+            f = e.force()
+            # the bound of the lists' forces above
+            bound = 2e-4 * (np.sqrt(np.mean(f ** 2)) + np.max(np.abs(f)) * 1e-2) + 4e-2 * (48 * RC ** -7)
+            assert np.max(np.abs(fl - f)) <= bound, lanes
+            e.integrate(chmc.LEAPFROG, dt, 3)
+            end = e.momenta()
+            # four kicks of dt with two forces each off by at most the bound (which also holds for the later
+            # configurations: their forces are not larger by more than a factor of two)
+            first = end if first is None else first
+            assert np.max(np.abs(end - first)) <= 4 * dt * 2 * 2 * bound, lanes
