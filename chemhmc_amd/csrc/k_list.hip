@@ -297,54 +297,76 @@ __device__ __forceinline__ void block_scan(int* a, int n, int* wsum)
     __syncthreads();
 }
 
-// U groups of 64 staged members from sj[j0] against the wave's own atom: the wave's hit mask straight
-// from the compares (4: ordered less, 2: ordered greater), the positions from mbcnt, the count in a
-// scalar.  Row offsets in 32 bits: Ntot * nbcap < 2^31 (checked at setup).  Entries of 16 or 32 bits (W16).
-template <int U, bool W16>
-__device__ __forceinline__ void build_step(const float4* sj, int j0, int lane, const float4& xi, float rl2,
-                                           int rowoff, int nbcap, char* __restrict__ nbb, int& count)
+// U groups of 64 staged members from sj[j0] against the wave's own atom: the hit mask is one unsigned compare of
+// r^2's bits less one (0 < r^2 < rl^2; rl2m is rl^2's bits less one; a NaN is larger), the position of a hit comes
+// from mbcnt, the row's count (n) is a scalar added to the store's address: 11 vector and 6 scalar instructions for
+// 64 tested pairs (two ordered compares, the count in a vector register and the capacity tested for every hit
+// took 14 and 9, and a rebuild of 617,055 atoms in 256 chains 305 us; now 296).  ROOM: the row has room for every
+// hit.  Entries of 16 or 32 bits (W16).
+template <int U, bool W16, bool ROOM>
+__device__ __forceinline__ void build_step(const float4* sj, int j0, int lane, const float4& xi, unsigned rl2m,
+                                           char* __restrict__ row, int nbcap, int& n)
 {
+    using E = std::conditional_t<W16, uint16_t, int>;
     float4 p[U];
-    float r2[U];
+    unsigned m2[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
         p[u] = sj[j0 + u * 64 + lane];
         const float dx = xi.x - p[u].x, dy = xi.y - p[u].y, dz = xi.z - p[u].z;
-        r2[u] = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+        m2[u] = (unsigned)__float_as_int(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx))) - 1u;
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
-        const unsigned long long hits = __builtin_amdgcn_fcmpf(r2[u], rl2, 4) & __builtin_amdgcn_fcmpf(r2[u], 0.f, 2);
-        const int pos = count + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(hits >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)hits, 0u));
-        if (r2[u] < rl2 && r2[u] > 0.f && pos < nbcap) {
-            if constexpr (W16) *reinterpret_cast<uint16_t*>(nbb + ((unsigned)(rowoff + pos) << 1)) = (uint16_t)__float_as_int(p[u].w);
-            else *reinterpret_cast<int*>(nbb + ((unsigned)(rowoff + pos) << 2)) = __float_as_int(p[u].w);
-        }
-        count += __popcll(hits);
+        const unsigned long long hits = __builtin_amdgcn_ballot_w64(m2[u] < rl2m);
+        const unsigned rank = __builtin_amdgcn_mbcnt_hi((unsigned)(hits >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)hits, 0u));
+        if (m2[u] < rl2m && (ROOM || n + (int)rank < nbcap))
+            *reinterpret_cast<E*>(row + (rank * (unsigned)sizeof(E) + (unsigned)n * (unsigned)sizeof(E))) = (E)__float_as_int(p[u].w);
+        n += __popcll(hits);
     }
 }
 
-// Pair tests of one staged pass: the own atoms si[0, ni) (slot in w, entry counts in icount) against the
-// staged members sj[0, jn), padded with kJPad far entries.  Each wave takes one own atom at a time and
-// its 64 lanes test 64 members each step, branch-free (the far padding fails every test); the hits are
-// appended in staging order.  With one own atom per wave the hit mask is wave-uniform (~12 VALU per
-// group of 64 tested pairs; two own atoms x 32 members took ~18 and 6-9 % more build time).  The loop
-// reads two groups of 64 while the second starts inside the members, then at most one more, so no read
-// passes jn + 63 and the padding stays one group.
+// What the rows of one staged pass are built from: the staged members sj[0, jn), padded with kJPad far entries
+struct BuildPass {
+    const float4* sj;
+    int jn;
+    float rl2;
+    int nbcap, span;
+    char* nb;              // the rows
+    bool first, last;      // of the passes; the last one finishes the rows
+};
+
+// Pair tests of one staged pass: the own atoms si[0, ni) (slot in w, entry counts in icount) against the staged
+// members.  Each wave takes one own atom at a time and its 64 lanes test 64 members each step, branch-free (the
+// far padding fails every test); the hits are appended in staging order.  With one own atom per wave the hit mask
+// is wave-uniform (two own atoms x 32 members took half as many instructions again and 6-9 % more build time; to
+// list the members near each quadrant of the cell first, and to test its atoms against those, took 16 % fewer
+// instructions and 6 % more time, in dependent LDS reads).  The loop reads two groups of 64 while the second
+// starts inside the members and the row has room for every hit, then one at a time, so no read passes jn + 63 and
+// the padding stays one group.
+// A finished row is padded past its count with no-op entries to the sweep shape's unconditional span.
 template <int W, bool W16>
-__device__ __forceinline__ void build_pass(const float4* sj, const float4* si, int* icount, int ni, int jn,
-                                           float rl2, int nbcap, char* __restrict__ nbb)
+__device__ __forceinline__ void build_pass(const BuildPass& B, const float4* si, int* icount, int ni, int tid)
 {
     static_assert(kJPad >= 64, "every step reads fewer than 64 entries past the members");
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned rl2m = (unsigned)__float_as_int(B.rl2) - 1u;
+    using E = std::conditional_t<W16, uint16_t, int>;
+    const size_t stride = (size_t)B.nbcap * sizeof(E);
     for (int i = wave; i < ni; i += W) {
         const float4 xi = si[i];
-        int count = icount[i];
-        const int rowoff = __float_as_int(xi.w) * nbcap;
+        const int slot = __builtin_amdgcn_readfirstlane(__float_as_int(xi.w));
+        int n = B.first ? 0 : __builtin_amdgcn_readfirstlane(icount[i]);
+        char* __restrict__ row = B.nb + (size_t)slot * stride;
         int j0 = 0;
-        for (; j0 + 64 < jn; j0 += 128) build_step<2, W16>(sj, j0, lane, xi, rl2, rowoff, nbcap, nbb, count);
-        if (j0 < jn) build_step<1, W16>(sj, j0, lane, xi, rl2, rowoff, nbcap, nbb, count);
-        if (lane == 0) icount[i] = count;
+        for (; j0 + 64 < B.jn && n + 128 <= B.nbcap; j0 += 128) build_step<2, W16, true>(B.sj, j0, lane, xi, rl2m, row, B.nbcap, n);
+        for (; j0 < B.jn; j0 += 64) build_step<1, W16, false>(B.sj, j0, lane, xi, rl2m, row, B.nbcap, n);
+        if (B.last) {
+            const E pad = W16 ? (E)kPadEntry : (E)((slot << kImageBits) | kFarCode);
+            for (int k = n; k < B.span; k += 64)
+                if (k + lane < B.span) reinterpret_cast<E*>(row)[k + lane] = pad;
+        }
+        if (lane == 0) icount[i] = n;
     }
 }
 
@@ -424,7 +446,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == kBu
 #pragma unroll
             for (int d = 0; d < 3; d++) {
                 j3[d] = b3[d] + dd[d];
-                if (j3[d] < 0 || j3[d] >= n3[d]) j3[d] = (b3[d] + n3[d] + dd[d]) % n3[d];
+                j3[d] += j3[d] < 0 ? n3[d] : j3[d] >= n3[d] ? -n3[d] : 0;
                 seg_sh[lane][d] = (float)dd[d] * C.lsize_f[d];
             }
             const int jl = j3[0] + nx * (j3[1] + j3[2] * ny);
@@ -460,7 +482,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == kBu
     const int ni = seg_cnt[13];                      // segment 13: the cell itself (ni <= lcap <= 256)
     if (ni == 0) return;
 
-    const int nbcap = v.nbcap;
+    const int nbcap = v.nbcap, span = v.lspan;
     int ibeg = 0;
     for (int k0 = 0; k0 < 27;) {
         const bool first = k0 == 0;
@@ -526,7 +548,6 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == kBu
             if (e16) L.lcs[slot] = lc;
             if ((slot - atom_off) % kTile == 0) v.tcur[tile_first + (slot - atom_off) / kTile] = tb;   // tile_cur_mark
             si[r] = make_float4(meo.x, meo.y, meo.z, __int_as_float(slot));
-            icount[r] = 0;
         }
 #pragma unroll
         for (int u = 0; u < PT; u++) {
@@ -549,7 +570,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == kBu
         }
         if (tid < kJPad) sj[jn + tid] = make_float4(kFarShift, kFarShift, kFarShift, 0.f);
         __syncthreads();
-        build_pass<W, W16>(sj, si, icount, ni, jn, rl2, nbcap, L.nb);
+        const BuildPass B = { sj, jn, rl2, nbcap, span, L.nb, first, k1 == 27 };
+        build_pass<W, W16>(B, si, icount, ni, tid);
         k0 = k1;
     }
     __syncthreads();
@@ -557,19 +579,6 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == kBu
         const int n = icount[r];
         L.nbn[ibeg + r] = min(n, nbcap);
         if (n > nbcap) atomicOr(&v.lflag[2], 2);
-    }
-    // rows padded to the sweep shape's unconditional span with no-op entries
-    const int span = v.lspan;
-    for (int r = wave; r < ni; r += W) {
-        const int slot = __float_as_int(si[r].w);
-        if (e16) {
-            uint16_t* __restrict__ row = list_row<uint16_t>(v, L, slot);
-            for (int k = icount[r] + lane; k < span; k += 64) row[k] = kPadEntry;
-        } else {
-            int* __restrict__ row = list_row<int>(v, L, slot);
-            const int pad = (slot << kImageBits) | kFarCode;
-            for (int k = icount[r] + lane; k < span; k += 64) row[k] = pad;
-        }
     }
 }
 
