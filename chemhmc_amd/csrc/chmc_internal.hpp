@@ -351,7 +351,7 @@ __device__ __forceinline__ int* perm_next(const DevView& v) { return v.perm_buf 
 hipError_t launch_count(const DevView& v, double drift_dt, hipStream_t s);
 hipError_t launch_scan(const DevView& v, hipStream_t s);
 hipError_t launch_place(const DevView& v, bool atom_id_order, hipStream_t s);
-constexpr int kBinSmall = 4096;
+constexpr int kBinSmall = 3072;
 inline bool bin_small(const DevView& v) { return v.Ntot <= kBinSmall && v.Ctot <= kBinSmall; }
 hipError_t launch_bin_small(const DevView& v, double drift_dt, bool atom_id_order, hipStream_t s);
 

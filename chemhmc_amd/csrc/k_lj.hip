@@ -198,7 +198,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_lj(DevView v, double kick_dt, d
 }
 
 // ---- FP64 sweep ------------------------------------------------------------------------------------
-// One workgroup of W wavefronts per i-cell, one wave per i-atom.  The 64 lanes test 64 staged j entries a step
+// One workgroup of W wavefronts per i-cell, or `parts` of them (forces), one wave per i-atom.  The 64 lanes test 64 staged j entries a step
 // (FP64 coordinates relative to the i-cell origin, 0 < r^2 < rc^2), and the pairs inside (14 % of the candidates
 // at liquid density) are appended by ballot prefix to the wave's LDS list; whenever 64 are pending, and at the
 // end, the lanes take one each and evaluate it: reciprocal from v_rcp_f64 with two Newton steps, per-lane sums.
@@ -207,15 +207,23 @@ __global__ __launch_bounds__(64 * kWaves) void k_lj(DevView v, double kick_dt, d
 //   the cell's atoms); reduced once in a fixed order into per-cell partials that the chain reduction sums.
 // Self-exclusion is r^2 > 0: the i-atom is its own staged copy.
 // Bound: VALU issue of the tests (14 instructions per 64 candidates) and the workgroups' start at large N, latency
-// at small N, where W = 16 leaves a wave one or two atoms (kSmallCells).  Evaluating every candidate, 8 i-slots x
-// 8 j-groups a wave, took 23.4 us at N = 512 (27 cells: chains of 128 dependent iterations) and 169 us for the
-// energy at N = 250,047; now 8.7 us (kick) and 110 us.  An FP32 copy of the entries for the tests cost more in LDS (6 instead of
-// 8 workgroups a CU) than its narrower reads saved (118 us there).
+// at small N.  Evaluating every candidate, 8 i-slots x 8 j-groups a wave, took 23.4 us at N = 512 (27 cells: chains
+// of 128 dependent iterations) and 169 us for the energy at N = 250,047; one wave per atom 8.7 us (kick) and 110 us.
+// An FP32 copy of the entries for the tests cost more in LDS (6 instead of 8 workgroups a CU) than its narrower
+// reads saved (118 us there).
+// Forces of up to kWideCells cells: workgroups of 8 waves, and so many per cell that a wave has one atom (1.3 times
+// the mean occupancy), as long as the launch stays within kForceGroups, two rounds of 2 a CU: 16 waves for each of
+// 27 cells used a tenth of the CUs, and most waves ran a second atom after the first.  A leapfrog step of the FP64
+// path (with its binning): N = 256 23.2 -> 13.7 us, 512 14.1 -> 12.4, 800 24.4 -> 15.6; 8,000 (512 cells, two each
+// instead of one of four waves) 30.2 -> 26.4, 16,384 36.0 -> 32.4.  From 2,197 cells on the chip is full and four
+// waves are as fast (42.8 against 42.2 us), from 4,096 faster (58.1 against 61.5).
+// Energies need a cell's sums in one workgroup: 16 waves below kSmallCells cells, else 4.
+constexpr int kWideCells = 2048, kForceGroups = 1024;
 constexpr int kSmallCells = 512;
 constexpr int kMaxJ64 = 512;          // j entries per LDS pass: seven workgroups of four waves a CU
 
 template <int W, int MODE>
-__global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt)
+__global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt, int parts)
 {
     constexpr int NT = 64 * W, PEND = 128;
     __shared__ double sx[kMaxJ64 + 64], sy[kMaxJ64 + 64], sz[kMaxJ64 + 64];     // padded with far entries
@@ -224,7 +232,7 @@ __global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt)
     __shared__ double seg_sh[27][3];
     __shared__ double wsum[W][4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c = xcd_block(blockIdx.x, v.Ctot);
+    const int item = xcd_block(blockIdx.x, v.Ctot * parts), c = item / parts, first = (item - c * parts) * W, step = W * parts;
     const ChainDev& C = v.chains[v.cell_chain[c]];
     const int nx = C.nbin[0], ny = C.nbin[1], nz = C.nbin[2];
     const int lc = c - C.cell_off;
@@ -235,7 +243,7 @@ __global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt)
     const int N = v.Ntot;
     double au = 0.0, aw = 0.0, ak = 0.0;
     int an = 0;
-    if (ni > 0) {
+    if (ni > first) {
         if (wave == 0) {
             int cnt = 0;
             if (lane < 27) {
@@ -286,9 +294,9 @@ __global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt)
         const double rc2 = C.rc2, sig2 = C.sigma2;
         const double kdt = kick_dt * C.beta;              // dt * coeff_p, coeff_p = beta (:642-644)
         // every wave runs the same number of rounds so that the multi-pass staging barriers match
-        const int rounds = (ni + W - 1) / W;
+        const int rounds = (ni - first + step - 1) / step;
         for (int rnd = 0; rnd < rounds; rnd++) {
-            const int i = rnd * W + wave;
+            const int i = rnd * step + first + wave;
             const bool ival = i < ni;                     // wave-uniform
             // the i-atom: its own staged copy (segment 13) where the whole j-list is staged
             double xi, yi, zi;
@@ -426,10 +434,16 @@ __global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt)
 template <int MODE>
 static hipError_t launch_lj64(const DevView& v, double kick_dt, hipStream_t s)
 {
-    if (v.Ctot < kSmallCells)
-        hipLaunchKernelGGL((k_lj64<16, MODE>), dim3(v.Ctot), dim3(1024), 0, s, v, kick_dt);
-    else
-        hipLaunchKernelGGL((k_lj64<4, MODE>), dim3(v.Ctot), dim3(256), 0, s, v, kick_dt);
+    if constexpr ((MODE & LJ_ENERGY) != 0) {
+        if (v.Ctot < kSmallCells) hipLaunchKernelGGL((k_lj64<16, MODE>), dim3(v.Ctot), dim3(1024), 0, s, v, kick_dt, 1);
+        else hipLaunchKernelGGL((k_lj64<4, MODE>), dim3(v.Ctot), dim3(256), 0, s, v, kick_dt, 1);
+    } else if (v.Ctot <= kWideCells) {
+        const int need = (int)((13LL * v.Ntot + 80LL * v.Ctot - 1) / (80LL * v.Ctot));     // waves for 1.3 x the mean, in eights
+        const int parts = std::min(need, std::max(1, kForceGroups / v.Ctot));
+        hipLaunchKernelGGL((k_lj64<8, MODE>), dim3(v.Ctot * parts), dim3(512), 0, s, v, kick_dt, parts);
+    } else {
+        hipLaunchKernelGGL((k_lj64<4, MODE>), dim3(v.Ctot), dim3(256), 0, s, v, kick_dt, 1);
+    }
     return hipGetLastError();
 }
 

@@ -1,4 +1,4 @@
-"""Binning at the edges of its paths (one workgroup up to 4096 atoms and cells, four launches beyond),
+"""Binning at the edges of its paths (one workgroup up to 3072 atoms and cells, four launches beyond),
 against the FP64 oracle's stable counting sort: bitwise."""
 import numpy as np
 import pytest
@@ -15,10 +15,11 @@ def _check(e, orc, x, L, prev, chain=0):
     return perm
 
 
-# one atom, one cell, the last sizes of one workgroup (4096 atoms, 4096 cells) and the first beyond in either
+# one atom, one cell, the last sizes of one workgroup (3072 atoms, 3072 cells) and the first beyond in either
 @pytest.mark.parametrize("N,L,order", [
     (1, 6.0, False), (7, 2.6, False), (1023, 11.0, False), (1025, (8.0, 13.0, 40.0), False), (4096, 40.0, False),
-    (4096, 17.0, True), (4095, 17.0, False), (4097, 17.0, False), (3000, 43.0, False), (3000, 43.0, True)])
+    (4096, 17.0, True), (4095, 17.0, False), (4097, 17.0, False), (3000, 43.0, False), (3000, 43.0, True),
+    (3072, (40.0, 40.0, 30.0), False), (3073, 17.0, True), (2000, (40.0, 40.0, 32.5), False)])
 def test_binning_sizes(chmc, orc, N, L, order):
     box = np.broadcast_to(np.asarray(L, float), (3,)).copy()
     rng = np.random.default_rng(N)
