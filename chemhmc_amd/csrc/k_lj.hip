@@ -199,16 +199,18 @@ __global__ __launch_bounds__(64 * kWaves) void k_lj(DevView v, double kick_dt, d
 
 // ---- FP64 sweep ------------------------------------------------------------------------------------
 // One workgroup of W wavefronts per i-cell, or `parts` of them (forces), one wave per i-atom.  The 64 lanes test 64 staged j entries a step
-// (FP64 coordinates relative to the i-cell origin, 0 < r^2 < rc^2), and the pairs inside (14 % of the candidates
+// (FP64 coordinates relative to the i-cell origin, r^2 < rc^2), and the pairs inside (14 % of the candidates
 // at liquid density) are appended by ballot prefix to the wave's LDS list; whenever 64 are pending, and at the
 // end, the lanes take one each and evaluate it: reciprocal from v_rcp_f64 with two Newton steps, per-lane sums.
 //   LJ_FORCE: a butterfly over the wave sums the three components per atom; lanes 0..2 store and kick.
 //   LJ_ENERGY: per-lane energy, virial and pair sums run on over the wave's atoms (and the kinetic energy over
 //   the cell's atoms); reduced once in a fixed order into per-cell partials that the chain reduction sums.
 // Self-exclusion is r^2 > 0: the i-atom is its own staged copy.
-// Bound: VALU issue of the tests (14 instructions per 64 candidates) and the workgroups' start at large N, latency
-// at small N.  Evaluating every candidate, 8 i-slots x 8 j-groups a wave, took 23.4 us at N = 512 (27 cells: chains
-// of 128 dependent iterations) and 169 us for the energy at N = 250,047; one wave per atom 8.7 us (kick) and 110 us.
+// Bound: VALU issue of the tests (12 instructions per 64 candidates, the next step's entries loaded ahead; r^2 > 0 is
+// tested with the pairs inside only, entries are LDS byte offsets) and the workgroups' start at large N, latency at
+// small N.  Evaluating every candidate, 8 i-slots x 8 j-groups a wave, took 23.4 us at N = 512 (27 cells: chains
+// of 128 dependent iterations) and 169 us for the energy at N = 250,047; one wave per atom 8.7 us (kick) and 110 us;
+// the tests' shorter steps (16 instructions before) 106 us there, and 0.5 us of a leapfrog step at N = 512.
 // An FP32 copy of the entries for the tests cost more in LDS (6 instead of 8 workgroups a CU) than its narrower
 // reads saved (118 us there).
 // Forces of up to kWideCells cells: workgroups of 8 waves, and so many per cell that a wave has one atom (1.3 times
@@ -226,7 +228,9 @@ template <int W, int MODE>
 __global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt, int parts)
 {
     constexpr int NT = 64 * W, PEND = 128;
-    __shared__ double sx[kMaxJ64 + 64], sy[kMaxJ64 + 64], sz[kMaxJ64 + 64];     // padded with far entries
+    constexpr double kFar2 = 1.0e36;
+    auto at8 = [](const double* a, unsigned j8) { return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(a) + j8); };
+    __shared__ double sx[kMaxJ64 + 128], sy[kMaxJ64 + 128], sz[kMaxJ64 + 128];     // padded with far entries
     __shared__ unsigned short pend[W][PEND];
     __shared__ int seg_beg[27], seg_pref[28];
     __shared__ double seg_sh[27][3];
@@ -284,7 +288,7 @@ __global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt, int 
                 sy[t - jlo] = v.xs64[(size_t)N + src] + seg_sh[k][1];
                 sz[t - jlo] = v.xs64[2 * (size_t)N + src] + seg_sh[k][2];
             }
-            if (tid < 64) sx[jhi - jlo + tid] = sy[jhi - jlo + tid] = sz[jhi - jlo + tid] = (double)kFarShift;
+            if (tid < 128) sx[jhi - jlo + tid] = sy[jhi - jlo + tid] = sz[jhi - jlo + tid] = (double)kFarShift;
         };
         const bool single = nj <= kMaxJ64;
         if (single) {
@@ -316,22 +320,25 @@ __global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt, int 
             double p_d = 0.0;
             if constexpr ((MODE & LJ_KICK) != 0) p_d = v.p[(size_t)min(lane, 2) * N + atom];
             double ax = 0.0, ay = 0.0, az = 0.0;
+            // the pending pair of this lane; the i-atom itself and coincident ones (r^2 = 0) count as far away
             auto evaluate = [&](bool on) {
-                const int j = pend[wave][on ? lane : 0];
-                const double dx = xi - sx[j], dy = yi - sy[j], dz = zi - sz[j];
-                const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+                const unsigned j8 = pend[wave][on ? lane : 0];
+                const double dx = xi - at8(sx, j8), dy = yi - at8(sy, j8), dz = zi - at8(sz, j8);
+                double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+                on = on && r2 > 0.0;
+                r2 = on ? r2 : kFar2;
                 const double inv = rcp64(r2);
                 const double s2 = sig2 * inv;
                 const double s6 = s2 * s2 * s2;
                 if constexpr ((MODE & LJ_FORCE) != 0) {
-                    const double gq = on ? s6 * (0.5 - s6) * inv : 0.0;      // sr6 (0.5 - sr6) / r^2, :611-613
+                    const double gq = s6 * (0.5 - s6) * inv;                 // sr6 (0.5 - sr6) / r^2, :611-613
                     ax = __builtin_fma(gq, dx, ax);
                     ay = __builtin_fma(gq, dy, ay);
                     az = __builtin_fma(gq, dz, az);
                 }
                 if constexpr ((MODE & LJ_ENERGY) != 0) {
-                    au += on ? s6 * (s6 - 1.0) : 0.0;
-                    aw += on ? s6 * (s6 - 0.5) : 0.0;
+                    au += s6 * (s6 - 1.0);
+                    aw += s6 * (s6 - 0.5);
                     an += on ? 1 : 0;
                 }
             };
@@ -349,13 +356,19 @@ __global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt, int 
                 }
                 if (!ival) continue;
                 int np = 0;
+                unsigned j8 = 8u * (unsigned)lane;
+                double px = at8(sx, j8), py = at8(sy, j8), pz = at8(sz, j8);
                 for (int j0 = 0; j0 < jn; j0 += 64) {
-                    const double dx = xi - sx[j0 + lane], dy = yi - sy[j0 + lane], dz = zi - sz[j0 + lane];
+                    const double dx = xi - px, dy = yi - py, dz = zi - pz;
+                    const unsigned t8 = j8;
+                    j8 += 512u;                           // the next step's entries (the padding after the last)
+                    px = at8(sx, j8);
+                    py = at8(sy, j8);
+                    pz = at8(sz, j8);
                     const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
-                    const bool hit = r2 < rc2 && r2 > 0.0;
-                    const unsigned long long m = __ballot(hit);
-                    const int pos = np + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-                    if (hit) pend[wave][pos] = (unsigned short)(j0 + lane);
+                    const unsigned long long m = __builtin_amdgcn_fcmp(r2, rc2, 4);            // ordered less
+                    const unsigned pos = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+                    if (r2 < rc2) (pend[wave] + np)[pos] = (unsigned short)t8;
                     np += __popcll(m);
                     if (np >= 64) {                       // np - 64 < 64 stay pending
                         lds_sync();
