@@ -1122,21 +1122,18 @@ __global__ __launch_bounds__(256) void k_lrel64(DevView v)
     for (int d = 0; d < 3; d++) v.rel64[4 * (size_t)s + d] = list_rel(C, ref, d, v.xl[d * N + s]);
 }
 
-__device__ __forceinline__ double tile_sum_256(double s, double* part)
+__device__ __forceinline__ double wave_sum64(double s)
 {
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) s += __shfl_xor(s, m, 64);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
-    __syncthreads();
-    return ((part[0] + part[1]) + part[2]) + part[3];
+    s = group_sum<16>(s);
+    s += __shfl_xor(s, 16, 64);
+    return s + __shfl_xor(s, 32, 64);
 }
 
 template <bool W16>
 __global__ __launch_bounds__(256) void k_lenergy(DevView v, int q)
 {
     constexpr int kShifts = W16 ? kSegStride : 64;
-    __shared__ double wpart[4];
+    __shared__ double wpart[4][4];
     __shared__ double shift64[kShifts][3];              // image shift by segment or image code, exact in FP64
     __shared__ int4 seg_tab[W16 ? kTile : 1][kSegStride / 4];   // W16: segment starts of each slot's cell
     const int tile = xcd_block(blockIdx.x, v.ntiles);
@@ -1176,10 +1173,16 @@ __global__ __launch_bounds__(256) void k_lenergy(DevView v, int q)
         // increasing order.  Entries past the count read the row's last one (with 16-bit entries only
         // those below the count, and the padding, decode to slots of this buffer).
         constexpr int kEB = 4;
+        unsigned next[kEB];
+        auto load = [&](int k0) {
+#pragma unroll
+            for (int u = 0; u < kEB; u++) next[u] = (unsigned)nbs[min(k0 + 8 * u, n - 1)];
+        };
+        if (sub < n) load(sub);
         for (int k0 = sub; k0 < n; k0 += 8 * kEB) {
             unsigned ent[kEB];
 #pragma unroll
-            for (int u = 0; u < kEB; u++) ent[u] = (unsigned)nbs[min(k0 + 8 * u, n - 1)];
+            for (int u = 0; u < kEB; u++) ent[u] = next[u];
             double2 ja[kEB];
             double jz[kEB];
 #pragma unroll
@@ -1188,6 +1191,7 @@ __global__ __launch_bounds__(256) void k_lenergy(DevView v, int q)
                 ja[u] = r64[2 * j];
                 jz[u] = v.rel64[4 * j + 2];
             }
+            if (k0 + 8 * kEB < n) load(k0 + 8 * kEB);
 #pragma unroll
             for (int u = 0; u < kEB; u++) {
                 const bool live = k0 + 8 * u < n;
@@ -1215,13 +1219,19 @@ __global__ __launch_bounds__(256) void k_lenergy(DevView v, int q)
             ak = (px * px + py * py + pz * pz) / (2 * C.mass);
         }
     }
-    au = tile_sum_256(au, wpart);
-    aw = tile_sum_256(aw, wpart);
-    an = tile_sum_256(an, wpart);
-    ak = tile_sum_256(ak, wpart);
+    // the four sums of the tile: butterflies in each wave (the first four steps without LDS), then one barrier
+    const double s4[4] = { au, aw, an, ak };
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const double t = wave_sum64(s4[k]);
+        if ((threadIdx.x & 63) == 0) wpart[k][threadIdx.x >> 6] = t;
+    }
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        const double* w = wpart[threadIdx.x];
+        v.tile_part[4 * tile + threadIdx.x] = ((w[0] + w[1]) + w[2]) + w[3];
+    }
     if (threadIdx.x == 0) {
-        double* tp = &v.tile_part[4 * tile];
-        tp[0] = au; tp[1] = aw; tp[2] = an; tp[3] = ak;
         // the requests of this parity are consumed (last, so that the chain's constants above stay scalar loads)
         if (tl.begin == atom_off) *req(v, q, tl.chain) = 0;
         if (blockIdx.x == 0) *req_any(v, q) = 0;

@@ -228,7 +228,7 @@ template <int W, int MODE>
 __global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt, int parts)
 {
     constexpr int NT = 64 * W, PEND = 128;
-    constexpr double kFar2 = 1.0e36;
+    constexpr double kFar2 = 1.0e300;     // its twelfth power underflows: no contribution
     auto at8 = [](const double* a, unsigned j8) { return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(a) + j8); };
     __shared__ double sx[kMaxJ64 + 128], sy[kMaxJ64 + 128], sz[kMaxJ64 + 128];     // padded with far entries
     __shared__ unsigned short pend[W][PEND];
