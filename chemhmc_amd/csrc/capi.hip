@@ -1709,7 +1709,7 @@ extern "C" int chmc_rdf(chmc_ctx* c, int chain, int nbins, double size_bin, unsi
         HIPCHK(c, hipMalloc(&c->d_rdfu, sizeof(uint4) * cd.natoms));
         c->rdfu_cap = cd.natoms;
     }
-    HIPCHK(c, launch_rdf(c->v, chain, cd.natoms, nbins, size_bin, c->d_rdfu, c->d_rdf, c->stream));
+    HIPCHK(c, launch_rdf(c->v, chain, cd.natoms, cd.L[0] == cd.L[1] && cd.L[1] == cd.L[2], nbins, size_bin, c->d_rdfu, c->d_rdf, c->stream));
     std::vector<unsigned long long> h(nbins);
     HIPCHK(c, hipMemcpyAsync(h.data(), c->d_rdf, sizeof(unsigned long long) * nbins, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));

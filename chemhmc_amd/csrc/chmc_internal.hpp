@@ -405,7 +405,7 @@ hipError_t launch_list_drift(const DevView& v, int q, double dt, hipStream_t s);
 // rel64: compute the FP64 relative positions first (false when the last sweep wrote them)
 hipError_t launch_list_energy(const DevView& v, int q, bool rel64, hipStream_t s);
 // u: natoms fixed-point coordinates of scratch; counts: nbins, cleared here
-hipError_t launch_rdf(const DevView& v, int chain, int natoms, int nbins, double size_bin, uint4* u,
+hipError_t launch_rdf(const DevView& v, int chain, int natoms, bool cube, int nbins, double size_bin, uint4* u,
                       unsigned long long* counts, hipStream_t s);
 // the open-boundary sum over n atoms (AoS) in T x T tiles, T = open_potential_tiles(n); partials: T * T doubles
 constexpr int kOpenSmall = 16384;

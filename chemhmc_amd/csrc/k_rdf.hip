@@ -59,12 +59,15 @@ constexpr int kRdfJ = 32;          // j atoms per step of a workgroup
 // workgroup, added to the global counters once at its end.
 //   FP32 decision: with u exact to 2^-33 L, t = |d| / size_bin from three integer differences, converted,
 // scaled and summed in FP32 is within 6.5 * 2^-24 t + 2^-32 |L| / size_bin of the exact quotient (3 roundings
-// per component, 3 of the sum of squares, halved by the root, and 1 ulp of v_sqrt_f32).  A pair whose t is
+// per component, 3 of the sum of squares, halved by the root, and 1 ulp of v_sqrt_f32; in a cube (CUBE) the root
+// is scaled instead of the components: 2 roundings for 2).  A pair whose t is
 // farther than eps from an integer, eps = (nbins + 1) 2^-21 + 2^-31 |L| / size_bin, therefore has the exact
 // bin (int)t; the others (0.05 % at 500 bins) and any NaN are binned in FP64.  Bins from nbins + 1 up are
 // never counted and need no decision.
-//   Bound: VALU issue, ~22 slots a pair.  N = 32768, 500 bins up to L / 2 (5.4e8 pairs): 308 us, at the
-// VALU time of those slots (300 us), against 1531 us with the FP64 root and division for every pair.
+//   Bound: VALU issue, ~20 slots a pair (22 outside a cube).  N = 32768, 500 bins up to L / 2 (5.4e8 pairs): 271 us,
+// against 308 us with the components scaled and the tests repeated as selects, and 1531 us with the FP64 root and
+// division for every pair.
+template <bool CUBE>
 __global__ __launch_bounds__(256) void k_rdf(DevView v, int chain, int nbins, double size_bin,
                                              const uint4* __restrict__ u, unsigned long long* __restrict__ counts)
 {
@@ -86,7 +89,7 @@ __global__ __launch_bounds__(256) void k_rdf(DevView v, int chain, int nbins, do
                 sz = (float)(C.L[2] / 4294967296.0 / size_bin);
     const double diag = sqrt(C.L[0] * C.L[0] + C.L[1] * C.L[1] + C.L[2] * C.L[2]);
     const float half = (float)(0.5 - ((nbins + 1) / 2097152.0 + diag / size_bin / 2147483648.0) - 1e-7);
-    const float edge = (float)(nbins + 1);
+    const float edge = (float)(nbins + 1), nb = (float)nbins;
     auto exact = [&](int j) {
         const int b = rdf_bin_exact(C, xi, yi, zi, v.x[off + j], v.x[(size_t)N + off + j], v.x[2 * (size_t)N + off + j], size_bin);
         if (b < nbins) atomicAdd(&hist[b], 1u);
@@ -98,18 +101,28 @@ __global__ __launch_bounds__(256) void k_rdf(DevView v, int chain, int nbins, do
 #pragma unroll
         for (int k = 0; k < KB; k++) {
             const uint4 uj = u[j0 + k];
-            const float dx = sx * (float)(int)(uj.x - ui.x), dy = sy * (float)(int)(uj.y - ui.y), dz = sz * (float)(int)(uj.z - ui.z);
+            float dx = (float)(int)(uj.x - ui.x), dy = (float)(int)(uj.y - ui.y), dz = (float)(int)(uj.z - ui.z);
+            if constexpr (!CUBE) {
+                dx *= sx;
+                dy *= sy;
+                dz *= sz;
+            }
             t[k] = __builtin_amdgcn_sqrtf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)));
+            if constexpr (CUBE) t[k] *= sx;
         }
         unsigned late = 0u;
 #pragma unroll
         for (int k = 0; k < KB; k++) {
-            const bool on = !check || (ival && j0 + k > i);
-            // not clearly inside a bin, and not clearly beyond the last one (either is true for a NaN)
-            const bool un = on && !(fabsf(__builtin_amdgcn_fractf(t[k]) - 0.5f) <= half) && !(t[k] >= edge);
-            late |= un ? 1u << k : 0u;
-            const int b = (int)t[k];
-            if (on && !un && b < nbins) atomicAdd(&hist[b], 1u);
+            // clearly inside a bin; a pair that is not, and not clearly beyond the last bin, is decided exactly
+            // (a NaN is neither).  Whole waves; the masks of the compares themselves (5: ordered <=, 4: <, 3: >=)
+            const float mid = fabsf(__builtin_amdgcn_fractf(t[k]) - 0.5f);
+            const unsigned long long on = check ? __ballot(ival && j0 + k > i) : ~0ull;
+            const unsigned long long sure = __builtin_amdgcn_fcmpf(mid, half, 5);
+            if (__builtin_amdgcn_inverse_ballot_w64(sure & on & __builtin_amdgcn_fcmpf(t[k], nb, 4))) atomicAdd(&hist[(int)t[k]], 1u);
+            const unsigned long long un = on & ~sure;
+            if (un != 0ull) {                      // rare
+                if (__builtin_amdgcn_inverse_ballot_w64(un & ~__builtin_amdgcn_fcmpf(t[k], edge, 3))) late |= 1u << k;
+            }
         }
         if (__ballot(late != 0u) != 0ull)
             while (late != 0u) {
@@ -218,7 +231,7 @@ __global__ __launch_bounds__(1024) void k_open_sum(const double* __restrict__ pa
 
 // about 2048 workgroups (8 a CU): few enough that adding their histograms to the counters stays small,
 // rows in order, so that the long ones start first
-hipError_t launch_rdf(const DevView& v, int chain, int natoms, int nbins, double size_bin, uint4* u,
+hipError_t launch_rdf(const DevView& v, int chain, int natoms, bool cube, int nbins, double size_bin, uint4* u,
                       unsigned long long* counts, hipStream_t s)
 {
     hipLaunchKernelGGL(k_rdf_prep, dim3((std::max(natoms, nbins) + 255) / 256), dim3(256), 0, s, v, chain, nbins, u, counts);
@@ -226,7 +239,9 @@ hipError_t launch_rdf(const DevView& v, int chain, int natoms, int nbins, double
     if (e != hipSuccess || natoms == 0) return e;
     const int rows = (natoms + 255) / 256, steps = (natoms + kRdfJ - 1) / kRdfJ;
     const int gx = std::min(steps, std::max(1, 4096 / rows));
-    hipLaunchKernelGGL(k_rdf, dim3(gx, rows), dim3(256), sizeof(unsigned int) * nbins, s, v, chain, nbins, size_bin, u, counts);
+    const size_t lds = sizeof(unsigned int) * nbins;
+    if (cube) hipLaunchKernelGGL(k_rdf<true>, dim3(gx, rows), dim3(256), lds, s, v, chain, nbins, size_bin, u, counts);
+    else hipLaunchKernelGGL(k_rdf<false>, dim3(gx, rows), dim3(256), lds, s, v, chain, nbins, size_bin, u, counts);
     return hipGetLastError();
 }
 
