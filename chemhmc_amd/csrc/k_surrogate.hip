@@ -36,6 +36,13 @@ __device__ __forceinline__ float dsilu_f(float a)
     return s * (1.0f + a * (1.0f - s));
 }
 
+// a descriptor's Gaussian exp(-t^2 / 2 w^2) at distance t from its centre, as one power of two of one product
+__device__ __forceinline__ float gauss(float t)
+{
+    constexpr float k = (float)(-1.4426950408889634 / (2.0 * (double)kSurrWidth * (double)kSurrWidth));      // log2(e)
+    return __builtin_amdgcn_exp2f(t * t * k);
+}
+
 // --------------------------------------------------------------------------------------------------
 // pair list
 // --------------------------------------------------------------------------------------------------
@@ -43,14 +50,15 @@ __device__ __forceinline__ float dsilu_f(float a)
 // a step and the hits go, by ballot prefix, to an LDS list of staged positions; then, 64 hits at a time and
 // densely, their geometry (dx, dy, dz, neighbour slot) goes to the atom's global list and (r, fc) to LDS, and
 // the descriptors follow with lane = (feature, every second pair).  Bound: VALU issue (402 candidate tests and
-// 32 x 55 Gaussians an atom) and the 16 B a pair written.  N = 32768, rho* = 0.84: 35.6 us; before, the test
+// 32 x 55 Gaussians an atom) and the 16 B a pair written.  N = 32768, rho* = 0.84: 33 us (35.2 with the ends of the
+// list and of the staged atoms tested for every candidate and three products a Gaussian); before, the test
 // loop paid the root, sine and cosine of each hit at 14 % of its lanes and wrote 28 B a pair (38 us), and a
 // second kernel read them back one pair a step (40 us).
 __global__ __launch_bounds__(256) void k_surr_pairs(DevView v, SurrView s, float* __restrict__ G_out)
 {
     constexpr int NT = 256, W = 4;
-    __shared__ float4 sj[kMaxJ];                      // (x, y, z, sorted slot) seen from the i cell's origin
-    __shared__ unsigned short hl[W][kSurrMaxNb];      // staged positions of the wave's hits
+    __shared__ float4 sj[kMaxJ + 64];                 // (x, y, z, sorted slot) seen from the i cell's origin; far entries
+    __shared__ unsigned short hl[W][kSurrMaxNb + 64]; // staged positions of the wave's hits
     __shared__ float2 rf[W][kSurrMaxNb];              // their r and fc
     __shared__ int seg_beg[27], seg_pref[28];
     __shared__ float seg_sh[27][3];
@@ -97,22 +105,24 @@ __global__ __launch_bounds__(256) void k_surr_pairs(DevView v, SurrView s, float
         const float4 q = v.xs[src];
         sj[t] = make_float4(q.x + seg_sh[k][0], q.y + seg_sh[k][1], q.z + seg_sh[k][2], __int_as_float(src));
     }
+    if (tid < 64) sj[nj + tid] = make_float4(kFarShift, kFarShift, kFarShift, 0.f);
     __syncthreads();
-    const float rc2 = C.rc2_f, rc = sqrtf(C.rc2_f);
-    const float mu = mu_k(lane & 31), c2 = 1.0f / (2.0f * kSurrWidth * kSurrWidth);
+    const float rc = sqrtf(C.rc2_f);
+    const unsigned rc2m = (unsigned)__float_as_int(C.rc2_f) - 1u;
+    const float mu = mu_k(lane & 31);
     for (int i = wave; i < ni; i += W) {
         const int slot = ibeg + i;
         const float4 xi = v.xs[slot];
         int count = 0;
         for (int j0 = 0; j0 < nj; j0 += 64) {
-            const int j = j0 + lane;
-            const float4 q = sj[min(j, nj - 1)];
+            const float4 q = sj[j0 + lane];
             const float dx = xi.x - q.x, dy = xi.y - q.y, dz = xi.z - q.z;
             const float r2 = dx * dx + dy * dy + dz * dz;
-            const bool hit = j < nj && r2 < rc2 && r2 > 0.f;
-            const unsigned long long m = __ballot(hit);
-            const int pos = count + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-            if (hit && pos < kSurrMaxNb) hl[wave][pos] = (unsigned short)j;
+            // 0 < r^2 < rc^2 as one compare of the bits less one; hits past the list's capacity go to its spare end
+            const unsigned m2 = (unsigned)__float_as_int(r2) - 1u;
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(m2 < rc2m);
+            const unsigned pos = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+            if (m2 < rc2m) (hl[wave] + min(count, kSurrMaxNb))[pos] = (unsigned short)(j0 + lane);
             count += __popcll(m);
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -134,7 +144,7 @@ __global__ __launch_bounds__(256) void k_surr_pairs(DevView v, SurrView s, float
         for (int k = lane >> 5; k < n; k += 2) {
             const float2 q = rf[wave][k];
             const float t = q.x - mu;
-            acc = __builtin_fmaf(__expf(-t * t * c2), q.y, acc);
+            acc = __builtin_fmaf(gauss(t), q.y, acc);
         }
         acc += __shfl_xor(acc, 32, 64);
         if (lane < 32) G_out[(size_t)slot * kSurrFeat + lane] = acc;
@@ -150,7 +160,7 @@ __global__ __launch_bounds__(256) void k_surr_pairs(DevView v, SurrView s, float
 // first take one pair each (r, fc and fc' from the stored geometry) and leave what the feature loop needs in
 // LDS, from where every lane reads each pair: a global load of one pair for all 32 lanes moves the same 512
 // bytes as 32 different ones, and those loads bound the loops: at N = 32768 the force-matching residual took
-// 135 us and its v 99, now 48 and 23.
+// 135 us and its v 99, now 48 and 22.
 struct SurrPair {
     float4 d;                     // dx, dy, dz, neighbour slot
     float r, fc, dfc, ir;         // distance, cutoff function and its derivative, 1 / r
@@ -182,14 +192,13 @@ struct SurrForcePairs {
 __device__ __forceinline__ float3 surr_force_sum(const SurrForcePairs& st, int row, int n, const float* __restrict__ g,
                                                  float gi, int f, float mu)
 {
-    const float c2 = 1.0f / (2.0f * kSurrWidth * kSurrWidth);
     float fx = 0.f, fy = 0.f, fz = 0.f;
 #pragma unroll 4
     for (int q = 0; q < n; q++) {
         const float4 a = st.a[row][q], u = st.u[row][q];
         const float gj = g[(size_t)__float_as_int(a.w) * kSurrFeat + f];
         const float t = a.x - mu;
-        const float term = (gi + gj) * (__expf(-t * t * c2) * (a.y - t * a.z));
+        const float term = (gi + gj) * (gauss(t) * (a.y - t * a.z));
         fx = __builtin_fmaf(term, u.x, fx);
         fy = __builtin_fmaf(term, u.y, fy);
         fz = __builtin_fmaf(term, u.z, fz);
@@ -835,7 +844,7 @@ __global__ __launch_bounds__(256) void k_surr_fm_v(DevView v, SurrView s, const 
     const int f = threadIdx.x & 31;
     if (a >= v.Ntot) return;
     const ChainDev& C = v.chains[v.atom_chain[__float_as_int(v.xs[a].w)]];
-    const float mu = mu_k(f), c2 = 1.0f / (2.0f * kSurrWidth * kSurrWidth), iw2 = 1.0f / (kSurrWidth * kSurrWidth);
+    const float mu = mu_k(f), iw2 = 1.0f / (kSurrWidth * kSurrWidth);
     const float rc = sqrtf(C.rc2_f);
     const float4 Ri = R[a];
     const int n = s.nb_n[a];
@@ -851,7 +860,7 @@ __global__ __launch_bounds__(256) void k_surr_fm_v(DevView v, SurrView s, const 
     for (int q = 0; q < n; q++) {
         const float4 p = st[row][q];
         const float t = p.x - mu;
-        acc = __builtin_fmaf(__expf(-t * t * c2), p.y - t * p.z, acc);
+        acc = __builtin_fmaf(gauss(t), p.y - t * p.z, acc);
     }
     vout[(size_t)a * kSurrFeat + f] = cw * acc;
 }
