@@ -11,8 +11,8 @@
 // so a chain of a batch evolves exactly as it does alone):
 //   k_lcount  atoms -> list cells (floor(x / lsize), clamped), arrival order into a dense member array
 //             that carries each member's FP32 cell-relative position
-//   k_lscan   only for chains of more than kScanCells cells: one workgroup scans the cell counts and
-//             the others rank each list cell's members by atom id once, for every build workgroup
+//   k_lscan   only for chains of more than kScanCells cells: the first workgroups scan the cell counts, a part
+//             each, and the others rank each list cell's members by atom id once, for every build workgroup
 //             that stages them (k_lscan_chains: the same for batches of chains of kScanChainCells cells
 //             or more, one scan workgroup per chain)
 //   k_lbuild  one workgroup per list cell: (small chains: the counts scanned in LDS) the cell's members
@@ -21,15 +21,16 @@
 //             image shift dd * lsize folded in (the way k_lj stages its j-list), and each own atom's
 //             list of the entries within rc + skin is appended in slot order, as 32-bit entries (slot,
 //             image code) or, in contexts of large lists, 16-bit ones (neighbour segment, rank in that
-//             cell; the cell's segment starts go to ctab).  Rows are then padded past their count to
+//             cell; the cell's segment starts go to ctab).  Each row is padded past its count to
 //             the sweep span with no-op entries (image code kFarCode, or segment kPadSeg)
 // Sweep: 32 slots x LP lanes per workgroup (LP = 4, 8 or 16, tuned); each lane reads its first kBatch
 //   entries without a count test (the padding), gathers the neighbours' FP32 coordinates (16-bit
 //   entries: slot = segment start from the slot's LDS segment row + rank), adds the image shift from an
 //   LDS table by code or segment (padding: 1e18 away), walks the rest of the list,
-//   and the partial sums meet in a butterfly.  Three lanes of an atom then kick p in FP64, optionally
-//   drift x in FP64 (identical_particles.cpp:651-673), and lane 0 writes the FP32 coordinates of the
-//   other parity and raises the rebuild request when the atom is beyond skin / 2 from x0.
+//   and the partial sums meet in a butterfly and go through LDS to four lanes an atom.  Three of them then
+//   kick p in FP64, optionally drift x in FP64 (identical_particles.cpp:651-673), and the first writes the
+//   FP32 coordinates of the other parity and raises the rebuild request when the atom is beyond skin / 2
+//   from x0.
 // Energy: FP64 coordinates relative to the rebuild cell origins (rel64 = r0 + wrap(x - x0)), the
 //   potential's r < rc test (identical_particles.cpp:432-435), entries in batches of 4 per lane,
 //   per-tile fixed-order partials.
