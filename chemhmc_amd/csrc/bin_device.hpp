@@ -76,10 +76,10 @@ __device__ inline void scan_counts_block(const DevView& v)
     if (tid == 0) offs[n] = carry;
 }
 
-// cell of a position
-__device__ __forceinline__ int cell_index(const ChainDev& C, const double x3[3])
+// cell of a position, and its grid coordinates b (C: the chain, or the members of it that are used here)
+template <typename Grid>
+__device__ __forceinline__ int cell_index(const Grid& C, const double x3[3], int b[3])
 {
-    int b[3];
 #pragma unroll
     for (int d = 0; d < 3; d++) b[d] = clampi((int)floor(x3[d] / C.sizebin[d]), 0, C.nbin[d] - 1);
     return C.cell_off + b[0] + C.nbin[0] * (b[1] + b[2] * C.nbin[1]);
@@ -89,9 +89,8 @@ __device__ __forceinline__ int cell_index(const ChainDev& C, const double x3[3])
 // there.  One atomic per distinct cell among the wave's active lanes, all issued together (one after another,
 // each waiting for the last, they made the count of 250,047 atoms 23.6 us; with the rest of its loads now 11.6).  The arrival slot
 // only has to be unique within the cell: the placement ranks the cell's entries by key.
-__device__ __forceinline__ void count_atom(const DevView& v, const ChainDev& C, int a, const double x3[3])
+__device__ __forceinline__ void count_atom(const DevView& v, int cell, int a)
 {
-    const int cell = cell_index(C, x3);
     v.cell_of[a] = cell;
     const int lane = threadIdx.x & 63;
     unsigned long long left = __ballot(1);
@@ -109,6 +108,11 @@ __device__ __forceinline__ void count_atom(const DevView& v, const ChainDev& C, 
     int base = 0;
     if (lane == lead) base = atomicAdd(&v.count[cell], size);
     v.slot[a] = __shfl(base, lead, 64) + rank;
+}
+__device__ __forceinline__ void count_atom(const DevView& v, const ChainDev& C, int a, const double x3[3])
+{
+    int b[3];
+    count_atom(v, cell_index(C, x3, b), a);
 }
 
 }  // namespace chmc

@@ -22,26 +22,53 @@
 
 namespace chmc {
 
+// What the binning of one atom needs, read together before the first store: the compiler takes no load of the
+// chain's constants ahead of a store, so that each dimension waited for its own loads after the one before it (an
+// FP64 leapfrog step of N = 512 11.9 us, then 11.2; of 2,744 21.2, then 18.5)
+struct BinAtom {
+    double x[3], p[3], L[3], sizebin[3], coeff_x;
+    int nbin[3], cell_off;
+};
+__device__ __forceinline__ BinAtom load_atom(const DevView& v, const ChainDev& C, int a, int do_drift)
+{
+    BinAtom b;
+    const int N = v.Ntot;
+    b.coeff_x = C.coeff_x;                             // compute_coeff_position, identical_particles.cpp:646-648
+    b.cell_off = C.cell_off;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        b.x[d] = v.x[d * N + a];
+        b.p[d] = do_drift ? v.p[d * N + a] : 0.0;
+        b.L[d] = C.L[d];
+        b.sizebin[d] = C.sizebin[d];
+        b.nbin[d] = C.nbin[d];
+    }
+    return b;
+}
+// the drifted position in dimension d (written back), or the position itself
+__device__ __forceinline__ double drift_dim(const DevView& v, const BinAtom& b, int a, int d, double drift_dt, int do_drift)
+{
+    double xv = b.x[d];
+    if (do_drift) {
+        xv += drift_dt * b.coeff_x * b.p[d];
+        xv = lp_round(xv, v.lp_scale);
+        xv = wrap_box(xv, b.L[d]);
+        v.x[d * v.Ntot + a] = xv;
+    }
+    return xv;
+}
+
 __global__ __launch_bounds__(256) void k_count(DevView v, double drift_dt, int do_drift)
 {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a < v.Ntot) {
         const ChainDev& C = v.chains[v.atom_chain[a]];
-        const int N = v.Ntot;
-        const double coeff_x = C.coeff_x;              // compute_coeff_position, identical_particles.cpp:646-648
+        const BinAtom b = load_atom(v, C, a, do_drift);
         double x3[3];
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-            double xv = v.x[d * N + a];
-            if (do_drift) {
-                xv += drift_dt * coeff_x * v.p[d * N + a];
-                xv = lp_round(xv, v.lp_scale);
-                xv = wrap_box(xv, C.L[d]);
-                v.x[d * N + a] = xv;
-            }
-            x3[d] = xv;
-        }
-        count_atom(v, C, a, x3);
+        for (int d = 0; d < 3; d++) x3[d] = drift_dim(v, b, a, d, drift_dt, do_drift);
+        int g[3];
+        count_atom(v, cell_index(b, x3, g), a);
     }
 }
 
@@ -124,37 +151,32 @@ __global__ __launch_bounds__(256) void k_cell_rank(DevView v)
 // The whole binning of a context of at most kBinSmall atoms and cells in one workgroup: counts, their scan and
 // the sort keys stay in LDS, each thread keeps its (up to three) atoms.  Four launches of a few microseconds of
 // latency each otherwise: N = 512, FP64 leapfrog, count + scan + placement took 21 us an evaluation, now
-// 5.7.  Bound: latency (three global round trips, six barriers), and one CU's instructions from about 2000 atoms
-// on: an FP64 leapfrog step of 2,744 atoms takes 21.6 us with it and 22.4 without, of 4,096 29.7 and 25.4.
-__global__ __launch_bounds__(1024) void k_bin_small(DevView v, double drift_dt, int do_drift, int atom_id_order)
+// 4.9.  Bound: latency (three global round trips, six barriers), and one CU's instructions from about 2000 atoms
+// on: an FP64 leapfrog step of 2,744 atoms takes 18.5 us with it and 22.4 without, of 4,096 29.7 (before the loads
+// were brought together) and 24.1.  512 threads where an atom each is enough: 11.2 -> 10.9 us a step of N = 512.
+template <int T, int PT>
+__global__ __launch_bounds__(T) void k_bin_small(DevView v, double drift_dt, int do_drift, int atom_id_order)
 {
-    constexpr int T = 1024, PT = kBinSmall / T;
-    __shared__ int cnt[kBinSmall], key[kBinSmall], wsum[16];
+    constexpr int kMax = T * PT;
+    __shared__ int cnt[kMax], key[kMax], wsum[T / 64];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int N = v.Ntot, nc = v.Ctot;
 #pragma unroll
     for (int k = 0; k < PT; k++) cnt[k * T + tid] = 0;
-    double x3[PT][3];
-    int cell[PT], slot[PT], mykey[PT], chain[PT];
+    double x3[PT][3], o3[PT][3];
+    int cell[PT], slot[PT], mykey[PT];
 #pragma unroll
     for (int k = 0; k < PT; k++) {
         const int a = k * T + tid;
         if (a >= N) continue;
-        chain[k] = v.atom_chain[a];
+        const BinAtom b = load_atom(v, v.chains[v.atom_chain[a]], a, do_drift);
         mykey[k] = atom_id_order ? a : v.invperm[a];
-        const ChainDev& C = v.chains[chain[k]];
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-            double xv = v.x[d * N + a];
-            if (do_drift) {
-                xv += drift_dt * C.coeff_x * v.p[d * N + a];
-                xv = lp_round(xv, v.lp_scale);
-                xv = wrap_box(xv, C.L[d]);
-                v.x[d * N + a] = xv;
-            }
-            x3[k][d] = xv;
-        }
-        cell[k] = cell_index(C, x3[k]);
+        for (int d = 0; d < 3; d++) x3[k][d] = drift_dim(v, b, a, d, drift_dt, do_drift);
+        int g[3];
+        cell[k] = cell_index(b, x3[k], g);
+#pragma unroll
+        for (int d = 0; d < 3; d++) o3[k][d] = g[d] * b.sizebin[d];       // cell_origin
     }
     __syncthreads();
 #pragma unroll
@@ -186,7 +208,7 @@ __global__ __launch_bounds__(1024) void k_bin_small(DevView v, double drift_dt, 
         if (c <= nc) offs[c] = run;            // cells from nc on are empty: the end offset is N
         run += c4[k];
     }
-    if (tid == 0 && nc == kBinSmall) offs[nc] = N;
+    if (tid == 0 && nc == kMax) offs[nc] = N;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < PT; k++)
@@ -197,14 +219,11 @@ __global__ __launch_bounds__(1024) void k_bin_small(DevView v, double drift_dt, 
     for (int k = 0; k < PT; k++) {
         const int a = k * T + tid;
         if (a >= N) continue;
-        const ChainDev& C = v.chains[chain[k]];
-        double o[3];
-        cell_origin(C, cell[k], o);
-        const int beg = cnt[cell[k]], end = cell[k] + 1 < kBinSmall ? cnt[cell[k] + 1] : N;
+        const int beg = cnt[cell[k]], end = cell[k] + 1 < kMax ? cnt[cell[k] + 1] : N;
         int rank = 0;
 #pragma unroll 4
         for (int q = beg; q < end; q++) rank += key[q] < mykey[k] ? 1 : 0;
-        place_atom(v, perm_n, beg + rank, a, x3[k], o);
+        place_atom(v, perm_n, beg + rank, a, x3[k], o3[k]);
     }
 }
 
@@ -242,7 +261,9 @@ hipError_t launch_place(const DevView& v, bool atom_id_order, hipStream_t s)
 
 hipError_t launch_bin_small(const DevView& v, double drift_dt, bool atom_id_order, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_bin_small, dim3(1), dim3(1024), 0, s, v, drift_dt, drift_dt != 0.0 ? 1 : 0, atom_id_order ? 1 : 0);
+    const int drift = drift_dt != 0.0 ? 1 : 0, order = atom_id_order ? 1 : 0;
+    if (v.Ntot <= 512 && v.Ctot <= 512) hipLaunchKernelGGL((k_bin_small<512, 1>), dim3(1), dim3(512), 0, s, v, drift_dt, drift, order);
+    else hipLaunchKernelGGL((k_bin_small<1024, kBinSmall / 1024>), dim3(1), dim3(1024), 0, s, v, drift_dt, drift, order);
     return hipGetLastError();
 }
 

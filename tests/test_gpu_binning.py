@@ -15,11 +15,13 @@ def _check(e, orc, x, L, prev, chain=0):
     return perm
 
 
-# one atom, one cell, the last sizes of one workgroup (3072 atoms, 3072 cells) and the first beyond in either
+# one atom, one cell, the last sizes of one workgroup (3072 atoms, 3072 cells; of 512 threads: 512 and 512) and the
+# first beyond in either
 @pytest.mark.parametrize("N,L,order", [
     (1, 6.0, False), (7, 2.6, False), (1023, 11.0, False), (1025, (8.0, 13.0, 40.0), False), (4096, 40.0, False),
     (4096, 17.0, True), (4095, 17.0, False), (4097, 17.0, False), (3000, 43.0, False), (3000, 43.0, True),
-    (3072, (40.0, 40.0, 30.0), False), (3073, 17.0, True), (2000, (40.0, 40.0, 32.5), False)])
+    (3072, (40.0, 40.0, 30.0), False), (3073, 17.0, True), (2000, (40.0, 40.0, 32.5), False),
+    (512, 20.0, False), (513, 20.0, True), (300, (20.0, 20.0, 22.5), False)])
 def test_binning_sizes(chmc, orc, N, L, order):
     box = np.broadcast_to(np.asarray(L, float), (3,)).copy()
     rng = np.random.default_rng(N)
