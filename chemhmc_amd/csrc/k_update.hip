@@ -58,16 +58,16 @@ __global__ __launch_bounds__(256) void k_heatbath(DevView v, uint64_t seed, long
     const ChainDev& C = v.chains[ch];
     const uint64_t traj = traj_explicit >= 0 ? (uint64_t)traj_explicit : (uint64_t)(*v.traj + 1 + (spec ? ch : 0));
     const uint64_t key_chain = spec ? 0 : (uint64_t)ch;
-    const double sd = sqrt(C.mass / C.beta);
+    const double mass = C.mass, sd = sqrt(mass / C.beta);
     const double twopi = 6.283185307179586;
-    const int N = v.Ntot;
+    const int N = v.Ntot, atom_off = C.atom_off;
     double s = 0.0;
     const int* lperm = slots ? list_buf(v, *list_cur(v, ch)).lperm : nullptr;
     double* pout = slots ? v.pl : v.p;
-    if (slots && ck.begin == C.atom_off && threadIdx.x == 0) *list_pord(v, ch) = -1;   // pl in the current order
+    if (slots && ck.begin == atom_off && threadIdx.x == 0) *list_pord(v, ch) = -1;     // pl in the current order
     for (int i = ck.begin + (int)threadIdx.x; i < ck.end; i += 256) {
         const int a = slots ? lperm[i] : i;       // i: the atom, or the slot of atom a
-        const u64x4 r = philox4x64_10((uint64_t)(a - C.atom_off), traj, key_chain, 0, seed, kKeyHeatbath);
+        const u64x4 r = philox4x64_10((uint64_t)(a - atom_off), traj, key_chain, 0, seed, kKeyHeatbath);
         const double r0 = sqrt(-2.0 * log(u01_oo(r.v[0])));
         const double a0 = twopi * u01_co(r.v[1]);
         const double r1 = sqrt(-2.0 * log(u01_oo(r.v[2])));
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(256) void k_heatbath(DevView v, uint64_t seed, long
         pout[i] = px;
         pout[N + i] = py;
         pout[2 * N + i] = pz;
-        s += (px * px + py * py + pz * pz) / (2 * C.mass);
+        s += (px * px + py * py + pz * pz) / (2 * mass);
         if (count) {
             const double x3[3] = { v.x[a], v.x[N + a], v.x[2 * N + a] };
             count_atom(v, C, a, x3);
@@ -88,20 +88,49 @@ __global__ __launch_bounds__(256) void k_heatbath(DevView v, uint64_t seed, long
 
 // per-chain sums (one 256-thread workgroup per chain) of the LJ sweep's per-cell partials and/or the
 // per-chunk kinetic partials
-__device__ void chain_sums(const DevView& v, int ch, int what)
+// K sums over the 256 threads, each as block_sum_256 forms it (in thread 0), behind one barrier; once a kernel
+template <int K>
+__device__ __forceinline__ void block_sums_256(double (&s)[K])
+{
+    __shared__ double wpart[K][4];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        s[k] = group_sum<16>(s[k]);
+        s[k] += __shfl_xor(s[k], 16, 64);
+        s[k] += __shfl_xor(s[k], 32, 64);
+        if ((threadIdx.x & 63) == 0) wpart[k][threadIdx.x >> 6] = s[k];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < K; k++) s[k] = ((wpart[k][0] + wpart[k][1]) + wpart[k][2]) + wpart[k][3];
+}
+
+// The sums of a chain, to red and, in thread 0, to out[RED_NSLOT] (those that `what` does not form are read there
+// too).  All loads come before the first store and the five sums share a barrier: one after the other, with thread 0
+// reading back what it had written, the decision took 4.6 us at N = 512 and 26 at N = 1,048,576; now 3.7 and 24.
+__device__ void chain_sums(const DevView& v, int ch, int what, double out[RED_NSLOT])
 {
     const ChainDev& C = v.chains[ch];
     double* red = &v.red[ch * RED_NSLOT];
-    if (what & (SUM_CELLS | SUM_TILES)) {
+    const double eps = C.eps;
+#pragma unroll
+    for (int k = 0; k < RED_NSLOT; k++) out[k] = red[k];
+    double s[5] = { 0.0, 0.0, 0.0, 0.0, 0.0 };           // energy, virial, pairs, kinetic; kinetic of the chunks
+    const bool parts = (what & (SUM_CELLS | SUM_TILES)) != 0, chunks = (what & (SUM_CHUNKS_KI | SUM_CHUNKS_K)) != 0;
+    if (chunks) {
+#pragma unroll 8
+        for (int k = threadIdx.x; k < C.nchunks; k += 256) s[4] += v.chunk_part[C.chunk_first + k];
+    }
+    if (parts) {
         const bool cells = (what & SUM_CELLS) != 0;
         const double4* part = reinterpret_cast<const double4*>(cells ? v.cell_part + 4 * (size_t)C.cell_off
                                                                      : v.tile_part + 4 * (size_t)C.tile_first);
         const int n = cells ? C.ncells : C.ntiles;
         // a thread adds partials threadIdx, threadIdx + 256, ... in order, 16 of them loaded together (one
         // at a time the sum was a chain of load latencies: 16.4 us over 19,683 cells, 55 us with the decision over
-        // the 32,768 tiles of N = 1,048,576; now 9.7 and 25 us)
+        // the 32,768 tiles of N = 1,048,576; then 9.7 and 25 us)
         constexpr int U = 16;
-        double su = 0.0, sw = 0.0, sn = 0.0, sk = 0.0;
         for (int q0 = threadIdx.x; q0 < n; q0 += 256 * U) {
             double4 p[U];
 #pragma unroll
@@ -109,38 +138,34 @@ __device__ void chain_sums(const DevView& v, int ch, int what)
 #pragma unroll
             for (int u = 0; u < U; u++)
                 if (q0 + 256 * u < n) {
-                    su += p[u].x;
-                    sw += p[u].y;
-                    sn += p[u].z;
-                    sk += p[u].w;
+                    s[0] += p[u].x;
+                    s[1] += p[u].y;
+                    s[2] += p[u].z;
+                    s[3] += p[u].w;
                 }
         }
-        su = block_sum_256(su);
-        sw = block_sum_256(sw);
-        sn = block_sum_256(sn);
-        sk = block_sum_256(sk);
-        if (threadIdx.x == 0) {
-            red[RED_V] = 2 * C.eps * su;      // identical_particles.cpp:392, pairs counted twice
-            red[RED_W] = 24 * C.eps * sw;     // sum_{i<j} 48 eps (sr12 - sr6/2)
-            red[RED_NINT] = sn;               // ordered interacting pairs
-            red[RED_K] = sk;
-        }
     }
-    if (what & (SUM_CHUNKS_KI | SUM_CHUNKS_K)) {
-        double q = 0.0;
-#pragma unroll 8
-        for (int k = threadIdx.x; k < C.nchunks; k += 256) q += v.chunk_part[C.chunk_first + k];
-        q = block_sum_256(q);
-        if (threadIdx.x == 0) red[(what & SUM_CHUNKS_KI) ? RED_KI : RED_K] = q;
+    block_sums_256(s);
+    if (threadIdx.x != 0) return;
+    if (parts) {
+        out[RED_V] = 2 * eps * s[0];          // identical_particles.cpp:392, pairs counted twice
+        out[RED_W] = 24 * eps * s[1];         // sum_{i<j} 48 eps (sr12 - sr6/2)
+        out[RED_NINT] = s[2];                 // ordered interacting pairs
+        out[RED_K] = s[3];
     }
+    if ((what & SUM_CHUNKS_KI) != 0) out[RED_KI] = s[4];
+    else if (chunks) out[RED_K] = s[4];
+#pragma unroll
+    for (int k = 0; k < RED_NSLOT; k++) red[k] = out[k];
 }
 
 __global__ __launch_bounds__(256) void k_reduce(DevView v, int what)
 {
-    chain_sums(v, blockIdx.x, what);
-    // thread 0 wrote the sums: for the host too
+    double sums[RED_NSLOT];
+    chain_sums(v, blockIdx.x, what, sums);
+    // for the host too
     if ((what & SUM_HOST) && threadIdx.x == 0)
-        for (int k = 0; k < RED_NSLOT; k++) v.host_red[blockIdx.x * RED_NSLOT + k] = v.red[blockIdx.x * RED_NSLOT + k];
+        for (int k = 0; k < RED_NSLOT; k++) v.host_red[blockIdx.x * RED_NSLOT + k] = sums[k];
 }
 
 // One workgroup per chain: V_f, W_f, K_f from the energy sweep's partials, K_i from the heat bath's,
@@ -150,20 +175,21 @@ __global__ __launch_bounds__(256) void k_metropolis(DevView v, const double* __r
                                                     int surr, int what)
 {
     const int ch = blockIdx.x;
-    chain_sums(v, ch, what | SUM_CHUNKS_KI);
-    if (threadIdx.x != 0) return;
     const int i = *v.traj + 1;                 // 1-based index of this trajectory (first_traj = istart + 1)
     const ChainDev& C = v.chains[ch];
+    const double beta = C.beta;
     ChainState st = v.state[ch];
-    const double* r = &v.red[ch * RED_NSLOT];
+    // uniforms are consumed in order by the post-thermalisation trajectories of this run
+    const double u = i < therm ? 0.0 : uniforms[(size_t)ch * ustride + (i - ufirst)];
+    double r[RED_NSLOT];
+    chain_sums(v, ch, what | SUM_CHUNKS_KI, r);
+    if (threadIdx.x != 0) return;
     const double Ki = r[RED_KI], Kf = r[RED_K], Vf = r[RED_V], Wf = r[RED_W];
-    const double dh = C.beta * (Kf + Vf - Ki - st.Vi);
+    const double dh = beta * (Kf + Vf - Ki - st.Vi);
     int acc;
     if (i < therm) {
         acc = 1;
     } else {
-        // uniforms are consumed in order by the post-thermalisation trajectories of this run
-        const double u = uniforms[(size_t)ch * ustride + (i - ufirst)];
         acc = (u < exp(-dh)) ? 1 : 0;
         st.nacc += acc;
     }
