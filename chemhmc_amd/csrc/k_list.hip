@@ -71,9 +71,10 @@ __global__ __launch_bounds__(256) void k_lcount(DevView v, int q, int cb)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
+    const bool any = *req_any(v, q) != 0;                // read before the stores, so through the scalar cache
     int* __restrict__ prev = v.lcount + (size_t)(cb ^ 1) * v.Cl;
     for (int c = s; c < v.Cl; c += gridDim.x * blockDim.x) prev[c] = 0;
-    if (*req_any(v, q) == 0) return;
+    if (!any) return;
     // lanes of slots in requesting chains take part; whole waves stay together for the ballots below
     const int ch = s < v.Ntot ? v.atom_chain[s] : 0;     // a chain's slots span the same range as its atoms
     const bool part = s < v.Ntot && *req(v, q, ch) != 0;
