@@ -419,6 +419,7 @@ static long long first_outside(const double* xyz, int n, const double L[3])
 }
 
 static int flush_drift(chmc_ctx* c);
+static int stale_bins(chmc_ctx* c);
 
 extern "C" int chmc_set_positions(chmc_ctx* c, int chain, const double* xyz)
 {
@@ -430,8 +431,7 @@ extern "C" int chmc_set_positions(chmc_ctx* c, int chain, const double* xyz)
     if (out >= 0)
         return fail(c, CHMC_E_ARG, "particle " + std::to_string(out / 3) + " outside the box in dimension " + std::to_string(out % 3));
     int rc = flush_drift(c);
-    if (rc) return rc;
-    c->bin_state = 2;
+    if (rc || (rc = stale_bins(c))) return rc;
     c->have_bins = false;
     c->force_kind = 0;
     return put_soa(c, c->v.x, chain, xyz);
@@ -501,11 +501,15 @@ static bool id_order(const chmc_ctx* c) { return (c->flags & CHMC_ORDER_ATOM_ID)
 
 static int ensure_bins(chmc_ctx* c);
 
-// a count whose placement is still pending is placed before positions change again, so that every
-// count compares against the cells of a completed placement
-static int settle_bins(chmc_ctx* c)
+// The positions are about to change outside a count: the bins become stale.  A count whose placement is still
+// pending (the drift fused into an FP32 sweep that ends an EULER or RUTH sequence) is dropped: counts add up, so
+// they have to be zero when the next count starts.  The next binning then sorts from the last placement, as the
+// reference's does, which bins in its force and potential calls only.
+static int stale_bins(chmc_ctx* c)
 {
-    return c->bin_state == 1 ? ensure_bins(c) : CHMC_OK;
+    if (c->bin_state == 1) HIPCHK(c, launch_fill_int(c->v.count, 0, c->Ctot, c->stream));
+    c->bin_state = 2;
+    return CHMC_OK;
 }
 
 static int flush_drift(chmc_ctx* c)
@@ -550,9 +554,8 @@ static int do_drift(chmc_ctx* c, double dt)
     c->list_valid = false;             // positions change outside the lists
     int rc = flush_drift(c);
     if (rc) return rc;
-    if ((rc = settle_bins(c))) return rc;
+    if ((rc = stale_bins(c))) return rc;
     c->pending_drift = dt;
-    c->bin_state = 2;
     c->force_kind = 0;
     return CHMC_OK;
 }
@@ -747,9 +750,8 @@ extern "C" int chmc_update_positions(chmc_ctx* c, double dt)
     CHECK_CTX(c);
     int rc = flush_drift(c);
     if (rc) return rc;
-    if ((rc = settle_bins(c))) return rc;
+    if ((rc = stale_bins(c))) return rc;
     HIPCHK(c, launch_drift(c->v, dt, c->stream));
-    c->bin_state = 2;
     c->force_kind = 0;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return CHMC_OK;
@@ -1296,11 +1298,10 @@ extern "C" int chmc_restore_positions(chmc_ctx* c)
     CHECK_CTX(c);
     int rc = flush_drift(c);
     if (rc) return rc;
-    if ((rc = settle_bins(c))) return rc;
+    if ((rc = stale_bins(c))) return rc;
     const bool lists = c->saved_lists && list_md(c) && c->list_ready;
     c->list_valid = lists;             // the saved list buffer is valid for the restored positions
     HIPCHK(c, launch_save_restore(c->v, 1, lists ? c->lpar : -1, c->stream));
-    c->bin_state = 2;
     c->force_kind = 0;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return CHMC_OK;
@@ -2191,6 +2192,7 @@ extern "C" int chmc_surrogate_train_fm(chmc_ctx* c, int nsteps, double w_force, 
     int rc = surr_geometry(c);
     if (!rc) rc = surr_fm_ensure(c);
     if (!rc) rc = flush_drift(c);
+    if (!rc) rc = stale_bins(c);
     if (rc) return rc;
     Mt64 rng(seed);
     const size_t n3 = 3 * (size_t)c->Ntot;

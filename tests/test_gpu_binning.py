@@ -122,3 +122,42 @@ def test_evaluate_potential_with_old_bins(chmc, orc, N, step):
         assert abs(V - Vo) <= 1e-11 * abs(Vo)
         Vn = orc.potential_binning(x, [L] * 3, RC)
         assert abs(e.compute_potential()[0] - Vn) <= 1e-11 * abs(Vn)
+
+
+# An FP32 cell-path EULER or RUTH sequence ends with a drift that has been counted but not placed (contexts beyond
+# one workgroup's binning).  Whatever moves the positions next, the following binning is the stable counting sort
+# of the new positions from the last placement, the one of the last force evaluation.  RUTH's placements between
+# are not reproduced here, so it runs in atom id order, which does not depend on them.
+@pytest.mark.parametrize("N", [700, 4913])
+@pytest.mark.parametrize("scheme,order", [("EULER", False), ("RUTH", True)])
+@pytest.mark.parametrize("then", ["set", "update", "restore", "train", "bin"])
+def test_binning_after_a_counted_drift(chmc, orc, N, scheme, order, then):
+    L = (N / 0.7) ** (1 / 3)
+    rng = np.random.default_rng(N)
+    with chmc.Engine(chmc.Chain(N=N, L=L, cutoff=RC), cell_md=True, atom_id_order=order) as e:
+        if then == "train":
+            par = {k: rng.normal(size=shp) * 0.1 for k, shp in chmc.SURR_LAYOUT}
+            par["scale"] = np.ones(32)
+            e.surrogate_set_params(par)
+            e.surrogate_reserve_configs(1)
+            e.init_lattice(9, 0.1)
+            e.surrogate_collect_config()
+        e.init_lattice(5, 0.1)
+        e.set_momenta(rng.normal(size=(N, 3)))
+        e.save_positions()
+        prev = None if order else orc.binning(e.positions(), [L] * 3, RC)[0]
+        e.integrate(getattr(chmc, scheme), 0.02, 1)
+        if then == "set":
+            e.set_positions(rng.uniform(0, 1, (N, 3)) * L)
+        elif then == "update":
+            e.update_positions(0.9)
+        elif then == "restore":
+            e.restore_positions()
+        elif then == "train":
+            e.surrogate_train_fm(1, 0.1, 1e-6)
+        if then != "train":                    # the training pass has binned already
+            e.bin()
+        prev = _check(e, orc, e.positions(), [L] * 3, prev)
+        e.update_positions(0.3)
+        e.bin()
+        _check(e, orc, e.positions(), [L] * 3, None if order else prev)
