@@ -674,12 +674,9 @@ extern "C" int chmc_evaluate_potential(chmc_ctx* c, double* V)
     if (!c || !V) return CHMC_E_ARG;
     int rc = flush_drift(c);
     if (rc) return rc;
-    if (!c->have_bins || c->bin_state == 1) {
-        // evaluate_potential uses the bins as they are (identical_particles.cpp:387-393): positions moved
-        // since the last binning keep their old cells; a binning must exist at all
-        rc = ensure_bins(c);
-        if (rc) return rc;
-    }
+    // evaluate_potential uses the bins as they are (identical_particles.cpp:387-393): positions moved since the
+    // last placement keep their old cells, also where a count of the new ones is pending; a binning must exist
+    if (!c->have_bins && (rc = ensure_bins(c))) return rc;
     HIPCHK(c, launch_energy(c->v, c->bin_state != 0, c->stream));
     return reduce_read(c, SUM_CELLS, RED_V, V);
 }

@@ -161,3 +161,24 @@ def test_binning_after_a_counted_drift(chmc, orc, N, scheme, order, then):
         e.update_positions(0.3)
         e.bin()
         _check(e, orc, e.positions(), [L] * 3, None if order else prev)
+
+
+# evaluate_potential after an EULER sequence, whose last drift follows the last force evaluation: the bins are
+# those of that evaluation, in contexts of either size (a count of the drifted positions may be pending)
+@pytest.mark.parametrize("N", [700, 4913])
+def test_evaluate_potential_after_a_counted_drift(chmc, orc, N):
+    L = (N / 0.7) ** (1 / 3)
+    with chmc.Engine(chmc.Chain(N=N, L=L, cutoff=RC, sigma=0.3), cell_md=True) as e:
+        e.init_lattice(5, 0.05)
+        bins = orc.binning(e.positions(), [L] * 3, RC)
+        e.set_momenta(np.random.default_rng(N).normal(size=(N, 3)))
+        e.integrate(chmc.EULER, 0.2, 1)
+        x = e.positions()
+        V = e.evaluate_potential()[0]
+        Vo = orc.potential_binning(x, [L] * 3, RC, sigma=0.3, bins=bins)
+        Vn = orc.potential_binning(x, [L] * 3, RC, sigma=0.3)
+        assert abs(Vo - Vn) > 1e-7 * abs(Vn)               # the two binnings differ here
+        assert abs(V - Vo) <= 1e-11 * abs(Vo)
+        assert abs(e.compute_potential()[0] - Vn) <= 1e-11 * abs(Vn)
+        e.bin()
+        _check(e, orc, x, [L] * 3, bins[0])
