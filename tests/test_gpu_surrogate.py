@@ -360,3 +360,23 @@ def test_training_checkpoint_resumes_bitwise(chmc, osur):
     assert np.array_equal(c.surrogate_params(), a.surrogate_params())
     for e in (a, b, c):
         e.close()
+
+
+def _best(f, n=20, reps=10):
+    f()
+    best = 1e9
+    for _ in range(reps):
+        t0 = time.perf_counter()
+        for _ in range(n):
+            f()
+        best = min(best, (time.perf_counter() - t0) / n)
+    return best
+
+
+def test_features_of_small_chains_cross_whole(chmc, osur):
+    # G and g are two transfers of 64 KB; positions one of 12 KB.  A transfer is a launch and a wait; in parts of
+    # 16 KB the features took five times the positions' time, whole they take 2.2 times
+    with _engine(chmc, burn=0) as e:
+        e.surrogate_set_params(chmc.pack_surrogate(_params(osur, 1)))
+        e.surrogate_eval()
+        assert _best(e.surrogate_features) <= 3.5 * _best(e.positions)
