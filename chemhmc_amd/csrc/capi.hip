@@ -1942,21 +1942,26 @@ extern "C" int chmc_surrogate_eval(chmc_ctx* c, double* energy, int store_force)
     }
     if (store_force) c->force_kind = 1;
     if (energy) {
-        for (int k = 0; k < c->nchains; k++) {
-            const ChainDev& cd = c->hchains[k];
-            double sum = 0.0;                                   // in the order of the chain's sorted slots
-            const int rc2 = staged_get(c, (size_t)cd.natoms, sizeof(float),
-                                       [&](size_t r0, size_t n, char* buf) {
-                                           return launch_copy_words(c->se + cd.atom_off + r0, (int)n,
-                                                                    reinterpret_cast<float*>(buf), c->stream);
-                                       },
-                                       [&](const char* buf, size_t, size_t n) {
-                                           const float* e = reinterpret_cast<const float*>(buf);
-                                           for (size_t i = 0; i < n; i++) sum += e[i];
-                                       });
-            if (rc2) return rc2;
-            energy[k] = sum;
-        }
+        // per-chain sums in the order of the chain's sorted slots, all chains in one transfer (one each: 256
+        // launches and waits, a call of 3.5 ms for 256 chains of 512 atoms; now 0.35 ms)
+        std::fill(energy, energy + c->nchains, 0.0);
+        int k = 0;
+        rc = staged_get(c, (size_t)c->Ntot, sizeof(float),
+                        [&](size_t r0, size_t n, char* buf) {
+                            return launch_copy_words(c->se + r0, (int)n, reinterpret_cast<float*>(buf), c->stream);
+                        },
+                        [&](const char* buf, size_t r0, size_t n) {
+                            const float* e = reinterpret_cast<const float*>(buf);
+                            for (size_t r = r0; r < r0 + n; k++) {
+                                const ChainDev& cd = c->hchains[k];
+                                const size_t end = std::min(r0 + n, (size_t)cd.atom_off + cd.natoms);
+                                double sum = energy[k];
+                                for (; r < end; r++) sum += e[r - r0];
+                                energy[k] = sum;
+                                if (end < (size_t)cd.atom_off + cd.natoms) return;     // goes on in the next part
+                            }
+                        });
+        if (rc) return rc;
     }
     return CHMC_OK;
 }

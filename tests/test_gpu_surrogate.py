@@ -380,3 +380,34 @@ def test_features_of_small_chains_cross_whole(chmc, osur):
         e.surrogate_set_params(chmc.pack_surrogate(_params(osur, 1)))
         e.surrogate_eval()
         assert _best(e.surrogate_features) <= 3.5 * _best(e.positions)
+
+
+def test_energies_of_many_chains(chmc, osur):
+    # 100 chains of 700 atoms, energies in parts of 65,536 that end inside a chain: each the energy of its chain
+    # alone, bit for bit, and all of them in one transfer (a launch and a wait for each chain took seven times the
+    # evaluation of the same atoms in one chain)
+    n, K = 700, 100
+    box = (n / 0.8) ** (1 / 3)
+    par = chmc.pack_surrogate(_params(osur, 1))
+    alone, xs = {}, []
+    for k in range(K):
+        xs.append((np.stack((np.arange(n) % 9, (np.arange(n) // 9) % 9, np.arange(n) // 81), -1) + 0.5
+                   + np.random.default_rng(k).uniform(-0.2, 0.2, (n, 3))) * (box / 9))
+    for k in (0, 1, 92, 93, 94, 99):
+        with chmc.Engine(chmc.Chain(N=n, L=box, cutoff=RC)) as e:
+            e.set_positions(xs[k])
+            e.surrogate_set_params(par)
+            alone[k] = e.surrogate_eval()[0]
+    with chmc.Engine([chmc.Chain(N=n, L=box, cutoff=RC)] * K) as e:
+        for k in range(K):
+            e.set_positions(xs[k], k)
+        e.surrogate_set_params(par)
+        E = e.surrogate_eval()
+        t_many = _best(e.surrogate_eval)
+    for k, v in alone.items():
+        assert E[k] == v, k
+    with chmc.Engine(chmc.Chain(N=n * K, L=(n * K / 0.8) ** (1 / 3), cutoff=RC)) as e:
+        e.init_lattice(3, 0.1)
+        e.surrogate_set_params(par)
+        t_one = _best(e.surrogate_eval)
+    assert t_many <= 2.5 * t_one, (t_many, t_one)
