@@ -10,13 +10,16 @@
 //   k_scan           : one workgroup scans the counts into the next offsets (and clears them)
 //   k_scatter        : atom -> (cell offset + arrival slot), with its sort key (its previous sorted slot, or
 //                      its id for in-cell order by atom id)
-//   k_cell_rank      : 16 lanes per cell rank the cell's entries by key -> the stable order
+//   k_cell_rank      : 16 lanes per cell, or for a cell of many atoms a workgroup, rank its entries by key -> the
+//                      stable order
 //   k_bin_small      : all of it in one workgroup's LDS for small contexts
 // The placement writes the next perm/offs buffers, invperm and the sorted coordinates (FP64, and FP32 relative
 // to the cell); the
 // host then flips the parity argument that selects the current buffers.
 #include "chmc_internal.hpp"
 #include "bin_device.hpp"
+
+#include <climits>
 
 #pragma clang fp contract(off)   // drift and cell index must match the FP64 oracle bit for bit
 
@@ -123,28 +126,161 @@ __device__ __forceinline__ void place_atom(const DevView& v, int* perm_n, int po
     v.xs[pos] = make_float4((float)(x3[0] - o[0]), (float)(x3[1] - o[1]), (float)(x3[2] - o[2]), __int_as_float(atom));
 }
 
-// 16 lanes per cell, each entry's position is its rank among the cell's (unique) keys
-__global__ __launch_bounds__(256) void k_cell_rank(DevView v)
+// Ranks of a cell's n entries by a whole workgroup of 256 threads, where 16 lanes that compare every pair would
+// take long (n^2 / 16 loads a lane: a binning of 100,000 atoms in 125 cells 1.3 ms, in 27 cells 19 ms, 5,000
+// atoms of which 2,900 share a cell 8.4 ms; this way 33, 54 and 42 us, the launches of a sparse binning being 31).
+// Up to kRankTile entries, the pairwise count from LDS, n^2 / 256 compares a thread; or a bit for each key in a
+// window of kRankWindow keys, set, counted by prefix, the rank of an entry the bits below its own: linear in n and in
+// the range of keys (the previous slots of a cell's atoms are near each other, so that one or two windows hold them;
+// atom ids range over Ntot).  A window costs about the pairwise count of 362 entries (six barriers, 16 KB of LDS
+// written and read).
+constexpr int kRankWindow = 65536, kRankTile = 4096;
+__device__ __forceinline__ void rank_dense(const DevView& v, int* perm_n, int beg, int n, const double o[3], int (&lds)[kRankTile],
+                                           int (&part)[8])
 {
-    const int c = blockIdx.x * 16 + (threadIdx.x >> 4);
-    const int sub = threadIdx.x & 15;
-    if (c >= v.Ctot) return;
+    const int N = v.Ntot, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    auto place = [&](int e, int rank) {
+        const int atom = v.satom[beg + e];
+        const double x3[3] = { v.x[atom], v.x[N + atom], v.x[2 * N + atom] };
+        place_atom(v, perm_n, beg + rank, atom, x3, o);
+    };
+    int lo = INT_MAX, hi = 0;
+#pragma unroll 8
+    for (int e = tid; e < n; e += 256) {
+        const int k = v.skey[beg + e];
+        lo = min(lo, k);
+        hi = max(hi, k);
+    }
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+        lo = min(lo, __shfl_xor(lo, m, 64));
+        hi = max(hi, __shfl_xor(hi, m, 64));
+    }
+    __syncthreads();                                       // lds and part free
+    if (lane == 0) {
+        part[wid] = lo;
+        part[4 + wid] = hi;
+    }
+    __syncthreads();
+    lo = min(min(part[0], part[1]), min(part[2], part[3]));
+    hi = max(max(part[4], part[5]), max(part[6], part[7]));
+    const int windows = (hi - lo) / kRankWindow + 1;
+    if (n <= kRankTile && n * n / 131072 < windows) {
+        for (int t = tid; t < (n + 3) / 4 * 4; t += 256) lds[t] = t < n ? v.skey[beg + t] : INT_MAX;
+        __syncthreads();
+        for (int e = tid; e < n; e += 256) {
+            const int key = lds[e];
+            int rank = 0;
+            for (int q = 0; q < n; q += 4) {
+                const int4 k4 = *reinterpret_cast<const int4*>(&lds[q]);
+                rank += (k4.x < key ? 1 : 0) + (k4.y < key ? 1 : 0) + (k4.z < key ? 1 : 0) + (k4.w < key ? 1 : 0);
+            }
+            place(e, rank);
+        }
+        return;
+    }
+    static_assert(kRankWindow / 32 == 8 * 256 && kRankTile >= kRankWindow / 16, "8 words a thread");
+    unsigned* bits = reinterpret_cast<unsigned*>(lds);     // the bits, then for each word the ranks before it
+    int* pre = lds + kRankWindow / 32;
+    int before = 0;
+    for (int w = 0; w < windows; w++) {
+        const int base = lo + w * kRankWindow;
+        __syncthreads();                                   // lds and part free
+#pragma unroll
+        for (int u = 0; u < 8; u++) bits[u * 256 + tid] = 0u;
+        __syncthreads();
+#pragma unroll 8
+        for (int e = tid; e < n; e += 256) {
+            const unsigned k = (unsigned)(v.skey[beg + e] - base);
+            if (k < (unsigned)kRankWindow) atomicOr(&bits[k >> 5], 1u << (k & 31u));
+        }
+        __syncthreads();
+        int s = 0, c8[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            c8[u] = s;
+            s += __popc(bits[8 * tid + u]);
+        }
+        int incl = s;
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) {
+            const int t = __shfl_up(incl, m, 64);
+            if (lane >= m) incl += t;
+        }
+        if (lane == 63) part[wid] = incl;
+        __syncthreads();
+        int run = before + incl - s;
+        for (int k = 0; k < wid; k++) run += part[k];
+#pragma unroll
+        for (int u = 0; u < 8; u++) pre[8 * tid + u] = run + c8[u];
+        before += part[0] + part[1] + part[2] + part[3];
+        __syncthreads();
+        // two entries a thread together: the loads of the second ahead of the first one's stores
+        constexpr int U = 2;
+        for (int e0 = tid; e0 < n; e0 += 256 * U) {
+            unsigned k[U];
+            int atom[U];
+            double x[U][3];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int e = beg + min(e0 + 256 * u, n - 1);
+                k[u] = (unsigned)(v.skey[e] - base);
+                atom[u] = v.satom[e];
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int d = 0; d < 3; d++) x[u][d] = v.x[(size_t)d * N + atom[u]];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (e0 + 256 * u < n && k[u] < (unsigned)kRankWindow)
+                    place_atom(v, perm_n, beg + pre[k[u] >> 5] + __popc(bits[k[u] >> 5] & ((1u << (k[u] & 31u)) - 1u)), atom[u], x[u], o);
+        }
+    }
+}
+
+// 16 lanes per cell, each entry's position is its rank among the cell's (unique) keys; cells of more than
+// kDenseCell atoms by the whole workgroup (rank_dense).  A workgroup has 16 cells, or PER = 1 in contexts of
+// kDenseMean atoms a cell and more, whose dense cells would otherwise wait for each other.
+constexpr int kDenseCell = 64, kDenseMean = 32;
+template <int PER>
+__global__ __launch_bounds__(256, 8) void k_cell_rank(DevView v)
+{
+    __shared__ alignas(16) int lds[kRankTile];
+    __shared__ int part[8];
+    const int c = blockIdx.x * PER + (PER == 1 ? 0 : threadIdx.x >> 4);
+    const int sub = PER == 1 ? threadIdx.x : threadIdx.x & 15;
     const int N = v.Ntot;
     const int* offs = offs_next(v);
     int* perm_n = perm_next(v);
-    const int beg = offs[c];
-    const int n = offs[c + 1] - beg;
-    const ChainDev& C = v.chains[v.cell_chain[c]];
-    double o[3];
-    cell_origin(C, c, o);
-    for (int e = sub; e < n; e += 16) {
-        const int key = v.skey[beg + e];
-        const int atom = v.satom[beg + e];
-        const double x3[3] = { v.x[atom], v.x[N + atom], v.x[2 * N + atom] };
-        int rank = 0;
+    bool dense = false;
+    if (c < v.Ctot) {
+        const int beg = offs[c];
+        const int n = offs[c + 1] - beg;
+        dense = n > kDenseCell;
+        const ChainDev& C = v.chains[v.cell_chain[c]];
+        double o[3];
+        cell_origin(C, c, o);
+        for (int e = dense ? n : sub; e < n; e += 256 / PER) {
+            const int key = v.skey[beg + e];
+            const int atom = v.satom[beg + e];
+            const double x3[3] = { v.x[atom], v.x[N + atom], v.x[2 * N + atom] };
+            int rank = 0;
 #pragma unroll 8
-        for (int q = 0; q < n; q++) rank += (v.skey[beg + q] < key) ? 1 : 0;
-        place_atom(v, perm_n, beg + rank, atom, x3, o);
+            for (int q = 0; q < n; q++) rank += (v.skey[beg + q] < key) ? 1 : 0;
+            place_atom(v, perm_n, beg + rank, atom, x3, o);
+        }
+    }
+    if (__syncthreads_or(dense) == 0) return;
+    for (int k = 0; k < PER; k++) {
+        const int c = blockIdx.x * PER + k;
+        if (c >= v.Ctot) break;
+        const int beg = offs[c];
+        const int n = offs[c + 1] - beg;
+        if (n <= kDenseCell) continue;
+        double o[3];
+        cell_origin(v.chains[v.cell_chain[c]], c, o);
+        rank_dense(v, perm_n, beg, n, o, lds, part);
     }
 }
 
@@ -154,12 +290,18 @@ __global__ __launch_bounds__(256) void k_cell_rank(DevView v)
 // 4.9.  Bound: latency (three global round trips, six barriers), and one CU's instructions from about 2000 atoms
 // on: an FP64 leapfrog step of 2,744 atoms takes 18.5 us with it and 22.4 without, of 4,096 29.7 (before the loads
 // were brought together) and 24.1.  512 threads where an atom each is enough: 11.2 -> 10.9 us a step of N = 512.
+// Cells of more than kSmallDense atoms (clustered systems, or those of few cells) follow at the end and rank their
+// keys by a bit for each, in the cell's own part of key[] (16 KB more LDS made a step of 2,744 atoms 1 % longer):
+// 3000 atoms in one cell, pairwise 217 us a binning, now 26.  The test for them costs 0.2 of the 20 us a step of
+// 2,744 atoms takes, and nothing measurable of the 11 us at 512.
+constexpr int kSmallDense = 160;
 template <int T, int PT>
 __global__ __launch_bounds__(T) void k_bin_small(DevView v, double drift_dt, int do_drift, int atom_id_order)
 {
-    constexpr int kMax = T * PT;
+    constexpr int kMax = T * PT, kWords = kMax / 32;
+    static_assert(kWords + kWords / 2 <= kSmallDense, "the bits and their counts before each word, in 16 bits");
     __shared__ int cnt[kMax], key[kMax], wsum[T / 64];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int N = v.Ntot, nc = v.Ctot;
 #pragma unroll
     for (int k = 0; k < PT; k++) cnt[k * T + tid] = 0;
@@ -184,22 +326,26 @@ __global__ __launch_bounds__(T) void k_bin_small(DevView v, double drift_dt, int
         if (k * T + tid < N) slot[k] = atomicAdd(&cnt[cell[k]], 1);
     __syncthreads();
     // exclusive scan of the counts, PT contiguous cells a thread
-    int c4[PT], s = 0;
+    int c4[PT], s = 0, most = 0;
 #pragma unroll
     for (int k = 0; k < PT; k++) {
         c4[k] = cnt[tid * PT + k];
         s += c4[k];
+        most = max(most, c4[k]);
     }
+    const bool dense_wave = __ballot(most > kSmallDense) != 0ull;
     int incl = s;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
         const int t = __shfl_up(incl, o, 64);
         if (lane >= o) incl += t;
     }
-    if (lane == 63) wsum[wid] = incl;
+    if (lane == 63) wsum[wid] = incl | (dense_wave ? 1 << 16 : 0);
     __syncthreads();
+    const int ws = wsum[lane & (T / 64 - 1)];
+    const bool dense = __ballot(ws >> 16 != 0) != 0ull;                // in any wave
     int run = incl - s;
-    for (int w = 0; w < wid; w++) run += wsum[w];
+    for (int w = 0; w < wid; w++) run += __builtin_amdgcn_readlane(ws, w) & 0xffff;
     int* offs = offs_next(v);
 #pragma unroll
     for (int k = 0; k < PT; k++) {
@@ -215,14 +361,60 @@ __global__ __launch_bounds__(T) void k_bin_small(DevView v, double drift_dt, int
         if (k * T + tid < N) key[cnt[cell[k]] + slot[k]] = mykey[k];
     __syncthreads();
     int* perm_n = perm_next(v);
+    auto end_of = [&](int k) { return cell[k] + 1 < kMax ? cnt[cell[k] + 1] : N; };
 #pragma unroll
     for (int k = 0; k < PT; k++) {
         const int a = k * T + tid;
         if (a >= N) continue;
-        const int beg = cnt[cell[k]], end = cell[k] + 1 < kMax ? cnt[cell[k] + 1] : N;
+        const int beg = cnt[cell[k]], end = end_of(k);
+        if (end - beg > kSmallDense) continue;
         int rank = 0;
 #pragma unroll 4
         for (int q = beg; q < end; q++) rank += key[q] < mykey[k] ? 1 : 0;
+        place_atom(v, perm_n, beg + rank, a, x3[k], o3[k]);
+    }
+    if (!dense) return;
+    // f(begin) for every dense cell, by the wave of the thread that scanned it
+    auto dense_cells = [&](auto f) {
+#pragma unroll
+        for (int k = 0; k < PT; k++)
+            for (unsigned long long m = __ballot(c4[k] > kSmallDense); m != 0ull; m &= m - 1ull)
+                f(__shfl(cnt[tid * PT + k], __ffsll((long long)m) - 1, 64));
+    };
+    dense_cells([&](int beg) {
+        for (int w = lane; w < kWords; w += 64) key[beg + w] = 0;
+    });
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PT; k++) {
+        if (k * T + tid >= N) continue;
+        const int beg = cnt[cell[k]];
+        if (end_of(k) - beg > kSmallDense) atomicOr(&key[beg + (mykey[k] >> 5)], (int)(1u << (mykey[k] & 31)));
+    }
+    __syncthreads();
+    dense_cells([&](int beg) {
+        int before = 0;
+        for (int w0 = 0; w0 < kWords; w0 += 64) {
+            const int n = w0 + lane < kWords ? __popc((unsigned)key[beg + w0 + lane]) : 0;
+            int incl = n;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int t = __shfl_up(incl, o, 64);
+                if (lane >= o) incl += t;
+            }
+            if (w0 + lane < kWords) reinterpret_cast<unsigned short*>(key + beg + kWords)[w0 + lane] = (unsigned short)(before + incl - n);
+            before += __shfl(incl, 63, 64);
+        }
+    });
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PT; k++) {
+        const int a = k * T + tid;
+        if (a >= N) continue;
+        const int beg = cnt[cell[k]], w = mykey[k] >> 5;
+        if (end_of(k) - beg <= kSmallDense) continue;
+        const int rank = reinterpret_cast<const unsigned short*>(key + beg + kWords)[w] +
+                         __popc((unsigned)key[beg + w] & ((1u << (mykey[k] & 31)) - 1u));
         place_atom(v, perm_n, beg + rank, a, x3[k], o3[k]);
     }
 }
@@ -255,7 +447,8 @@ hipError_t launch_scan(const DevView& v, hipStream_t s)
 hipError_t launch_place(const DevView& v, bool atom_id_order, hipStream_t s)
 {
     hipLaunchKernelGGL(k_scatter, dim3((v.Ntot + 255) / 256), dim3(256), 0, s, v, atom_id_order ? 1 : 0);
-    hipLaunchKernelGGL(k_cell_rank, dim3((v.Ctot + 15) / 16), dim3(256), 0, s, v);
+    if (v.Ntot / kDenseMean >= v.Ctot) hipLaunchKernelGGL(k_cell_rank<1>, dim3(v.Ctot), dim3(256), 0, s, v);
+    else hipLaunchKernelGGL(k_cell_rank<16>, dim3((v.Ctot + 15) / 16), dim3(256), 0, s, v);
     return hipGetLastError();
 }
 

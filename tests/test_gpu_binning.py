@@ -1,5 +1,7 @@
 """Binning at the edges of its paths (one workgroup up to 3072 atoms and cells, four launches beyond),
 against the FP64 oracle's stable counting sort: bitwise."""
+import time
+
 import numpy as np
 import pytest
 
@@ -182,3 +184,69 @@ def test_evaluate_potential_after_a_counted_drift(chmc, orc, N):
         assert abs(e.compute_potential()[0] - Vn) <= 1e-11 * abs(Vn)
         e.bin()
         _check(e, orc, x, [L] * 3, bins[0])
+
+
+def _dense_case(name):
+    """(positions, box, cut-off) of a system with cells of many atoms"""
+    rng = np.random.default_rng(len(name))
+    N, L, rc, ball = {
+        "one_cell_160": (160, 5.0, 2.6, None), "one_cell_161": (161, 5.0, 2.6, None), "one_cell_512": (512, 5.0, 2.6, None),
+        "eight_cells_512": (512, 5.1, 2.5, None), "one_cell_3072": (3072, 9.0, 5.0, None), "27_cells_3000": (3000, 16.0, 5.3, None),
+        "3000_in_a_corner": (3000, 30.0, 2.5, 6.0),
+        "one_cell_3073": (3073, 9.0, 5.0, None), "27_cells_4096": (4096, 16.0, 5.3, None), "27_cells_8000": (8000, 20.0, 6.6, None),
+        "64_a_cell": (8000, 12.6, 2.5, None), "8_cells_20000": (20000, 29.0, 14.0, None),
+        "droplet": (9000, 45.0, 2.5, 9.0), "corner": (9000, 45.0, 2.5, 4.0),
+        "windows": (140000, 50.0, 10.0, None), "windows_corner": (70000, 80.0, 2.5, 4.0)}[name]
+    x = rng.uniform(0, 1, (N, 3)) * L
+    if ball:                       # two thirds of the atoms close together, in random order of their ids
+        k = rng.permutation(N)[:2 * N // 3]
+        x[k] = rng.uniform(0, ball, (len(k), 3)) + 1.0
+    return x, L, rc
+
+
+# cells of many atoms: of the one-launch binning at the limit of its pairwise ranking (160 atoms a cell), with 8, 27
+# and few dense cells among many; of the four-launch one at its limit (64) with a workgroup a cell and with sixteen,
+# pairwise (up to 362 keys in one window) and by bits in one window and in several
+@pytest.mark.parametrize("name", ["one_cell_160", "one_cell_161", "one_cell_512", "eight_cells_512", "one_cell_3072",
+                                  "27_cells_3000", "3000_in_a_corner", "one_cell_3073", "27_cells_4096", "27_cells_8000",
+                                  "64_a_cell", "8_cells_20000", "droplet", "corner", "windows", "windows_corner"])
+@pytest.mark.parametrize("order", [False, True])
+def test_binning_dense_cells(chmc, orc, name, order):
+    x, L, rc = _dense_case(name)
+    N = len(x)
+    prev = None
+    with chmc.Engine(chmc.Chain(N=N, L=L, cutoff=rc), atom_id_order=order) as e:
+        e.set_momenta(np.random.default_rng(3).normal(size=(N, 3)))
+        for k in range(3):                       # from atom ids, then from the last order, after small and large moves
+            if k == 0:
+                e.set_positions(x)
+            else:
+                e.update_positions(0.1 if k == 1 else 2.0)
+            e.bin()
+            perm, cnt, off = e.bins()
+            po, co, oo = orc.binning(e.positions(), [L] * 3, rc, perm=prev)
+            assert np.array_equal(cnt, co) and np.array_equal(off, oo) and np.array_equal(perm, po), k
+            prev = None if order else perm
+
+
+# the time of a binning does not grow with the square of a cell's atoms: systems in eight cells or in one take 1.1
+# (3000 atoms), 1.5 to 2.8 (20,000) and 2.2 to 7.1 times (100,000, one cell being one workgroup's work) as long as
+# spread out; ranked pairwise they took 9, 200 and 2000 times as long and more
+@pytest.mark.parametrize("N,L,times", [(3000, 30.0, 4), (20000, 60.0, 8), (100000, 110.0, 16)])
+def test_binning_time_of_dense_cells(chmc, N, L, times):
+    rng = np.random.default_rng(N)
+
+    def best(x):
+        with chmc.Engine(chmc.Chain(N=N, L=L, cutoff=RC)) as e:
+            e.set_positions(x)
+            e.bin()
+            t = []
+            for _ in range(30):
+                t0 = time.perf_counter()
+                e.bin()
+                t.append(time.perf_counter() - t0)
+            return min(t)
+
+    spread = best(rng.uniform(0, L, (N, 3)))
+    assert best(rng.uniform(0, 5.0, (N, 3))) <= times * spread
+    assert best(rng.uniform(0, 2.4, (N, 3))) <= times * spread
