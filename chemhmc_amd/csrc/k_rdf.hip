@@ -62,8 +62,8 @@ constexpr int kRdfJ = 32;          // j atoms per step of a workgroup
 // per component, 3 of the sum of squares, halved by the root, and 1 ulp of v_sqrt_f32; in a cube (CUBE) the root
 // is scaled instead of the components: 2 roundings for 2).  A pair whose t is
 // farther than eps from an integer, eps = (nbins + 1) 2^-21 + 2^-31 |L| / size_bin, therefore has the exact
-// bin (int)t; the others (0.05 % at 500 bins) and any NaN are binned in FP64.  Bins from nbins + 1 up are
-// never counted and need no decision.
+// bin (int)t; the others (0.05 % at 500 bins) and any NaN are binned in FP64.  Pairs whose t is beyond nbins + 1 by
+// the fixed-point part of eps (more than a bin where size_bin < 2^-31 |L|) are never counted and need no decision.
 //   Bound: VALU issue, ~20 slots a pair (22 outside a cube).  N = 32768, 500 bins up to L / 2 (5.4e8 pairs): 271 us,
 // against 308 us with the components scaled and the tests repeated as selects, and 1531 us with the FP64 root and
 // division for every pair.
@@ -88,8 +88,9 @@ __global__ __launch_bounds__(256) void k_rdf(DevView v, int chain, int nbins, do
     const float sx = (float)(C.L[0] / 4294967296.0 / size_bin), sy = (float)(C.L[1] / 4294967296.0 / size_bin),
                 sz = (float)(C.L[2] / 4294967296.0 / size_bin);
     const double diag = sqrt(C.L[0] * C.L[0] + C.L[1] * C.L[1] + C.L[2] * C.L[2]);
-    const float half = (float)(0.5 - ((nbins + 1) / 2097152.0 + diag / size_bin / 2147483648.0) - 1e-7);
-    const float edge = (float)(nbins + 1), nb = (float)nbins;
+    const double fixed = diag / size_bin / 2147483648.0;
+    const float half = (float)(0.5 - ((nbins + 1) / 2097152.0 + fixed) - 1e-7);
+    const float edge = (float)((nbins + 1 + fixed) * (1.0 + 1e-6)), nb = (float)nbins;
     auto exact = [&](int j) {
         const int b = rdf_bin_exact(C, xi, yi, zi, v.x[off + j], v.x[(size_t)N + off + j], v.x[2 * (size_t)N + off + j], size_bin);
         if (b < nbins) atomicAdd(&hist[b], 1u);

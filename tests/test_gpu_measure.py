@@ -69,3 +69,21 @@ def test_open_potential_coincident_pair(chmc):
     x = np.zeros((5, 3))
     x[2:] = [[1, 0, 0], [0, 1.2, 0], [0, 0, 1.3]]
     assert np.isnan(chmc.potential_energy_open(x, a=4.0, b=4.0))      # inf - inf, as a / 0 - b / 0
+
+
+# bins far below the fixed-point step of the coordinates (2^-32 L = 2e-9): pairs all over the counted range, the last
+# bins among them, for which the FP32 quotient is off by several bins
+@pytest.mark.parametrize("L,nb,size", [(9.0, 50, 1e-9), ((7.0, 9.0, 11.0), 50, 1e-9), (9.0, 400, 1e-10), (9.0, 3, 5e-11)])
+def test_rdf_counts_bins_below_the_coordinate_step(chmc, L, nb, size):
+    box = np.broadcast_to(np.asarray(L, float), (3,))
+    rng = np.random.default_rng(nb)
+    a = rng.uniform(0.1, 0.9, (400, 3)) * box
+    u = rng.normal(size=(400, 3))
+    u /= np.sqrt((u * u).sum(1))[:, None]
+    x = np.concatenate((a, a + u * (rng.uniform(0, 1.2, 400) * nb * size)[:, None]))
+    want = _rdf_counts(x, box, nb, size)
+    assert want.sum() > 600 and want[-(nb // 20 + 1):].sum() > 0
+    with chmc.Engine(chmc.Chain(N=800, L=tuple(box), cutoff=2.5)) as e:
+        e.set_positions(x)
+        counts, _ = e.rdf(nb, size)
+    assert np.array_equal(counts, want)
