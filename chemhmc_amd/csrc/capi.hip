@@ -1771,10 +1771,10 @@ static hipError_t open_memory(OpenMem* out)
 // upload, sum and read back on the calling thread's stream; part: tile partials, then the result
 static hipError_t open_sum(const double* xyz, int np, int n, double a, double b, double* dx, double* part, double* result)
 {
-    const size_t nt = (size_t)open_potential_tiles(np);
+    const size_t nparts = open_potential_partials(np);
     hipError_t e = hipMemcpyAsync(dx, xyz, sizeof(double) * 3 * (size_t)np, hipMemcpyHostToDevice, hipStreamPerThread);
-    if (e == hipSuccess) e = launch_open_potential(dx, np, n, a, b, part, part + nt * nt, hipStreamPerThread);
-    if (e == hipSuccess) e = hipMemcpyAsync(result, part + nt * nt, sizeof(double), hipMemcpyDeviceToHost, hipStreamPerThread);
+    if (e == hipSuccess) e = launch_open_potential(dx, np, n, a, b, part, part + nparts, hipStreamPerThread);
+    if (e == hipSuccess) e = hipMemcpyAsync(result, part + nparts, sizeof(double), hipMemcpyDeviceToHost, hipStreamPerThread);
     const hipError_t es = hipStreamSynchronize(hipStreamPerThread);
     return e == hipSuccess ? es : e;
 }
@@ -1797,9 +1797,8 @@ extern "C" int chmc_potential_energy_open(const double* xyz, int n_particles, in
             e = open_sum(xyz, np, n, a, b, m.buf, m.buf + 3 * (size_t)kOpenSmall, &r);
         }
     } else {
-        const size_t nt = (size_t)open_potential_tiles(np);
         double* d = nullptr;
-        e = hipMalloc(&d, sizeof(double) * (3 * (size_t)np + nt * nt + 1));
+        e = hipMalloc(&d, sizeof(double) * (3 * (size_t)np + open_potential_partials(np) + 1));
         if (e == hipSuccess) e = open_sum(xyz, np, n, a, b, d, d + 3 * (size_t)np, &r);
         if (d) hipFree(d);
     }

@@ -407,9 +407,11 @@ hipError_t launch_list_energy(const DevView& v, int q, bool rel64, hipStream_t s
 // u: natoms fixed-point coordinates of scratch; counts: nbins, cleared here
 hipError_t launch_rdf(const DevView& v, int chain, int natoms, bool cube, int nbins, double size_bin, uint4* u,
                       unsigned long long* counts, hipStream_t s);
-// the open-boundary sum over n atoms (AoS) in T x T tiles, T = open_potential_tiles(n); partials: T * T doubles
+// the open-boundary sum over n atoms (AoS) in T x T tiles, T = open_potential_tiles(n), one partial each (more than
+// 2^31 of them from 11.9 million atoms on)
 constexpr int kOpenSmall = 16384;
 int open_potential_tiles(int n);
+size_t open_potential_partials(int n);
 hipError_t launch_open_potential(const double* xyz, int n, int nexp, double a, double b, double* partials, double* result,
                                  hipStream_t s);
 hipError_t launch_fill_int(int* p, int value, int n, hipStream_t s);

@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) void k_open_potential(const double* __restrict
     __shared__ double wpart[4];
     const int I = blockIdx.y, J = blockIdx.x;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int pid = I * gridDim.x + J;
+    const size_t pid = (size_t)I * gridDim.x + J;
     if (J < I) {
         if (tid == 0) partials[pid] = 0.0;
         return;
@@ -215,11 +215,11 @@ __global__ __launch_bounds__(256) void k_open_potential(const double* __restrict
 }
 
 // the sum of the tile partials in a fixed order: 1024 strided sums, then a tree
-__global__ __launch_bounds__(1024) void k_open_sum(const double* __restrict__ partials, int count, double* __restrict__ result)
+__global__ __launch_bounds__(1024) void k_open_sum(const double* __restrict__ partials, size_t count, double* __restrict__ result)
 {
     __shared__ double wpart[16];
     double s = 0.0;
-    for (int k = threadIdx.x; k < count; k += 1024) s += partials[k];
+    for (size_t k = threadIdx.x; k < count; k += 1024) s += partials[k];
 #pragma unroll
     for (int m = 1; m < 64; m <<= 1) s += __shfl_xor(s, m, 64);
     if ((threadIdx.x & 63) == 0) wpart[threadIdx.x >> 6] = s;
@@ -252,6 +252,12 @@ int open_potential_tiles(int n)
     return n <= kOpenSmall ? (n + 63) / 64 : (n + 255) / 256;
 }
 
+size_t open_potential_partials(int n)
+{
+    const size_t T = (size_t)open_potential_tiles(n);
+    return T * T;
+}
+
 hipError_t launch_open_potential(const double* xyz, int n, int nexp, double a, double b, double* partials, double* result,
                                  hipStream_t s)
 {
@@ -264,7 +270,7 @@ hipError_t launch_open_potential(const double* xyz, int n, int nexp, double a, d
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(k_open_sum, dim3(1), dim3(1024), 0, s, partials, T * T, result);
+    hipLaunchKernelGGL(k_open_sum, dim3(1), dim3(1024), 0, s, partials, open_potential_partials(n), result);
     return hipGetLastError();
 }
 

@@ -34,3 +34,13 @@ def test_no_device_means_clean_error(chmc):
     else:
         e.close()
         pytest.skip("a GPU is present")
+
+
+def test_open_sum_counts_tiles_in_64_bits(chmc):
+    # one partial per pair of tiles: 2^31 of them from 46,341 tiles of 256 atoms on (11.9 million atoms), where a
+    # 32-bit count is negative.  chmc::open_potential_partials(int) sizes the memory and bounds the sum over it
+    f = getattr(ctypes.CDLL(chmc.LIB_PATH), "_ZN4chmc23open_potential_partialsEi")
+    f.restype, f.argtypes = ctypes.c_size_t, [ctypes.c_int]
+    for n, tiles in ((0, 0), (1, 1), (64, 1), (65, 2), (16384, 256), (16385, 65), (65536, 256), (11_863_041, 46341),
+                     (12_000_000, 46875), (16_777_217, 65537)):
+        assert f(n) == tiles * tiles, n
