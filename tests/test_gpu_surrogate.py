@@ -411,3 +411,34 @@ def test_energies_of_many_chains(chmc, osur):
         e.surrogate_set_params(par)
         t_one = _best(e.surrogate_eval)
     assert t_many <= 2.5 * t_one, (t_many, t_one)
+
+
+# a loss gradient beyond FP32 is an infinity with its sign, as the FP32 products give it, and no NaN: all terms of
+# the W1, b1, W2 and b2 gradients are products of a positive delta with positive inputs
+@pytest.mark.parametrize("w3", [1e25, 1e30])
+def test_fm_gradient_infinities(chmc, osur, w3):
+    with _engine(chmc, burn=0) as e:
+        par = {k: np.full(shp, 0.01) for k, shp in chmc.SURR_LAYOUT}
+        par.update(b1=np.ones(64), b2=np.ones(64), w3=np.full(64, w3), b3=np.zeros(1), shift=np.full(32, -5.0), scale=np.ones(32))
+        e.surrogate_set_params(chmc.pack_surrogate(par))
+        g = chmc.unpack_surrogate(e.surrogate_fm_loss_grad(0.0)[0], trained_only=True)
+        for k in ("W1", "b1", "W2", "b2"):
+            assert np.all(g[k] == np.inf), (k, g[k].reshape(-1)[:4])
+
+
+# deltas that round to infinity in bfloat16 (from 3.3962e38), below the largest float (3.4028e38): 64 units, all alike, with a1 = 1e-6 and
+# a2 = 1, so that D2 = de w3 silu'(1), de = 2 / N (64 w3 bf16(silu(1)) + b3) with w3 a bfloat16 number; the gradient of
+# W2 is N D2 bf16(silu(1e-6))
+def test_fm_gradient_next_to_the_largest_float(chmc, osur):
+    silu, dsilu, h1 = 0.73046875, 0.9276705, 4.991889e-07       # silu(1) in bfloat16, silu'(1), silu(1e-6) in bfloat16
+    D2, w3 = 3.400e38, 2.0 ** 65
+    b3 = D2 / (w3 * dsilu) * N / 2 - 64 * w3 * silu
+    with _engine(chmc, burn=0) as e:
+        par = {k: np.zeros(shp) for k, shp in chmc.SURR_LAYOUT}
+        par.update(b1=np.full(64, 1e-6), b2=np.ones(64), w3=np.full(64, w3), b3=np.full(1, b3), scale=np.ones(32))
+        e.surrogate_set_params(chmc.pack_surrogate(par))
+        g = chmc.unpack_surrogate(e.surrogate_fm_loss_grad(0.0)[0], trained_only=True)
+        de = g["b3"][0] / N
+        assert 3.3963e38 < de * w3 * dsilu < 3.4026e38            # the deltas lie where they should
+        # FP32 activations and sums of 512 terms
+        assert np.allclose(g["W2"], N * D2 * h1, rtol=1e-4, atol=0), g["W2"].reshape(-1)[:4]
