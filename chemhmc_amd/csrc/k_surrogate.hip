@@ -1020,10 +1020,11 @@ __global__ __launch_bounds__(256) void k_surr_grad_fm(SurrView s, const float* _
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const float dl = gam[t][i] * s1[t][i];
-                const float zb1 = d2silu_f(o.a1[t][i]) * t1[t][i] * gam[t][i] + s1[t][i] * ab1[t][i];
+                // the roundings of zb1 and D1 are fixed, whatever the compiler fuses around them
+                const float zb1 = __builtin_fmaf(s1[t][i], ab1[t][i], d2silu_f(o.a1[t][i]) * t1[t][i] * gam[t][i]);
                 const float h2 = (float)(__bf16)silu_f(o.a2[t][i]);
                 dl1[t][i] = valid[i] ? dl : 0.f;
-                D1[t][i] = valid[i] ? de[i] * dl + zb1 : 0.f;
+                D1[t][i] = valid[i] ? __builtin_fmaf(de[i], dl, zb1) : 0.f;
                 D2[t][i] = valid[i] ? de[i] * dl2[t][i] + zb2[t][i] : 0.f;
                 dl2[t][i] = valid[i] ? dl2[t][i] : 0.f;
                 accb1[t] += D1[t][i];
