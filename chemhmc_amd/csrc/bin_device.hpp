@@ -1,6 +1,7 @@
 // Device helpers shared by the kernels that bin atoms (k_bin.hip, and the fused drift + count of the
 // FP32 force sweep and of the heat bath): cell index with the reference's floor(x / sizebin)
-// (particles.hpp:108-113) clamped to the grid, the count phase of one atom and the one-workgroup exclusive scan of the per-cell counts.
+// (particles.hpp:108-113) clamped to the grid, the count phase of one atom and the one-workgroup exclusive scan of
+// the per-cell counts.
 #pragma once
 #include "chmc_internal.hpp"
 
@@ -87,8 +88,8 @@ __device__ __forceinline__ int cell_index(const Grid& C, const double x3[3], int
 
 // Count phase of one atom at its current position (any drift already applied): its cell and its arrival slot
 // there.  One atomic per distinct cell among the wave's active lanes, all issued together (one after another,
-// each waiting for the last, they made the count of 250,047 atoms 23.6 us; with the rest of its loads now 11.6).  The arrival slot
-// only has to be unique within the cell: the placement ranks the cell's entries by key.
+// each waiting for the last, they made the count of 250,047 atoms 23.6 us; with the rest of its loads now 11.6).  The
+// arrival slot only has to be unique within the cell: the placement ranks the cell's entries by key.
 __device__ __forceinline__ void count_atom(const DevView& v, int cell, int a)
 {
     v.cell_of[a] = cell;

@@ -14,8 +14,7 @@
 //                      stable order
 //   k_bin_small      : all of it in one workgroup's LDS for small contexts
 // The placement writes the next perm/offs buffers, invperm and the sorted coordinates (FP64, and FP32 relative
-// to the cell); the
-// host then flips the parity argument that selects the current buffers.
+// to the cell); the host then flips the parity argument that selects the current buffers.
 #include "chmc_internal.hpp"
 #include "bin_device.hpp"
 
@@ -289,11 +288,13 @@ __global__ __launch_bounds__(256, 8) void k_cell_rank(DevView v)
 // latency each otherwise: N = 512, FP64 leapfrog, count + scan + placement took 21 us an evaluation, now
 // 4.9.  Bound: latency (three global round trips, six barriers), and one CU's instructions from about 2000 atoms
 // on: an FP64 leapfrog step of 2,744 atoms takes 18.5 us with it and 22.4 without, of 4,096 29.7 (before the loads
-// were brought together) and 24.1.  512 threads where an atom each is enough: 11.2 -> 10.9 us a step of N = 512.
+// were brought together) and 24.1.  Up to 512 atoms and cells, 512 threads with an atom each: 11.2 -> 10.9 us a step
+// of N = 512; contexts beyond take 1024 threads with up to three atoms each, also those of 513 to 1024, for which an
+// instance of one atom a thread has not been measured.
 // Cells of more than kSmallDense atoms (clustered systems, or those of few cells) follow at the end and rank their
 // keys by a bit for each, in the cell's own part of key[] (16 KB more LDS made a step of 2,744 atoms 1 % longer):
 // 3000 atoms in one cell, pairwise 217 us a binning, now 26.  The test for them costs 0.2 of the 20 us a step of
-// 2,744 atoms takes, and nothing measurable of the 11 us at 512.
+// 2,744 atoms takes and 0.1 of the 11 us at 512.
 constexpr int kSmallDense = 160;
 template <int T, int PT>
 __global__ __launch_bounds__(T) void k_bin_small(DevView v, double drift_dt, int do_drift, int atom_id_order)

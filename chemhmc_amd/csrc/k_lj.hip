@@ -198,8 +198,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_lj(DevView v, double kick_dt, d
 }
 
 // ---- FP64 sweep ------------------------------------------------------------------------------------
-// One workgroup of W wavefronts per i-cell, or `parts` of them (forces), one wave per i-atom.  The 64 lanes test 64 staged j entries a step
-// (FP64 coordinates relative to the i-cell origin, r^2 < rc^2), and the pairs inside (14 % of the candidates
+// One workgroup of W wavefronts per i-cell, or `parts` of them (forces), one wave per i-atom.  The 64 lanes test 64
+// staged j entries a step (FP64 coordinates relative to the i-cell origin, r^2 < rc^2), and the pairs inside (14 % of the candidates
 // at liquid density) are appended by ballot prefix to the wave's LDS list; whenever 64 are pending, and at the
 // end, the lanes take one each and evaluate it: reciprocal from v_rcp_f64 with two Newton steps, per-lane sums.
 //   LJ_FORCE: a butterfly over the wave sums the three components per atom; lanes 0..2 store and kick.
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_lj(DevView v, double kick_dt, d
 // Energies need a cell's sums in one workgroup: 16 waves below kSmallCells cells, else 4.
 constexpr int kWideCells = 2048, kForceGroups = 1024;
 constexpr int kSmallCells = 512;
-constexpr int kMaxJ64 = 512;          // j entries per LDS pass: seven workgroups of four waves a CU
+constexpr int kMaxJ64 = 512;          // j entries per LDS pass, 17 KB: nine workgroups of four waves fit a CU, its wave slots take eight
 
 template <int W, int MODE>
 __global__ __launch_bounds__(64 * W) void k_lj64(DevView v, double kick_dt, int parts)

@@ -230,8 +230,8 @@ __global__ __launch_bounds__(1024) void k_open_sum(const double* __restrict__ pa
     *result = s;
 }
 
-// about 2048 workgroups (8 a CU): few enough that adding their histograms to the counters stays small,
-// rows in order, so that the long ones start first
+// about 4096 workgroups, of which the half below the diagonal returns at once (8 a CU stay): few enough that adding
+// their histograms to the counters stays small, rows in order, so that the long ones start first
 hipError_t launch_rdf(const DevView& v, int chain, int natoms, bool cube, int nbins, double size_bin, uint4* u,
                       unsigned long long* counts, hipStream_t s)
 {

@@ -86,8 +86,6 @@ __global__ __launch_bounds__(256) void k_heatbath(DevView v, uint64_t seed, long
     if (threadIdx.x == 0) v.chunk_part[blockIdx.x] = t;
 }
 
-// per-chain sums (one 256-thread workgroup per chain) of the LJ sweep's per-cell partials and/or the
-// per-chunk kinetic partials
 // K sums over the 256 threads, each as block_sum_256 forms it (in thread 0), behind one barrier; once a kernel
 template <int K>
 __device__ __forceinline__ void block_sums_256(double (&s)[K])
@@ -159,6 +157,8 @@ __device__ void chain_sums(const DevView& v, int ch, int what, double out[RED_NS
     for (int k = 0; k < RED_NSLOT; k++) red[k] = out[k];
 }
 
+// per-chain sums (one 256-thread workgroup per chain) of the LJ sweep's per-cell partials and/or the
+// per-chunk kinetic partials
 __global__ __launch_bounds__(256) void k_reduce(DevView v, int what)
 {
     double sums[RED_NSLOT];
