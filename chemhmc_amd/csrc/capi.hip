@@ -322,18 +322,20 @@ extern "C" int chmc_num_atoms(const chmc_ctx* c, int* total, int* nchains)
 // Pageable copies of three SoA arrays with host transposes took most of a call: set_positions +
 // compute_force + get_force at N = 32768 216 us of which kernels are 45, now 167; the surrogate features there
 // (8 MB, permuted on the host) 0.8 ms of the evaluation 1.4.  Larger arrays alternate between the two buffers,
-// the copy of one overlapping the kernel of the other.  A buffer holds the largest chain's positions, at least
-// kStageMin: a part is a launch and a wait, ~10 us, and the features of a chain take 128 B an atom (of 512 atoms in
-// parts of 16 KB 75 us, whole 33; of 4,096 in parts of 96 KB 113, of 256 KB 68; pinning the larger pair of buffers
-// at first use costs no measurable time more).
-constexpr size_t kStageMin = (size_t)256 << 10, kStageMax = (size_t)4 << 20;
+// the copy of one overlapping the kernel of the other.  A buffer holds the largest chain's positions (24 B an
+// atom, up to kStageMax), and its features (128 B an atom) and the energies of all chains (4 B) up to kStageWhole:
+// a part is a launch and a wait, ~10 us (features of 512 atoms in parts of 16 KB 75 us, whole 33; of 4,096 in parts
+// of 96 KB 113, of 256 KB 68; pinning the larger pair of buffers at first use costs no measurable time more).
+constexpr size_t kStageWhole = (size_t)256 << 10, kStageMax = (size_t)4 << 20;
 
 static int stage_ensure(chmc_ctx* c)
 {
     if (c->stage_cap) return CHMC_OK;
     int nmax = 1;
     for (const ChainDev& cd : c->hchains) nmax = std::max(nmax, cd.natoms);
-    const size_t cap = std::min(kStageMax, std::max<size_t>((24 * (size_t)nmax + 4095) / 4096 * 4096, kStageMin));
+    const size_t whole = std::max(sizeof(float) * kSurrFeat * (size_t)nmax, sizeof(float) * (size_t)c->Ntot);
+    size_t cap = std::max({ std::min(24 * (size_t)nmax, kStageMax), std::min(whole, kStageWhole), (size_t)16384 });
+    cap = (cap + 4095) / 4096 * 4096;
     for (hipEvent_t& e : c->stage_ev)
         if (!e) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     void* p = nullptr;
