@@ -294,12 +294,14 @@ __global__ __launch_bounds__(256, 8) void k_cell_rank(DevView v)
 // Cells of more than kSmallDense atoms (clustered systems, or those of few cells) follow at the end and rank their
 // keys by a bit for each, in the cell's own part of key[] (16 KB more LDS made a step of 2,744 atoms 1 % longer):
 // 3000 atoms in one cell, pairwise 217 us a binning, now 26.  The test for them costs 0.2 of the 20 us a step of
-// 2,744 atoms takes and 0.1 of the 11 us at 512.
+// 2,744 atoms takes.  Contexts of up to 512 atoms go without: all of them in one cell, ranked pairwise, take 24 us a
+// binning against 15 spread out, and the test would cost each step 0.1 of 10.9 us.
 constexpr int kSmallDense = 160;
 template <int T, int PT>
 __global__ __launch_bounds__(T) void k_bin_small(DevView v, double drift_dt, int do_drift, int atom_id_order)
 {
     constexpr int kMax = T * PT, kWords = kMax / 32;
+    constexpr bool kDenseToo = PT > 1;
     static_assert(kWords + kWords / 2 <= kSmallDense, "the bits and their counts before each word, in 16 bits");
     __shared__ int cnt[kMax], key[kMax], wsum[T / 64];
     const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -334,7 +336,7 @@ __global__ __launch_bounds__(T) void k_bin_small(DevView v, double drift_dt, int
         s += c4[k];
         most = max(most, c4[k]);
     }
-    const bool dense_wave = __ballot(most > kSmallDense) != 0ull;
+    const bool dense_wave = kDenseToo && __ballot(most > kSmallDense) != 0ull;
     int incl = s;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -343,10 +345,15 @@ __global__ __launch_bounds__(T) void k_bin_small(DevView v, double drift_dt, int
     }
     if (lane == 63) wsum[wid] = incl | (dense_wave ? 1 << 16 : 0);
     __syncthreads();
-    const int ws = wsum[lane & (T / 64 - 1)];
-    const bool dense = __ballot(ws >> 16 != 0) != 0ull;                // in any wave
+    bool dense = false;                    // in any wave
     int run = incl - s;
-    for (int w = 0; w < wid; w++) run += __builtin_amdgcn_readlane(ws, w) & 0xffff;
+    if constexpr (kDenseToo) {
+        const int ws = wsum[lane & (T / 64 - 1)];
+        dense = __ballot(ws >> 16 != 0) != 0ull;
+        for (int w = 0; w < wid; w++) run += __builtin_amdgcn_readlane(ws, w) & 0xffff;
+    } else {
+        for (int w = 0; w < wid; w++) run += wsum[w];
+    }
     int* offs = offs_next(v);
 #pragma unroll
     for (int k = 0; k < PT; k++) {
@@ -368,13 +375,13 @@ __global__ __launch_bounds__(T) void k_bin_small(DevView v, double drift_dt, int
         const int a = k * T + tid;
         if (a >= N) continue;
         const int beg = cnt[cell[k]], end = end_of(k);
-        if (end - beg > kSmallDense) continue;
+        if (kDenseToo && end - beg > kSmallDense) continue;
         int rank = 0;
 #pragma unroll 4
         for (int q = beg; q < end; q++) rank += key[q] < mykey[k] ? 1 : 0;
         place_atom(v, perm_n, beg + rank, a, x3[k], o3[k]);
     }
-    if (!dense) return;
+    if (!kDenseToo || !dense) return;
     // f(begin) for every dense cell, by the wave of the thread that scanned it
     auto dense_cells = [&](auto f) {
 #pragma unroll

@@ -192,23 +192,27 @@ def _dense_case(name):
     N, L, rc, ball = {
         "one_cell_160": (160, 5.0, 2.6, None), "one_cell_161": (161, 5.0, 2.6, None), "one_cell_512": (512, 5.0, 2.6, None),
         "eight_cells_512": (512, 5.1, 2.5, None), "one_cell_3072": (3072, 9.0, 5.0, None), "27_cells_3000": (3000, 16.0, 5.3, None),
-        "3000_in_a_corner": (3000, 30.0, 2.5, 6.0),
+        "3000_in_a_corner": (3000, 30.0, 2.5, 6.0), "160_of_700": (700, 30.0, 2.5, None), "161_of_700": (700, 30.0, 2.5, None),
         "one_cell_3073": (3073, 9.0, 5.0, None), "27_cells_4096": (4096, 16.0, 5.3, None), "27_cells_8000": (8000, 20.0, 6.6, None),
         "64_a_cell": (8000, 12.6, 2.5, None), "8_cells_20000": (20000, 29.0, 14.0, None),
         "droplet": (9000, 45.0, 2.5, 9.0), "corner": (9000, 45.0, 2.5, 4.0),
         "windows": (140000, 50.0, 10.0, None), "windows_corner": (70000, 80.0, 2.5, 4.0)}[name]
     x = rng.uniform(0, 1, (N, 3)) * L
+    if name.endswith("_of_700"):   # so many in one cell of 729, the others elsewhere
+        x = 5.0 + x * (25.0 / L)
+        k = rng.permutation(N)[:int(name[:3])]
+        x[k] = rng.uniform(0, 2.4, (len(k), 3))
     if ball:                       # two thirds of the atoms close together, in random order of their ids
         k = rng.permutation(N)[:2 * N // 3]
         x[k] = rng.uniform(0, ball, (len(k), 3)) + 1.0
     return x, L, rc
 
 
-# cells of many atoms: of the one-launch binning at the limit of its pairwise ranking (160 atoms a cell), with 8, 27
-# and few dense cells among many; of the four-launch one at its limit (64) with a workgroup a cell and with sixteen,
+# cells of many atoms: of the one-launch binning at the limit of its pairwise ranking (160 atoms a cell in contexts of
+# more than 512 atoms or cells), with 8, 27 and few dense cells among many; of the four-launch one at its limit (64) with a workgroup a cell and with sixteen,
 # pairwise (up to 362 keys in one window) and by bits in one window and in several
 @pytest.mark.parametrize("name", ["one_cell_160", "one_cell_161", "one_cell_512", "eight_cells_512", "one_cell_3072",
-                                  "27_cells_3000", "3000_in_a_corner", "one_cell_3073", "27_cells_4096", "27_cells_8000",
+                                  "27_cells_3000", "3000_in_a_corner", "160_of_700", "161_of_700", "one_cell_3073", "27_cells_4096", "27_cells_8000",
                                   "64_a_cell", "8_cells_20000", "droplet", "corner", "windows", "windows_corner"])
 @pytest.mark.parametrize("order", [False, True])
 def test_binning_dense_cells(chmc, orc, name, order):
