@@ -198,7 +198,7 @@ def _dense_case(name):
         "droplet": (9000, 45.0, 2.5, 9.0), "corner": (9000, 45.0, 2.5, 4.0),
         "windows": (140000, 50.0, 10.0, None), "windows_corner": (70000, 80.0, 2.5, 4.0)}[name]
     x = rng.uniform(0, 1, (N, 3)) * L
-    if name.endswith("_of_700"):   # so many in one cell of 729, the others elsewhere
+    if name.endswith("_of_700"):   # so many in one cell of 1728, the others elsewhere
         x = 5.0 + x * (25.0 / L)
         k = rng.permutation(N)[:int(name[:3])]
         x[k] = rng.uniform(0, 2.4, (len(k), 3))
