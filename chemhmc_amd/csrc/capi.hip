@@ -346,11 +346,25 @@ static int stage_ensure(chmc_ctx* c)
     return CHMC_OK;
 }
 
+// The transfers launch kernels and record events, which belong to the context's device; copies, which they stand
+// for, took a stream of any device, so the caller may have another one current.
+struct OnDevice {
+    int prev = -1;
+    explicit OnDevice(int device)
+    {
+        if (hipGetDevice(&prev) == hipSuccess && prev != device) hipSetDevice(device);
+        else prev = -1;
+    }
+    ~OnDevice() { if (prev >= 0) hipSetDevice(prev); }
+    OnDevice(const OnDevice&) = delete;
+};
+
 // rows of row_bytes from the device: launch(first row, rows, buffer) writes a part, use(buffer, first row,
 // rows) takes it.  Returns with every part taken (and the stream drained up to the last kernel).
 template <typename Launch, typename Use>
 static int staged_get(chmc_ctx* c, size_t rows, size_t row_bytes, Launch launch, Use use)
 {
+    const OnDevice on(c->device);
     int rc = stage_ensure(c);
     if (rc) return rc;
     const size_t per = c->stage_cap / row_bytes, parts = (rows + per - 1) / per;
@@ -371,6 +385,7 @@ static int staged_get(chmc_ctx* c, size_t rows, size_t row_bytes, Launch launch,
 template <typename Fill, typename Launch>
 static int staged_put(chmc_ctx* c, size_t rows, size_t row_bytes, Fill fill, Launch launch)
 {
+    const OnDevice on(c->device);
     int rc = stage_ensure(c);
     if (rc) return rc;
     const size_t per = c->stage_cap / row_bytes, parts = (rows + per - 1) / per;
